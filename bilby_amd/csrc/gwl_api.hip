@@ -273,6 +273,76 @@ __global__ void k_ln_i0(const double* in, double* out, long long n) {
   if (i < n) out[i] = ln_i0(in[i]);
 }
 
+// ------------------------------------------------------------------ spline tables
+// Intervals by bucket (spline_interval): the interval of every bucket's
+// smallest value, buckets and knots walked together.
+static void spline_buckets(const double* t, int ncoef, unsigned short* idx) {
+  int l = 3;
+  for (unsigned k = 0; k < 65536; ++k) {
+    // the smallest value of the bucket (most negative: all lower bits set)
+    const uint64_t hi = (k & 0x8000u) ? ((uint64_t)(k << 16) & 0x7fffffffull)
+                                      : (uint64_t)(uint32_t)~(k << 16);
+    const uint64_t bits = (hi << 32) | ((k & 0x8000u) ? 0ull : 0xffffffffull);
+    double x;
+    memcpy(&x, &bits, sizeof x);
+    if (!std::isnan(x))
+      while (l < ncoef - 1 && t[l + 1] <= x) ++l;
+    idx[k] = (unsigned short)l;
+  }
+}
+
+// r[j - 1][l] = 1 / (t[l + 1] - t[l + 1 - j]), 0 where the knots coincide.
+static void spline_reciprocals(const double* t, int nt, double* r) {
+  for (int j = 1; j <= 3; ++j)
+    for (int l = 0; l < nt; ++l) {
+      const double w = l + 1 < nt && l + 1 >= j ? t[l + 1] - t[l + 1 - j] : 0.0;
+      r[(size_t)(j - 1) * nt + l] = w > 0.0 ? 1.0 / w : 0.0;
+    }
+}
+
+int spline_upload(int nx, int ny, const double* tx, const double* ty, const double* coeffs,
+                  const double* bbox, double** mem, size_t* bytes, SplineDev* sp) {
+  if (nx > 65535 || ny > 65535) {
+    set_error("distance spline: more than 65535 coefficients on an axis");
+    return GWL_E_UNSUPPORTED;
+  }
+  const size_t ni = 65536 * sizeof(unsigned short) / sizeof(double);
+  const size_t oix = 0, oiy = oix + ni, otx = oiy + ni, oty = otx + nx + 4, orx = oty + ny + 4,
+               ory = orx + 3 * (size_t)(nx + 4), oc = ory + 3 * (size_t)(ny + 4);
+  const size_t n = oc + (size_t)nx * ny;
+  std::vector<double> h(n);
+  spline_reciprocals(tx, nx + 4, h.data() + orx);
+  spline_reciprocals(ty, ny + 4, h.data() + ory);
+  spline_buckets(tx, nx, reinterpret_cast<unsigned short*>(h.data() + oix));
+  spline_buckets(ty, ny, reinterpret_cast<unsigned short*>(h.data() + oiy));
+  memcpy(h.data() + otx, tx, (size_t)(nx + 4) * sizeof(double));
+  memcpy(h.data() + oty, ty, (size_t)(ny + 4) * sizeof(double));
+  for (int i = 0; i < nx; ++i)
+    for (int j = 0; j < ny; ++j) h[oc + (size_t)j * nx + i] = coeffs[(size_t)i * ny + j];
+  if (*mem) {
+    (void)hipFree(*mem);
+    *mem = nullptr;
+  }
+  GWL_HIP_CHECK(hipMalloc(mem, n * sizeof(double)));
+  *bytes = n * sizeof(double);
+  GWL_HIP_CHECK(hipMemcpy(*mem, h.data(), n * sizeof(double), hipMemcpyHostToDevice));
+  const double* m = *mem;
+  sp->rx = m + orx;
+  sp->ry = m + ory;
+  sp->ix = reinterpret_cast<const unsigned short*>(m + oix);
+  sp->iy = reinterpret_cast<const unsigned short*>(m + oiy);
+  sp->tx = m + otx;
+  sp->ty = m + oty;
+  sp->ct = m + oc;
+  sp->nx = nx;
+  sp->ny = ny;
+  sp->xmin = bbox[0];
+  sp->xmax = bbox[1];
+  sp->ymin = bbox[2];
+  sp->ymax = bbox[3];
+  return GWL_OK;
+}
+
 // ------------------------------------------------------------------ host spline solve
 // Not-a-knot cubic knots on the data abscissae (FITPACK's choice for s = 0):
 // t = {x0 x4, x2 .. x_{n-3}, x_{n-1} x4}.
@@ -804,28 +874,9 @@ int gwl_event_set_distance_spline(gwl_event* e, int32_t nx, int32_t ny, const do
     return GWL_E_INVALID;
   }
   GWL_HIP_CHECK(hipSetDevice(e->ctx->device));
-  const size_t n = (size_t)(nx + 4) + (ny + 4) + (size_t)nx * ny;
-  if (e->spline) {
-    (void)hipFree(e->spline);
-    e->spline = nullptr;
-  }
-  GWL_HIP_CHECK(hipMalloc(&e->spline, n * sizeof(double)));
-  e->spline_bytes = n * sizeof(double);
-  GWL_HIP_CHECK(hipMemcpy(e->spline, tx, (nx + 4) * sizeof(double), hipMemcpyHostToDevice));
-  GWL_HIP_CHECK(hipMemcpy(e->spline + nx + 4, ty, (ny + 4) * sizeof(double), hipMemcpyHostToDevice));
-  GWL_HIP_CHECK(hipMemcpy(e->spline + nx + 4 + ny + 4, coeffs, (size_t)nx * ny * sizeof(double),
-                          hipMemcpyHostToDevice));
-  SplineDev sp;
-  sp.tx = e->spline;
-  sp.ty = e->spline + nx + 4;
-  sp.c = e->spline + nx + 4 + ny + 4;
-  sp.nx = nx;
-  sp.ny = ny;
-  sp.xmin = bbox[0];
-  sp.xmax = bbox[1];
-  sp.ymin = bbox[2];
-  sp.ymax = bbox[3];
-  e->dev.sp = sp;
+  if (int rc = spline_upload(nx, ny, tx, ty, coeffs, bbox, &e->spline, &e->spline_bytes,
+                             &e->dev.sp))
+    return rc;
   e->has_spline = true;
   return GWL_OK;
 }
@@ -1331,14 +1382,13 @@ int gwl_spline2d_eval_host(int32_t nx, int32_t ny, const double* tx, const doubl
   SplineDev sp;
   sp.tx = tx;
   sp.ty = ty;
-  sp.c = c;
   sp.nx = nx;
   sp.ny = ny;
   sp.xmin = tx[0];
   sp.xmax = tx[nx + 3];
   sp.ymin = ty[0];
   sp.ymax = ty[ny + 3];
-  for (int64_t i = 0; i < m; ++i) out[i] = spline2d(sp, x[i], y[i]);
+  for (int64_t i = 0; i < m; ++i) out[i] = spline2d(sp, c, x[i], y[i]);
   return GWL_OK;
 }
 

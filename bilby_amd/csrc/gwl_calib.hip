@@ -230,11 +230,8 @@ __device__ __forceinline__ double gval(const CalArgs& a, const void* g, size_t i
 // One wavefront per row, lanes over curves: ln L_c and their logsumexp
 // minus ln C (base.py:860-877; the value per curve as base.py:775-792).
 __global__ __launch_bounds__(256) void k_cal_epi(CalArgs a) {
-  extern __shared__ double knots[];
   const EvDev& ev = a.ev;
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
-  if (dist) stage_knots(ev, knots);
-  __syncthreads();
   const int lane = threadIdx.x & 63;
   const long long r = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= a.n) return;
@@ -252,9 +249,9 @@ __global__ __launch_bounds__(256) void k_cal_epi(CalArgs a) {
     const double hh = h0 + gval(a, a.g2, (size_t)r * a.N2p + c, a.nz2, z2);
     double v;
     if (dist) {
-      const double dd = (ev.flags & GWL_PHASE_MARG) ? hypot(dr, di) * hs : dr * hs;
-      const SplineY yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
-      v = spline_x(ev, knots, yy, dd);
+      const double dd = (ev.flags & GWL_PHASE_MARG) ? cabs2d(dr, di) * hs : dr * hs;
+      const SplineY yy = spline_y(ev.sp, hh * hs * hs);
+      v = spline_x(ev.sp, yy, dd);
     } else if (ev.flags & GWL_PHASE_MARG) {
       v = ln_i0(hypot(dr, di)) - hh / 2.0;
     } else {
@@ -623,9 +620,7 @@ int gwl_calib_eval(gwl_calib* c, const double* params, int64_t n, int32_t ld, in
                           stream))
       return rc;
   }
-  const size_t lds = (ev->dev.flags & GWL_DISTANCE_MARG)
-                         ? (size_t)(ev->dev.sp.nx + ev->dev.sp.ny + 8) * 8 : 0;
-  hipLaunchKernelGGL(gwl::k_cal_epi, dim3((unsigned)((n + 3) / 4)), dim3(256), lds, st, a);
+  hipLaunchKernelGGL(gwl::k_cal_epi, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, a);
   GWL_HIP_CHECK(hipGetLastError());
   return gwl::timing_end(ev, st);
 }

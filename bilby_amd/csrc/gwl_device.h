@@ -99,7 +99,14 @@ __device__ __forceinline__ double2 expm2pi(double r) {
 struct SplineDev {
   const double* tx;
   const double* ty;
-  const double* c;
+  const double* ct;  // coefficients [ny][nx]: a row's values share their y interval
+  // per axis: the interval of the smallest value of each bucket of the
+  // number's upper 16 bits, and the reciprocals of the spans of one, two and
+  // three knots [3][n + 4] (r[j - 1][l] = 1 / (t[l + 1] - t[l + 1 - j]))
+  const unsigned short* ix;
+  const unsigned short* iy;
+  const double* rx;
+  const double* ry;
   int nx, ny;  // coefficient counts (knots: nx + 4, ny + 4)
   double xmin, xmax, ymin, ymax;
 };
@@ -575,8 +582,9 @@ __host__ __device__ inline void bspline3(const double* t, int l, double x, doubl
 }
 
 // BoundedRectBivariateSpline (bilby/core/utils/calculus.py:221-262):
-// the bicubic interpolant, -inf outside the bounding box.
-__host__ __device__ inline double spline2d(const SplineDev& sp, double x, double y) {
+// the bicubic interpolant (coefficients [nx][ny]), -inf outside the bounding
+// box; host only, the device form is spline_x.
+inline double spline2d(const SplineDev& sp, const double* coef, double x, double y) {
   if (!(x >= sp.xmin && x <= sp.xmax && y >= sp.ymin && y <= sp.ymax)) return -INFINITY;
   int lx = knot_interval(sp.tx, sp.nx, x);
   int ly = knot_interval(sp.ty, sp.ny, y);
@@ -584,11 +592,9 @@ __host__ __device__ inline double spline2d(const SplineDev& sp, double x, double
   bspline3(sp.tx, lx, x, bx);
   bspline3(sp.ty, ly, y, by);
   double s = 0.0;
-  const double* c = sp.c + (size_t)(lx - 3) * sp.ny + (ly - 3);
-#pragma unroll
+  const double* c = coef + (size_t)(lx - 3) * sp.ny + (ly - 3);
   for (int i = 0; i < 4; ++i) {
     double r = 0.0;
-#pragma unroll
     for (int j = 0; j < 4; ++j) r += by[j] * c[(size_t)i * sp.ny + j];
     s += bx[i] * r;
   }
@@ -733,11 +739,49 @@ __device__ inline void fft_lds(C* buf, const C* tw, int B) {
 
 __device__ inline double row_valid_sentinel() { return -DBL_MAX; }  // base.py:424-425
 
-// Knots of the distance spline staged in LDS: tx[nx + 4] then ty[ny + 4].
-__device__ inline void stage_knots(const EvDev& ev, double* lds) {
-  const int nx4 = ev.sp.nx + 4, ny4 = ev.sp.ny + 4;
-  for (int i = threadIdx.x; i < nx4; i += blockDim.x) lds[i] = ev.sp.tx[i];
-  for (int i = threadIdx.x; i < ny4; i += blockDim.x) lds[nx4 + i] = ev.sp.ty[i];
+// The bucket of x in the interval tables: sign, exponent and 4 mantissa bits
+// in an order that follows x.
+__host__ __device__ __forceinline__ unsigned spline_bucket(unsigned hi) {
+  return ((hi & 0x80000000u) ? ~hi : (hi | 0x80000000u)) >> 16;
+}
+
+// knot_interval from the axis's bucket table: 16 buckets an octave put the
+// search one or two steps from its end (knots 15 decades / 799 apart), where
+// a binary search over LDS takes ten dependent reads.
+__device__ __forceinline__ int spline_interval(const unsigned short* idx, const double* t,
+                                               int ncoef, double x) {
+  int l = idx[spline_bucket((unsigned)__double2hiint(x))];
+  while (l < ncoef - 1 && t[l + 1] <= x) ++l;
+  return l;
+}
+
+// Four doubles in one (unaligned) load.
+typedef double f64x4 __attribute__((ext_vector_type(4), aligned(8)));
+typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8)));
+
+// The four cubic B-splines that are non-zero on interval l, at x: bspline3
+// with the tabled reciprocals in place of its six divisions.  The lanes of a
+// wavefront sit on neighbouring intervals, so each of these loads touches a
+// few cache lines (64 separate ones with a record per interval).
+__device__ __forceinline__ void spline_basis(const double* t, const double* r, int n, int l,
+                                             double x, double* h) {
+  const f64x2 lo = *reinterpret_cast<const f64x2*>(t + l - 2);
+  const f64x4 hi = *reinterpret_cast<const f64x4*>(t + l);
+  const double r1 = r[l];
+  const f64x2 r2 = *reinterpret_cast<const f64x2*>(r + (n + 4) + l);
+  const f64x2 r3 = *reinterpret_cast<const f64x2*>(r + 2 * (n + 4) + l);
+  const double r3c = r[2 * (n + 4) + l + 2];
+  const double d0 = x - hi.x, d1 = x - lo.y, d2 = x - lo.x;        // x - t_l, t_l-1, t_l-2
+  const double u1 = hi.y - x, u2 = hi.z - x, u3 = hi.w - x;        // t_l+1 - x, ...
+  // order 1, 2, 3
+  const double a0 = u1 * r1, a1 = d0 * r1;
+  const double f0 = a0 * r2.x, f1 = a1 * r2.y;
+  const double b0 = f0 * u1, b1 = fma(f0, d1, f1 * u2), b2 = f1 * d0;
+  const double g0 = b0 * r3.x, g1 = b1 * r3.y, g2 = b2 * r3c;
+  h[0] = g0 * u1;
+  h[1] = fma(g0, d2, g1 * u2);
+  h[2] = fma(g1, d1, g2 * u3);
+  h[3] = g2 * d0;
 }
 
 // y-part of the bicubic interpolant (fixed per row): interval and basis.
@@ -747,34 +791,39 @@ struct SplineY {
   bool inside;
 };
 
-__device__ inline SplineY spline_y(const EvDev& ev, const double* ty, double y) {
+__device__ inline SplineY spline_y(const SplineDev& sp, double y) {
   SplineY r;
-  r.inside = (y >= ev.sp.ymin && y <= ev.sp.ymax);
+  r.inside = (y >= sp.ymin && y <= sp.ymax);
   r.ly = 3;
   r.by[0] = r.by[1] = r.by[2] = r.by[3] = 0.0;
   if (r.inside) {
-    r.ly = knot_interval(ty, ev.sp.ny, y);
-    bspline3(ty, r.ly, y, r.by);
+    r.ly = spline_interval(sp.iy, sp.ty, sp.ny, y);
+    spline_basis(sp.ty, sp.ry, sp.ny, r.ly, y, r.by);
   }
   return r;
 }
 
 // BoundedRectBivariateSpline value at (x, y) with the y-part precomputed;
 // -inf outside the bounding box (calculus.py:252-260).
-__device__ inline double spline_x(const EvDev& ev, const double* tx, const SplineY& yy, double x) {
-  if (!yy.inside || !(x >= ev.sp.xmin && x <= ev.sp.xmax)) return -INFINITY;
-  const int lx = knot_interval(tx, ev.sp.nx, x);
+__device__ inline double spline_x(const SplineDev& sp, const SplineY& yy, double x) {
+  if (!yy.inside || !(x >= sp.xmin && x <= sp.xmax)) return -INFINITY;
+  const int lx = spline_interval(sp.ix, sp.tx, sp.nx, x);
   double bx[4];
-  bspline3(tx, lx, x, bx);
-  const double* c = ev.sp.c + (size_t)(lx - 3) * ev.sp.ny + (yy.ly - 3);
+  spline_basis(sp.tx, sp.rx, sp.nx, lx, x, bx);
+  const double* c = sp.ct + (size_t)(yy.ly - 3) * sp.nx + (lx - 3);
   double s = 0.0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const double* ci = c + (size_t)i * ev.sp.ny;
-    s += bx[i] * (yy.by[0] * ci[0] + yy.by[1] * ci[1] + yy.by[2] * ci[2] + yy.by[3] * ci[3]);
+  for (int j = 0; j < 4; ++j) {
+    const f64x4 cj = *reinterpret_cast<const f64x4*>(c + (size_t)j * sp.nx);
+    s += yy.by[j] * (bx[0] * cj.x + bx[1] * cj.y + bx[2] * cj.z + bx[3] * cj.w);
   }
   return s;
 }
+
+// |x + i y| for the distance table, whose axes end far inside the float64
+// range: where the squares overflow the value lies outside them either way
+// (the library hypot scales first).
+__device__ __forceinline__ double cabs2d(double x, double y) { return sqrt(fma(x, x, y * y)); }
 
 // Per-row constants of the TaylorF2 time transforms (k_rowconst).
 struct RowW {
@@ -801,13 +850,13 @@ struct RowW {
 
 // Marginalised lnL at one time (base.py:775-792): distance spline (y-part
 // precomputed per row), else ln I0 (phase) or the real part.
-__device__ inline double epi_value(const EvDev& ev, const double* knots, const SplineY& yy,
+__device__ inline double epi_value(unsigned flags, const SplineDev& sp, const SplineY& yy,
                                    double hh, double hs, double xr, double xi) {
-  if (ev.flags & GWL_DISTANCE_MARG) {
-    const double d = (ev.flags & GWL_PHASE_MARG) ? hypot(xr, xi) * hs : xr * hs;
-    return spline_x(ev, knots, yy, d);
+  if (flags & GWL_DISTANCE_MARG) {
+    const double d = (flags & GWL_PHASE_MARG) ? cabs2d(xr, xi) * hs : xr * hs;
+    return spline_x(sp, yy, d);
   }
-  if (ev.flags & GWL_PHASE_MARG) return ln_i0(hypot(xr, xi)) - hh / 2.0;
+  if (flags & GWL_PHASE_MARG) return ln_i0(hypot(xr, xi)) - hh / 2.0;
   return xr - hh / 2.0;
 }
 
@@ -856,19 +905,16 @@ __device__ __forceinline__ void lse_push(double& m, double& s, double v) {
   }
 }
 
-// Merge the logsumexp states of the 64 lanes of a wavefront.
+// Merge the logsumexp states of the 64 lanes of a wavefront: the maximum
+// first, then one exponential a lane (merging pair by pair takes twelve).
 __device__ __forceinline__ void lse_wave(double& m, double& s) {
+  double mx = m;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const double mo = __shfl_xor(m, off, 64), so = __shfl_xor(s, off, 64);
-    const double mn = fmax(m, mo);
-    if (mn > -INFINITY) {
-      s = (m > -INFINITY ? s * exp(m - mn) : 0.0) + (mo > -INFINITY ? so * exp(mo - mn) : 0.0);
-    } else {
-      s = 0.0;
-    }
-    m = mn;
-  }
+  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+  s = m > -INFINITY ? s * exp(m - mx) : 0.0;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  m = mx;
 }
 
 }  // namespace gwl

@@ -117,6 +117,10 @@ size_t workspace_bytes_for(const gwl_event* ev, int64_t rows, int precision);
 // upload a time-prior density table (n values at t0 + k dt) into *dst (freed
 // and replaced), checking the arguments
 int upload_time_prior(int64_t n, double t0, double dt, const double* density, double** dst);
+// the distance spline (host knots, coefficients and bounding box) with its
+// interval and reciprocal tables into *mem (freed and replaced)
+int spline_upload(int nx, int ny, const double* tx, const double* ty, const double* coeffs,
+                  const double* bbox, double** mem, size_t* bytes, SplineDev* sp);
 // this device's address of the gwl_eval_noalloc scratch array (gwl_noalloc.hip)
 int noalloc_scratch_init(int device, void** ptr);
 int launch_eval(gwl_event* ev, const double* params, int64_t n, int ld, int precision, double* out,

@@ -411,13 +411,10 @@ __device__ inline double escalation_scale(unsigned flags, double dhr, double dhi
 }
 
 // lnL from the summed inner products (base.py:448-477, 775-792); one thread
-// per row, knots in LDS.
+// per row.
 __global__ __launch_bounds__(128) void k_epi_plain(EpiArgs a) {
-  extern __shared__ double knots[];
   const EvDev& ev = a.ev;
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
-  if (dist) stage_knots(ev, knots);
-  __syncthreads();
   const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= live_rows(a.n, a.count)) return;
   const long long o = a.scatter ? (long long)a.scatter[r] : r;
@@ -462,9 +459,9 @@ __global__ __launch_bounds__(128) void k_epi_plain(EpiArgs a) {
   double ll;
   if (dist) {
     const double hs = sc.hscale;
-    const double d = (ev.flags & GWL_PHASE_MARG) ? hypot(dhr, dhi) * hs : dhr * hs;
-    const SplineY yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
-    ll = spline_x(ev, knots, yy, d);
+    const double d = (ev.flags & GWL_PHASE_MARG) ? cabs2d(dhr, dhi) * hs : dhr * hs;
+    const SplineY yy = spline_y(ev.sp, hh * hs * hs);
+    ll = spline_x(ev.sp, yy, d);
   } else if (ev.flags & GWL_PHASE_MARG) {
     ll = ln_i0(hypot(dhr, dhi)) - hh / 2.0;
   } else {
@@ -474,12 +471,12 @@ __global__ __launch_bounds__(128) void k_epi_plain(EpiArgs a) {
 }
 
 // Time-marginalised lnL: logsumexp over the prior window (base.py:794-820).
-// One wavefront per row, kEpiRows rows per workgroup, knots in LDS.
+// One wavefront per row, kEpiRows rows per workgroup.
 constexpr int kEpiRows = 4;
 
 // One wavefront finishes one row: sums the group partials, evaluates the
 // marginalised lnL at every window bin and reduces them with a running-max
-// logsumexp.  ``knots`` holds the spline knots in LDS (distance only).
+// logsumexp.
 // Merge two (running max, scaled sum) logsumexp states.
 __device__ __forceinline__ void lse_merge(double& m, double& s, double mo, double so) {
   const double mn = fmax(m, mo);
@@ -519,9 +516,9 @@ __device__ __forceinline__ void epi_row_inputs(const EvDev& ev, const double* pa
 
 // The time-conditioned lnL at window bin jj plus the log time-prior weight
 // (-inf outside the prior).
-__device__ __forceinline__ double epi_bin_value(const EvDev& ev, const double* knots,
-                                                const SplineY& yy, double hh, double hs,
-                                                double jit, const double2* prow, int G, int jj) {
+__device__ __forceinline__ double epi_bin_value(const EvDev& ev, const SplineY& yy, double hh,
+                                                double hs, double jit, const double2* prow, int G,
+                                                int jj) {
   const int j = ev.jlo + jj;
   const double t = (ev.start + (double)(j + 1) * ev.tstep) + jit;
   if (!(t >= ev.tmin && t <= ev.tmax)) return -INFINITY;
@@ -537,8 +534,8 @@ __device__ __forceinline__ double epi_bin_value(const EvDev& ev, const double* k
   xi *= norm;
   double v;
   if (ev.flags & GWL_DISTANCE_MARG) {
-    const double d = (ev.flags & GWL_PHASE_MARG) ? hypot(xr, xi) * hs : xr * hs;
-    v = spline_x(ev, knots, yy, d);
+    const double d = (ev.flags & GWL_PHASE_MARG) ? cabs2d(xr, xi) * hs : xr * hs;
+    v = spline_x(ev.sp, yy, d);
   } else if (ev.flags & GWL_PHASE_MARG) {
     v = ln_i0(hypot(xr, xi)) - hh / 2.0;
   } else {
@@ -567,8 +564,8 @@ __device__ __forceinline__ void epi_finish(const EvDev& ev, long long r, double 
 // per window bin, logsumexp.
 __device__ inline void epi_time_row(const EvDev& ev, const double* params, int ld, long long r,
                                     int G, const double2* part, const double* hhpart, double* out,
-                                    const double* knots, double2* lse = nullptr, int first = 1,
-                                    int last = 1, const double* rinfo = nullptr, int Gs = 0) {
+                                    double2* lse = nullptr, int first = 1, int last = 1,
+                                    const double* rinfo = nullptr, int Gs = 0) {
   if (Gs <= 0) Gs = G;  // groups per row in the buffers (G of them summed here)
   const int lane = threadIdx.x & 63;
   double hh = 0.0, jit = 0.0, hs = 1.0;
@@ -583,13 +580,12 @@ __device__ inline void epi_time_row(const EvDev& ev, const double* params, int l
     return;
   }
   SplineY yy;
-  if (ev.flags & GWL_DISTANCE_MARG) yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
+  if (ev.flags & GWL_DISTANCE_MARG) yy = spline_y(ev.sp, hh * hs * hs);
   // single-pass (running max, scaled sum) logsumexp per lane, then merged
   double m = -INFINITY, s = 0.0;
   const double2* prow = part + (size_t)r * Gs * ev.L;
-  for (int jj = lane; jj < ev.L; jj += 64) lse_push(m, s, epi_bin_value(ev, knots, yy, hh, hs, jit, prow, G, jj));
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) lse_merge(m, s, __shfl_xor(m, off, 64), __shfl_xor(s, off, 64));
+  for (int jj = lane; jj < ev.L; jj += 64) lse_push(m, s, epi_bin_value(ev, yy, hh, hs, jit, prow, G, jj));
+  lse_wave(m, s);
   if (lane == 0) epi_finish(ev, r, m, s, out, lse, first, last);
 }
 
@@ -599,12 +595,10 @@ __device__ inline void epi_time_row(const EvDev& ev, const double* params, int l
 constexpr int kEpiWideThreads = 512;
 
 __global__ __launch_bounds__(kEpiWideThreads) void k_epi_time_wide(EpiArgs a) {
-  extern __shared__ double knots[];
   __shared__ double s_in[4];
   __shared__ int s_valid;
   __shared__ double s_m[kEpiWideThreads / 64], s_s[kEpiWideThreads / 64];
   const EvDev& ev = a.ev;
-  if (ev.flags & GWL_DISTANCE_MARG) stage_knots(ev, knots);
   const long long r = blockIdx.x;
   const int Gs = a.gstride > 0 ? a.gstride : a.G;
   if (threadIdx.x == 0) {
@@ -623,13 +617,12 @@ __global__ __launch_bounds__(kEpiWideThreads) void k_epi_time_wide(EpiArgs a) {
   }
   const double hh = s_in[0], jit = s_in[1], hs = s_in[2];
   SplineY yy;
-  if (ev.flags & GWL_DISTANCE_MARG) yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
+  if (ev.flags & GWL_DISTANCE_MARG) yy = spline_y(ev.sp, hh * hs * hs);
   double m = -INFINITY, s = 0.0;
   const double2* prow = a.part + (size_t)r * Gs * ev.L;
   for (int jj = threadIdx.x; jj < ev.L; jj += kEpiWideThreads)
-    lse_push(m, s, epi_bin_value(ev, knots, yy, hh, hs, jit, prow, a.G, jj));
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) lse_merge(m, s, __shfl_xor(m, off, 64), __shfl_xor(s, off, 64));
+    lse_push(m, s, epi_bin_value(ev, yy, hh, hs, jit, prow, a.G, jj));
+  lse_wave(m, s);
   if ((threadIdx.x & 63) == 0) {
     s_m[threadIdx.x >> 6] = m;
     s_s[threadIdx.x >> 6] = s;
@@ -642,12 +635,9 @@ __global__ __launch_bounds__(kEpiWideThreads) void k_epi_time_wide(EpiArgs a) {
 }
 
 __global__ __launch_bounds__(64 * kEpiRows) void k_epi_time(EpiArgs a) {
-  extern __shared__ double knots[];
-  if (a.ev.flags & GWL_DISTANCE_MARG) stage_knots(a.ev, knots);
-  __syncthreads();
   const long long r = (long long)blockIdx.x * kEpiRows + (threadIdx.x >> 6);
   if (r >= a.n) return;
-  epi_time_row(a.ev, a.params, a.ld, r, a.G, a.part, a.hhpart, a.out, knots, a.lse, a.first,
+  epi_time_row(a.ev, a.params, a.ld, r, a.G, a.part, a.hhpart, a.out, a.lse, a.first,
                a.last, a.rinfo, a.gstride);
 }
 
@@ -747,7 +737,6 @@ struct MultiEpiArgs {
 };
 
 __global__ __launch_bounds__(64 * kEpiRows) void k_epi_time_multi(MultiEpiArgs a) {
-  extern __shared__ double knots[];
   __shared__ EvDev s_ev;
   if ((int)blockIdx.x >= *a.n_blocks) return;
   const int e = a.block_event[blockIdx.x];
@@ -756,11 +745,9 @@ __global__ __launch_bounds__(64 * kEpiRows) void k_epi_time_multi(MultiEpiArgs a
   unsigned* dst = reinterpret_cast<unsigned*>(&s_ev);
   for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[i] = src[i];
   __syncthreads();
-  if (s_ev.flags & GWL_DISTANCE_MARG) stage_knots(s_ev, knots);
-  __syncthreads();
   const long long r = a.block_row0[blockIdx.x] + (threadIdx.x >> 6);
   if (r >= a.rows[e]) return;
-  epi_time_row(s_ev, a.params[e], a.ld, r, a.groups[e], a.part[e], a.hhpart[e], a.out[e], knots);
+  epi_time_row(s_ev, a.params[e], a.ld, r, a.groups[e], a.part[e], a.hhpart[e], a.out[e]);
 }
 
 __global__ void k_zero_int(int* p) { *p = 0; }
@@ -855,7 +842,6 @@ int launch_epi_time(gwl_event* e, const double* params, int64_t n, int ld, int G
   ea.first = first;
   ea.last = last;
   ea.rinfo = rinfo;
-  const size_t klds = (ev.flags & GWL_DISTANCE_MARG) ? (size_t)(ev.sp.nx + ev.sp.ny + 8) * sizeof(double) : 0;
   // few rows: the groups summed bin-parallel first, then one workgroup per row
   if (n <= kEpiGsumRows) {
     if (G > 1) {
@@ -866,12 +852,12 @@ int launch_epi_time(gwl_event* e, const double* params, int64_t n, int ld, int G
       ea.G = 1;
       ea.gstride = G;
     }
-    hipLaunchKernelGGL(k_epi_time_wide, dim3((unsigned)n), dim3(kEpiWideThreads), klds, st, ea);
+    hipLaunchKernelGGL(k_epi_time_wide, dim3((unsigned)n), dim3(kEpiWideThreads), 0, st, ea);
     GWL_HIP_CHECK(hipGetLastError());
     return GWL_OK;
   }
   hipLaunchKernelGGL(k_epi_time, dim3((unsigned)((n + kEpiRows - 1) / kEpiRows)),
-                     dim3(64 * kEpiRows), klds, st, ea);
+                     dim3(64 * kEpiRows), 0, st, ea);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }
@@ -1070,8 +1056,7 @@ static int launch_reduce(gwl_event* e, const double* params, int64_t n, int ld, 
     ea.esc_coeff = e->esc_coeff;
     ea.esc_tol = e->esc_tol;
   }
-  const size_t klds = (ev.flags & GWL_DISTANCE_MARG) ? (size_t)(ev.sp.nx + ev.sp.ny + 8) * sizeof(double) : 0;
-  hipLaunchKernelGGL(k_epi_plain, dim3((unsigned)((n + 127) / 128)), dim3(128), klds, st, ea);
+  hipLaunchKernelGGL(k_epi_plain, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, ea);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }
@@ -1372,12 +1357,8 @@ int multi_launch_epi(gwl_multi* m, hipStream_t st) {
   ea.block_row0 = m->d_block_row0;
   ea.n_blocks = m->d_n_blocks;
   ea.ld = GWL_NPARAM;
-  size_t klds = 0;
-  for (auto* ev : m->events)
-    if (ev->dev.flags & GWL_DISTANCE_MARG)
-      klds = std::max(klds, (size_t)(ev->dev.sp.nx + ev->dev.sp.ny + 8) * sizeof(double));
   const size_t grid = m->capturing ? m->max_blocks : (size_t)std::max(1, m->n_blocks);
-  hipLaunchKernelGGL(k_epi_time_multi, dim3((unsigned)grid), dim3(64 * kEpiRows), klds, st, ea);
+  hipLaunchKernelGGL(k_epi_time_multi, dim3((unsigned)grid), dim3(64 * kEpiRows), 0, st, ea);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }

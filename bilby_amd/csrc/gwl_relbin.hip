@@ -789,11 +789,8 @@ __global__ __launch_bounds__(128) void k_mb_fft_sum(const double* part, long lon
 
 // One thread per row: base.py:448-477 on the summed inner products.
 __global__ __launch_bounds__(128) void k_relbin_epi(RelbinArgs a) {
-  extern __shared__ double knots[];
   const EvDev& ev = a.ev;
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
-  if (dist) stage_knots(ev, knots);
-  __syncthreads();
   const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= a.n) return;
   const double dh_re = a.sums[3 * r + 0], dh_im = a.sums[3 * r + 1], h2 = a.sums[3 * r + 2];
@@ -809,9 +806,9 @@ __global__ __launch_bounds__(128) void k_relbin_epi(RelbinArgs a) {
   double ll;
   if (dist) {
     const double hs = a.params[r * a.ld + GWL_P_LUMINOSITY_DISTANCE] / ev.dref;
-    const double dd = (ev.flags & GWL_PHASE_MARG) ? hypot(dh_re, dh_im) * hs : dh_re * hs;
-    const SplineY yy = spline_y(ev, knots + ev.sp.nx + 4, h2 * hs * hs);
-    ll = spline_x(ev, knots, yy, dd);
+    const double dd = (ev.flags & GWL_PHASE_MARG) ? cabs2d(dh_re, dh_im) * hs : dh_re * hs;
+    const SplineY yy = spline_y(ev.sp, h2 * hs * hs);
+    ll = spline_x(ev.sp, yy, dd);
   } else if (ev.flags & GWL_PHASE_MARG) {
     ll = ln_i0(hypot(dh_re, dh_im)) - h2 / 2.0;
   } else {
@@ -950,8 +947,6 @@ int eval_time_tiles(gwl_event* ev, const WinBasis& win, void** ws, size_t* ws_by
   a.sums = reinterpret_cast<double*>(w + ((size_t)tile * sizeof(RelRow) + 255) / 256 * 256);
   void* opa = win_a(win, *tws);
   void* c = win_c(win, *tws, tile);
-  const size_t lds = (ev->dev.flags & GWL_DISTANCE_MARG)
-                         ? (size_t)(ev->dev.sp.nx + ev->dev.sp.ny + 8) * 8 : 0;
   for (long long r0 = 0; r0 < n; r0 += tile) {
     const long long nt = std::min(tile, n - r0);
     a.params = params + r0 * ld;
@@ -964,7 +959,7 @@ int eval_time_tiles(gwl_event* ev, const WinBasis& win, void** ws, size_t* ws_by
     GWL_HIP_CHECK(hipGetLastError());
     if (int rc = kernel(a, opa)) return rc;
     if (a.aux) {  // the inner products at the row's own time
-      hipLaunchKernelGGL(k_relbin_epi, dim3(g128), dim3(128), lds, st, a);
+      hipLaunchKernelGGL(k_relbin_epi, dim3(g128), dim3(128), 0, st, a);
       GWL_HIP_CHECK(hipGetLastError());
     }
     if (int rc = win_finish(ev, win, opa, fp64, c, nt, a.params, ld, a.sums, valid_of(a.rows),
@@ -1173,8 +1168,6 @@ static int relbin_eval_impl(gwl_relbin* rb, const double* params, int64_t n, int
   a.sums = reinterpret_cast<double*>(w + ((size_t)n * sizeof(gwl::RelRow) + 255) / 256 * 256);
   a.out = out;
   a.aux = aux;
-  const size_t lds = (ev->dev.flags & GWL_DISTANCE_MARG)
-                         ? (size_t)(ev->dev.sp.nx + ev->dev.sp.ny + 8) * 8 : 0;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (int rc = gwl::timing_begin(ev, st)) return rc;
   if (timem) {
@@ -1200,7 +1193,7 @@ static int relbin_eval_impl(gwl_relbin* rb, const double* params, int64_t n, int
   const int rc = precision == GWL_FP64 ? gwl::launch_relbin_nd<double>(a, ev->dev.nd, st)
                                        : gwl::launch_relbin_nd<float>(a, ev->dev.nd, st);
   if (rc != GWL_OK) return rc;
-  hipLaunchKernelGGL(gwl::k_relbin_epi, dim3(g128), dim3(128), lds, st, a);
+  hipLaunchKernelGGL(gwl::k_relbin_epi, dim3(g128), dim3(128), 0, st, a);
   GWL_HIP_CHECK(hipGetLastError());
   return gwl::timing_end(ev, st);
 }
@@ -1544,8 +1537,6 @@ static int mb_eval_impl(gwl_mb* mb, const double* params, int64_t n, int32_t ld,
   m.rows_n = n;
   m.rows = a.rows;
   m.sums = a.sums;
-  const size_t lds = (ev->dev.flags & GWL_DISTANCE_MARG)
-                         ? (size_t)(ev->dev.sp.nx + ev->dev.sp.ny + 8) * 8 : 0;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (int rc = gwl::timing_begin(ev, st)) return rc;
   if (timem) {
@@ -1576,7 +1567,7 @@ static int mb_eval_impl(gwl_mb* mb, const double* params, int64_t n, int32_t ld,
                                        : gwl::launch_mb_nd<float>(m, ev->dev.nd, st);
   if (rc != GWL_OK) return rc;
   if (int rf = gwl::mb_fft_launch(mb, a.rows, n, a.sums, st)) return rf;
-  hipLaunchKernelGGL(gwl::k_relbin_epi, dim3(g128), dim3(128), lds, st, a);
+  hipLaunchKernelGGL(gwl::k_relbin_epi, dim3(g128), dim3(128), 0, st, a);
   GWL_HIP_CHECK(hipGetLastError());
   return gwl::timing_end(ev, st);
 }

@@ -629,14 +629,7 @@ template <typename T>
 __global__ __launch_bounds__(64 * kRoqEpiRows) void k_roq_epi(RoqDev rd, const T* Z,
                                                               const RoqRow* rows, long long n,
                                                               double* out) {
-  extern __shared__ double knots[];
   const bool dist = (rd.flags & GWL_DISTANCE_MARG) != 0;
-  if (dist) {
-    const int nx4 = rd.sp.nx + 4, ny4 = rd.sp.ny + 4;
-    for (int i = threadIdx.x; i < nx4; i += blockDim.x) knots[i] = rd.sp.tx[i];
-    for (int i = threadIdx.x; i < ny4; i += blockDim.x) knots[nx4 + i] = rd.sp.ty[i];
-  }
-  __syncthreads();
   const int lane = threadIdx.x & 63;
   const long long r = (long long)blockIdx.x * kRoqEpiRows + (threadIdx.x >> 6);
   if (r >= n) return;
@@ -648,34 +641,10 @@ __global__ __launch_bounds__(64 * kRoqEpiRows) void k_roq_epi(RoqDev rd, const T
   const T* zr = Z + (size_t)r * rd.Np;
   const double hs = rr.hscale;
   const double hh = rr.hh;
-  double yy_by[4] = {0, 0, 0, 0};
-  int yy_ly = 3;
-  bool yy_in = false;
-  if (dist) {
-    const double y = hh * hs * hs;
-    yy_in = (y >= rd.sp.ymin && y <= rd.sp.ymax);
-    if (yy_in) {
-      yy_ly = knot_interval(knots + rd.sp.nx + 4, rd.sp.ny, y);
-      bspline3(knots + rd.sp.nx + 4, yy_ly, y, yy_by);
-    }
-  }
+  SplineY yy;
+  if (dist) yy = spline_y(rd.sp, hh * hs * hs);
   auto lnl_of = [&](double xr, double xi) -> double {
-    if (dist) {
-      const double d = (rd.flags & GWL_PHASE_MARG) ? hypot(xr, xi) * hs : xr * hs;
-      if (!yy_in || !(d >= rd.sp.xmin && d <= rd.sp.xmax)) return -INFINITY;
-      const int lx = knot_interval(knots, rd.sp.nx, d);
-      double bx[4];
-      bspline3(knots, lx, d, bx);
-      const double* c = rd.sp.c + (size_t)(lx - 3) * rd.sp.ny + (yy_ly - 3);
-      double s = 0.0;
-      for (int i = 0; i < 4; ++i) {
-        const double* ci = c + (size_t)i * rd.sp.ny;
-        s += bx[i] * (yy_by[0] * ci[0] + yy_by[1] * ci[1] + yy_by[2] * ci[2] + yy_by[3] * ci[3]);
-      }
-      return s;
-    }
-    if (rd.flags & GWL_PHASE_MARG) return ln_i0(hypot(xr, xi)) - hh / 2.0;
-    return xr - hh / 2.0;
+    return epi_value(rd.flags, rd.sp, yy, hh, hs, xr, xi);
   };
   auto dh_at = [&](double toff, double extra, bool single, bool& ok, double& sr, double& si) {
     ok = roq_dh_at(rd, zr, rr, toff, extra, single, sr, si);
@@ -701,23 +670,9 @@ __global__ __launch_bounds__(64 * kRoqEpiRows) void k_roq_epi(RoqDev rd, const T
     dh_at(tj - rd.start, rr.jitter, false, ok, sr, si);
     double v = ok ? lnl_of(sr, si) : -INFINITY;
     if (rd.tpd) v += time_log_density(rd.tpd, rd.tp_t0, rd.tp_ih, rd.tp_n, t);
-    if (v > m) {
-      s = (m > -INFINITY ? s * exp(m - v) : 0.0) + 1.0;
-      m = v;
-    } else if (v > -INFINITY) {
-      s += exp(v - m);
-    }
+    lse_push(m, s, v);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const double mo = __shfl_xor(m, off, 64), so = __shfl_xor(s, off, 64);
-    const double mn = fmax(m, mo);
-    if (mn > -INFINITY)
-      s = (m > -INFINITY ? s * exp(m - mn) : 0.0) + (mo > -INFINITY ? so * exp(mo - mn) : 0.0);
-    else
-      s = 0.0;
-    m = mn;
-  }
+  lse_wave(m, s);
   if (lane == 0) {
     const double b = rd.tpd ? rd.dtc : rd.dtc / (rd.tmax - rd.tmin);
     out[r] = (m > -INFINITY) ? log(b * s) + m : -INFINITY;
@@ -1021,25 +976,9 @@ int gwl_roq_set_distance_spline(gwl_roq* e, int32_t nx, int32_t ny, const double
     return GWL_E_INVALID;
   }
   GWL_HIP_CHECK(hipSetDevice(e->ctx->device));
-  const size_t n = (size_t)(nx + 4) + (ny + 4) + (size_t)nx * ny;
-  if (e->spline) (void)hipFree(e->spline);
-  e->spline = nullptr;
-  GWL_HIP_CHECK(hipMalloc(&e->spline, n * sizeof(double)));
-  GWL_HIP_CHECK(hipMemcpy(e->spline, tx, (nx + 4) * sizeof(double), hipMemcpyHostToDevice));
-  GWL_HIP_CHECK(hipMemcpy(e->spline + nx + 4, ty, (ny + 4) * sizeof(double), hipMemcpyHostToDevice));
-  GWL_HIP_CHECK(hipMemcpy(e->spline + nx + 4 + ny + 4, coeffs, (size_t)nx * ny * sizeof(double),
-                          hipMemcpyHostToDevice));
-  SplineDev sp;
-  sp.tx = e->spline;
-  sp.ty = e->spline + nx + 4;
-  sp.c = e->spline + nx + 4 + ny + 4;
-  sp.nx = nx;
-  sp.ny = ny;
-  sp.xmin = bbox[0];
-  sp.xmax = bbox[1];
-  sp.ymin = bbox[2];
-  sp.ymax = bbox[3];
-  e->dev.sp = sp;
+  size_t bytes = 0;
+  if (int rc = spline_upload(nx, ny, tx, ty, coeffs, bbox, &e->spline, &bytes, &e->dev.sp))
+    return rc;
   e->has_spline = true;
   return GWL_OK;
 }
@@ -1084,13 +1023,12 @@ int gwl_roq_eval(gwl_roq* e, const double* params, int64_t n, int32_t ld, int32_
   if (int rc = roq_prep_gemm(e, params, n, ld, mode, st, &Cv, &rows)) return rc;
   const RoqDev& rd = e->dev;
   const char* Cp = static_cast<const char*>(Cv);
-  const size_t klds = (rd.flags & GWL_DISTANCE_MARG) ? (size_t)(rd.sp.nx + rd.sp.ny + 8) * 8 : 0;
   const dim3 eg((unsigned)((n + kRoqEpiRows - 1) / kRoqEpiRows));
   if (mode == ROQ_FP64)
-    hipLaunchKernelGGL(k_roq_epi<double>, eg, dim3(64 * kRoqEpiRows), klds, st, rd,
+    hipLaunchKernelGGL(k_roq_epi<double>, eg, dim3(64 * kRoqEpiRows), 0, st, rd,
                        reinterpret_cast<const double*>(Cp), rows, (long long)n, out);
   else
-    hipLaunchKernelGGL(k_roq_epi<float>, eg, dim3(64 * kRoqEpiRows), klds, st, rd,
+    hipLaunchKernelGGL(k_roq_epi<float>, eg, dim3(64 * kRoqEpiRows), 0, st, rd,
                        reinterpret_cast<const float*>(Cp), rows, (long long)n, out);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;

@@ -461,10 +461,8 @@ __global__ __launch_bounds__(64 * kWaves, 4) void k_time_w(TimeWArgs a) {
   float2* tw2 = reinterpret_cast<float2*>(wt + kWP);               // [7][8]
   float2* tw3 = tw2 + kTw2;                                        // [7][64]
   float2* xch = tw3 + kTw3;                                        // [kWaves][kXch]
-  double* knots = reinterpret_cast<double*>(xch + kWaves * kXch);  // tx, ty
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
   init_row_tables(tw2, tw3, wt, ev.N, ev.jlo);
-  if (a.fused && dist) stage_knots(ev, knots);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -493,7 +491,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void k_time_w(TimeWArgs a) {
   const double norm = 4.0 / ev.T;
   const double hh = rw.hh * norm, hs = rw.hscale, jit = rw.jitter;
   SplineY yy;
-  if (dist) yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
+  if (dist) yy = spline_y(ev.sp, hh * hs * hs);
   double m = -INFINITY, sum = 0.0;
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
@@ -502,7 +500,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void k_time_w(TimeWArgs a) {
       const int j = ev.jlo + jj;
       const double t = (ev.start + (double)(j + 1) * ev.tstep) + jit;
       if (t >= ev.tmin && t <= ev.tmax)
-        lse_push(m, sum, epi_value(ev, knots, yy, hh, hs, norm * accr[s], norm * acci[s]) +
+        lse_push(m, sum, epi_value(ev.flags, ev.sp, yy, hh, hs, norm * accr[s], norm * acci[s]) +
                              time_log_weight(ev, t));
     }
   }
@@ -696,10 +694,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
   float2* tw = reinterpret_cast<float2*>(lds_d);
   float2* tw3 = tw + kWP;
   float2* xch = tw3 + kTw3;
-  double* knots = reinterpret_cast<double*>(xch + kWaves * kXch);
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
   init_wave_tables(tw, tw3);
-  if (dist) stage_knots(ev, knots);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -774,7 +770,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
     }
     hh *= norm;
     SplineY yy;
-    if (dist) yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
+    if (dist) yy = spline_y(ev.sp, hh * hs * hs);
     double m = -INFINITY, sum = 0.0;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -783,7 +779,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
         const int j = ev.jlo + jj;
         const double t = (ev.start + (double)(j + 1) * ev.tstep) + jit;
         if (t >= ev.tmin && t <= ev.tmax)
-          lse_push(m, sum, epi_value(ev, knots, yy, hh, hs, norm * accr[cc][s],
+          lse_push(m, sum, epi_value(ev.flags, ev.sp, yy, hh, hs, norm * accr[cc][s],
                                      norm * acci[cc][s]) +
                                time_log_weight(ev, t));
       }
@@ -806,7 +802,6 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_cal_time_w64(CalTimeArgs a) 
   double2* tw = reinterpret_cast<double2*>(lds_d);
   double2* tw3 = tw + kWP;
   double2* xch = tw3 + kTw3;
-  double* knots = reinterpret_cast<double*>(xch + kWaves * kXch);
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
   for (int k = threadIdx.x; k < kWP; k += 64 * kWaves) {
     double sn, cs;
@@ -819,7 +814,6 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_cal_time_w64(CalTimeArgs a) 
     sincospi(-2.0 * (double)e / (double)kWP, &sn, &cs);
     tw3[k] = make_double2(cs, sn);
   }
-  if (dist) stage_knots(ev, knots);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -900,7 +894,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_cal_time_w64(CalTimeArgs a) 
     }
     hh *= norm;
     SplineY yy;
-    if (dist) yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
+    if (dist) yy = spline_y(ev.sp, hh * hs * hs);
     double m = -INFINITY, sum = 0.0;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -909,7 +903,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_cal_time_w64(CalTimeArgs a) 
         const int j = ev.jlo + jj;
         const double t = (ev.start + (double)(j + 1) * ev.tstep) + jit;
         if (t >= ev.tmin && t <= ev.tmax)
-          lse_push(m, sum, epi_value(ev, knots, yy, hh, hs, norm * accr[cc][s],
+          lse_push(m, sum, epi_value(ev.flags, ev.sp, yy, hh, hs, norm * accr[cc][s],
                                      norm * acci[cc][s]) +
                                time_log_weight(ev, t));
       }
@@ -1050,16 +1044,13 @@ int init_time_wave_tables(const EvDev& ev, double* tb, float2* dwa) {
 }
 
 size_t time_wave_lds_bytes(const EvDev& ev, bool fused) {
-  size_t b = (size_t)kWP * sizeof(double2) + (size_t)(kTw2 + kTw3 + kWaves * kXch) * sizeof(float2);
-  if (fused && (ev.flags & GWL_DISTANCE_MARG)) b += (size_t)(ev.sp.nx + ev.sp.ny + 8) * sizeof(double);
-  return b;
+  return (size_t)kWP * sizeof(double2) + (size_t)(kTw2 + kTw3 + kWaves * kXch) * sizeof(float2);
 }
 
-// k_cal_time_w: the 512-entry pass-2 table, tw3, the exchange buffers, knots
+// k_cal_time_w: the 512-entry pass-2 table, tw3, the exchange buffers
 // (float64 kernel: the same tables in float64)
 static size_t cal_time_lds_bytes(const EvDev& ev, bool fp64) {
   size_t b = (size_t)(kWP + kTw3 + kWaves * kXch) * (fp64 ? sizeof(double2) : sizeof(float2));
-  if (ev.flags & GWL_DISTANCE_MARG) b += (size_t)(ev.sp.nx + ev.sp.ny + 8) * sizeof(double);
   return b;
 }
 

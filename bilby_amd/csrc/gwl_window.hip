@@ -236,11 +236,8 @@ constexpr int kWinEpiRows = 4;
 // window bins, running-max logsumexp with the uniform time prior weight
 // delta_tc / (t_max - t_min).
 __global__ __launch_bounds__(64 * kWinEpiRows) void k_win_epi(WinEpiArgs a) {
-  extern __shared__ double knots[];
   const EvDev& ev = a.ev;
   const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
-  if (dist) stage_knots(ev, knots);
-  __syncthreads();
   const long long r = (long long)blockIdx.x * kWinEpiRows + (threadIdx.x >> 6);
   if (r >= a.n) return;
   const int lane = threadIdx.x & 63;
@@ -253,7 +250,7 @@ __global__ __launch_bounds__(64 * kWinEpiRows) void k_win_epi(WinEpiArgs a) {
   const double hs = dist ? p[GWL_P_LUMINOSITY_DISTANCE] / ev.dref : 1.0;
   const double jit = (ev.flags & GWL_JITTER_TIME) ? p[GWL_P_TIME_JITTER] : 0.0;
   SplineY yy;
-  if (dist) yy = spline_y(ev, knots + ev.sp.nx + 4, hh * hs * hs);
+  if (dist) yy = spline_y(ev.sp, hh * hs * hs);
   double m = -INFINITY, s = 0.0;
   for (int jj = lane; jj < a.L; jj += 64) {
     const double t = (a.start + (double)(a.j_first + jj + a.offset) * a.t_step) + jit;
@@ -270,7 +267,7 @@ __global__ __launch_bounds__(64 * kWinEpiRows) void k_win_epi(WinEpiArgs a) {
         xi += (double)crow[a.L + jj];
       }
     }
-    lse_push(m, s, epi_value(ev, knots, yy, hh, hs, xr, xi) + time_log_weight(ev, t));
+    lse_push(m, s, epi_value(ev.flags, ev.sp, yy, hh, hs, xr, xi) + time_log_weight(ev, t));
   }
   lse_wave(m, s);
   if (lane == 0) {
@@ -473,10 +470,8 @@ int win_finish(gwl_event* ev, const WinBasis& wb, const void* a, bool fp64, void
     GWL_HIP_CHECK(hipGetLastError());
     return GWL_OK;
   }
-  const size_t lds = (ev->dev.flags & GWL_DISTANCE_MARG)
-                         ? (size_t)(ev->dev.sp.nx + ev->dev.sp.ny + 8) * sizeof(double) : 0;
   hipLaunchKernelGGL(k_win_epi, dim3((unsigned)((n + kWinEpiRows - 1) / kWinEpiRows)),
-                     dim3(64 * kWinEpiRows), lds, st, e);
+                     dim3(64 * kWinEpiRows), 0, st, e);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }
