@@ -2,7 +2,7 @@
 
 For an event and a batch shape it times the candidate tiles (rows of the
 parameter batch per workgroup, target resident workgroups per CU; rows 0
-selects the wave-per-row TaylorF2 time transform where the event allows it,
+selects the block-projected TaylorF2 time transform where the event allows it,
 and the second number is then the target wavefronts per CU) on the
 device with HIP events, keeps the fastest, and caches the choice per
 (device, source model, marginalisation flags, detectors, bin-count bucket,
@@ -59,7 +59,7 @@ def set_tile(likelihood, rows_per_workgroup, workgroups_per_cu):
 
 
 def set_transform(likelihood, transform):
-    """0 automatic, 1 tiled, 2 wave per row (bilby_amd.abi)."""
+    """0 automatic, 1 tiled, 2 block-projected (bilby_amd.abi)."""
     check(LIB.gwl_event_set_transform(likelihood._event, int(transform)), "gwl_event_set_transform")
 
 

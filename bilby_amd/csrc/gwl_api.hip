@@ -696,7 +696,9 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
   const size_t bw = wave_tables ? ((size_t)N * 3 * sizeof(double) + n_el * sizeof(float2)) +
                                       hps.size() * sizeof(double) + 4096
                                 : 0;
-  e->data_bytes = b32 + b64 + bw + 1024;
+  const bool band = wave_tables && band_tables_wanted(ev);
+  const size_t bb = band ? band_table_bytes(ev) + 256 : 0;
+  e->data_bytes = b32 + b64 + bw + bb + 1024;
   if (hipMalloc(&e->data, e->data_bytes) != hipSuccess) {
     delete e;
     set_error("hipMalloc failed for event data");
@@ -720,6 +722,8 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
     ev.hps = reinterpret_cast<double*>(p);
     p += hps.size() * sizeof(double);
   }
+  char* const band_mem =
+      reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
   hipError_t err = hipSuccess;
   if (err == hipSuccess) err = hipMemcpy((void*)ev.dw64, dw64.data(), n_el * sizeof(double2), hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy((void*)ev.w64, w64.data(), n_el * sizeof(double), hipMemcpyHostToDevice);
@@ -733,7 +737,9 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
     return hip_fail(err, "gwl_event_create upload");
   }
   if (wave_tables) {
-    int rc = init_time_wave_tables(ev, const_cast<double*>(ev.tf2b), const_cast<float2*>(ev.dwa32));
+    int rc = band ? band_table_init(ev, band_mem) : GWL_OK;
+    if (rc == GWL_OK)
+      rc = init_time_wave_tables(ev, const_cast<double*>(ev.tf2b), const_cast<float2*>(ev.dwa32));
     if (rc != GWL_OK) {
       (void)hipFree(e->data);
       delete e;
@@ -1132,6 +1138,14 @@ int gwl_distance_table(gwl_ctx* ctx, const double* dist, const double* prior, in
   return GWL_OK;
 }
 
+// Parts of a row's work at ``steps`` sub-sequence steps an item: up to 16
+// groups of sub-sequences, or the block groups of the block-projected
+// transform.
+static int multi_groups(const gwl_multi* m, int Q, int steps) {
+  const int G = (Q + steps - 1) / steps;
+  return std::max(1, std::min(G, m->wave_path ? kBandGroups : std::min(Q, 16)));
+}
+
 int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
                      const double* const* params_dev, double* const* out_dev,
                      const int64_t* max_rows, gwl_multi** out) {
@@ -1147,7 +1161,7 @@ int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
   m->wave = events[0]->dev.approx;
   m->wave_path = true;
   for (int e = 0; e < n_events; ++e)
-    if (!events[e] || events[e]->dev.approx != GWL_TAYLORF2 || !events[e]->dev.tf2b)
+    if (!events[e] || !events[e]->dev.band32.uv)
       m->wave_path = false;
   size_t items = 0, blocks = 0;
   for (int e = 0; e < n_events; ++e) {
@@ -1169,22 +1183,22 @@ int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
     const int Q = ev->dev.N / 512;
     // sub-sequence steps per item: the event's tuned choice, else ~32
     const int st = ev->multi_steps > 0 ? ev->multi_steps : 32;
-    int G = (Q + st - 1) / st;
-    G = std::max(1, std::min(G, std::min(Q, 16)));
-    m->groups.push_back(G);
-    items += (size_t)((max_rows[e] + 3) / 4) * std::min(Q, 16);
+    m->groups.push_back(multi_groups(m, Q, st));
+    items += (size_t)((max_rows[e] + 7) / 8) * (m->wave_path ? kBandGroups : std::min(Q, 16));
     blocks += (size_t)((max_rows[e] + 3) / 4);
   }
   m->max_items = std::max<size_t>(items, 1);
   m->max_blocks = std::max<size_t>(blocks, 1);
-  // per-event partials for up to 16 groups
+  // per-event partials for up to 16 groups, or the block sums
   for (int e = 0; e < n_events; ++e) {
     const size_t L = (size_t)m->events[e]->dev.L;
     void* part = nullptr;
     double* hh = nullptr;
     const size_t rows = (size_t)std::max<int64_t>(1, m->max_rows[e]);
-    if (hipMalloc(&part, rows * 16 * L * sizeof(double2)) != hipSuccess ||
-        hipMalloc((void**)&hh, rows * 16 * sizeof(double)) != hipSuccess) {
+    const size_t part_bytes =
+        m->wave_path ? rows * band_multi_row_bytes() : rows * 16 * L * sizeof(double2);
+    if (hipMalloc(&part, part_bytes) != hipSuccess ||
+        (!m->wave_path && hipMalloc((void**)&hh, rows * 16 * sizeof(double)) != hipSuccess)) {
       if (part) (void)hipFree(part);
       m->parts.push_back(nullptr);
       m->hhs.push_back(nullptr);
@@ -1254,7 +1268,7 @@ int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
     gwl_multi_destroy(m);
     return rc;
   }
-  if ((m->wave_path ? multi_wave_lds_bytes() : multi_lds_bytes()) > ctx->lds_per_block) {
+  if ((m->wave_path ? band_multi_lds_bytes() : multi_lds_bytes()) > ctx->lds_per_block) {
     gwl_multi_destroy(m);
     set_error("multi-event tile exceeds the LDS of a workgroup");
     return GWL_E_UNSUPPORTED;
@@ -1267,9 +1281,7 @@ int gwl_multi_set_tile(gwl_multi* m, const int32_t* steps_per_item) {
   if (!m || !steps_per_item) { set_error("gwl_multi_set_tile: invalid argument"); return GWL_E_INVALID; }
   for (int e = 0; e < m->n_events; ++e) {
     const int Q = m->events[e]->dev.N / 512;
-    int st = steps_per_item[e];
-    int G = st > 0 ? (Q + st - 1) / st : (Q + 31) / 32;
-    m->groups[e] = std::max(1, std::min(G, std::min(Q, 16)));
+    m->groups[e] = multi_groups(m, Q, steps_per_item[e] > 0 ? steps_per_item[e] : 32);
   }
   GWL_HIP_CHECK(hipSetDevice(m->ctx->device));
   GWL_HIP_CHECK(hipMemcpy(m->d_groups, m->groups.data(), m->groups.size() * sizeof(int),

@@ -111,6 +111,16 @@ struct SplineDev {
   double xmin, xmax, ymin, ymax;
 };
 
+// Tables of the block-projected window transform (gwl_band.hip; uv null: none).
+struct BandDev {
+  const double2* uv;   // [N] (f^1/3, f^-1/3)
+  const double* lf;    // [N] ln f
+  const void* dw;      // [nd][N] d / S f^-7/6 exp(2 pi i n jd / N), complex
+  const void* u;       // [steps][64] block functions
+  const double2* v;    // [8][L] their transforms (even, odd function)
+  const double2* rot;  // [L] exp(-i pi (B - 1) kappa / N)
+};
+
 struct EvDev {
   int nd, nf, N, P, Q, logP;
   double T, fs, df, start;
@@ -131,11 +141,12 @@ struct EvDev {
   const float* w32;    // [nd][N]  sigma^2 / S
   const double2* dw64;
   const double* w64;
-  // TaylorF2 tables for the wave-per-row time transform (null otherwise):
+  // TaylorF2 tables of the time transforms (null otherwise):
   const double* tf2b;   // [N][3] (f^1/3, f^-1/3, ln f), decimated order
   const float2* dwa32;  // [nd][N] dw32 f^-7/6, decimated order
   const double* hps;    // [nd][N + 2] prefix sums of f^-7/3 sigma^2 / S over bins
                         //   0..N in natural order, hps[d][n] = sum of bins < n
+  BandDev band32;
   // Nyquist bin (n = N), kept apart from the power-of-two FFT range
   double dwN[GWL_MAX_DET][2];
   double wN[GWL_MAX_DET];
@@ -834,12 +845,12 @@ struct RowW {
   double hh;                   // sum over the support of |h|^2 sigma^2 / S
   double hscale, jitter;
   double cabs2[GWL_MAX_DET];   // |complex detector amplitude / sigma|^2, float64
-  // the wave-per-row transform's reference detector ref (the largest
+  // the window transform's reference detector ref (the largest
   // amplitude C_ref): its delay and the phase of C_ref enter the float64
   // phase, |C_ref| scales the result, and the other detectors (in index
   // order, ref skipped) carry rho_k = C_k / C_ref and rotate relative to it
-  float rre[GWL_MAX_DET - 1];
-  float rim[GWL_MAX_DET - 1];
+  double rre[GWL_MAX_DET - 1];
+  double rim[GWL_MAX_DET - 1];
   double amp;                  // |C_ref|
   double c4r;                  // c[4] - arg(C_ref) / 2 pi
   int kb, ke, valid, ref;

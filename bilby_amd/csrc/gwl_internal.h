@@ -54,7 +54,7 @@ struct gwl_event {
 
 namespace gwl {
 // one item of the multi-event work list: rows [row0, row0 + 8) of event e,
-// group g of its decimated sub-sequences
+// group g of its decimated sub-sequences (or of its blocks)
 struct MultiItem {
   int e;
   int g;
@@ -73,8 +73,8 @@ struct gwl_multi {
   std::vector<int> groups;              // G_e (groups of sub-sequences per row)
   std::vector<const double*> params;    // caller-owned device buffers
   std::vector<double*> outs;
-  std::vector<void*> parts;             // [max_rows][16][L] double2 per event
-  std::vector<double*> hhs;             // [max_rows][16] per event
+  std::vector<void*> parts;             // [max_rows][16][L] double2 per event (tiled)
+  std::vector<double*> hhs;             // [max_rows][16] per event (tiled)
   void* dev = nullptr;                  // device tables (events, pointers, items, blocks)
   size_t dev_bytes = 0;
   gwl::EvDev* d_evs = nullptr;
@@ -95,8 +95,8 @@ struct gwl_multi {
   bool captured = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  // TaylorF2 events with 512-point transforms: wave-per-row kernels, row
-  // constants [max_rows] per event
+  // TaylorF2 events with block-projected window transforms: row constants
+  // [max_rows] per event, parts hold the block sums
   bool wave_path = false;
   bool capturing = false;   // a capture records grids for the largest work list
   int n_blocks = 0;         // epilogue blocks of the current rows
@@ -140,14 +140,26 @@ int launch_epi_time(gwl_event* ev, const double* params, int64_t n, int ld, int 
                     const double2* part, const double* hhpart, double* out, hipStream_t stream,
                     const gwl::EvDev* slice = nullptr, double2* lse = nullptr, int first = 1,
                     int last = 1, const double* rinfo = nullptr);
-// wave-per-row TaylorF2 time transform (gwl_time_wave.hip)
-bool time_wave_eligible(const gwl_event* ev);
-int time_wave_groups(const gwl_event* ev, long long n);
-size_t time_wave_ws_bytes(const gwl_event* ev, int64_t rows);
-size_t time_wave_lds_bytes(const EvDev& ev, bool fused);
+// TaylorF2 row constants (gwl_time_wave.hip)
+int launch_rowconst(gwl_event* ev, const double* params, int64_t n, int ld, RowW* rows,
+                    hipStream_t stream);
+int multi_launch_rowconst(gwl_multi* m, hipStream_t stream);
 int init_time_wave_tables(const EvDev& ev, double* tf2b, float2* dwa32);
-int launch_time_wave(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
+// block-projected window transform (gwl_band.hip)
+bool band_tables_wanted(const EvDev& ev);
+size_t band_table_bytes(const EvDev& ev);
+int band_table_init(EvDev& ev, char* p);  // p: band_table_bytes of device memory
+bool band_eligible(const gwl_event* ev);
+size_t band_ws_bytes(const gwl_event* ev, int64_t rows);      // workspace taken
+size_t band_ws_min_bytes(const gwl_event* ev, int64_t rows);  // workspace it can do with
+int launch_band_eval(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
                      hipStream_t stream);
+size_t band_multi_row_bytes();
+size_t band_multi_lds_bytes();
+int band_multi_launch(gwl_multi* m, hipStream_t stream);
+constexpr int kBandItemRows = 8;   // rows per item of the multi-event list
+constexpr int kBandGroups = 8;     // parts a row can be cut into
+constexpr int kMultiEpiRows = 4;   // rows per block of the multi-event epilogue list
 size_t roww_bytes(int64_t rows);
 int launch_time_series(gwl_event* ev, const double* params, int64_t n, int ld, int precision,
                        double* dh, double* hh, hipStream_t stream);
@@ -160,8 +172,6 @@ int launch_cal_time(gwl_event* ev, const double* params, int64_t n, int ld, int 
                     const float2* cal, const double* calps, void* ws, double* per_curve,
                     double* out, hipStream_t stream, bool fp64 = false,
                     const float2* cal_lo = nullptr, const double2* wN = nullptr);
-size_t multi_wave_lds_bytes();
-int multi_launch_wave(gwl_multi* m, hipStream_t stream);
 }  // namespace gwl
 
 #define GWL_HIP_CHECK(expr)                                   \

@@ -472,7 +472,7 @@ __global__ __launch_bounds__(128) void k_epi_plain(EpiArgs a) {
 
 // Time-marginalised lnL: logsumexp over the prior window (base.py:794-820).
 // One wavefront per row, kEpiRows rows per workgroup.
-constexpr int kEpiRows = 4;
+constexpr int kEpiRows = kMultiEpiRows;
 
 // One wavefront finishes one row: sums the group partials, evaluates the
 // marginalised lnL at every window bin and reduces them with a running-max
@@ -1066,7 +1066,7 @@ static int eval_typed(gwl_event* e, const double* params, int64_t n, int ld, dou
                       double* aux, hipStream_t st) {
   const EvDev& ev = e->dev;
   if constexpr (std::is_same<R, float>::value && WAVE == GWL_TAYLORF2) {
-    if (time_wave_eligible(e)) return launch_time_wave(e, params, n, ld, out, st);
+    if (band_eligible(e)) return launch_band_eval(e, params, n, ld, out, st);
   }
   if (ev.flags & GWL_TIME_MARG) {
     // a window longer than one transform: slices of P bins, one pass each,
@@ -1116,11 +1116,9 @@ static int eval_nd(gwl_event* e, const double* params, int64_t n, int ld, double
 }
 
 size_t workspace_bytes_for(const gwl_event* e, int64_t rows, int precision) {
-  // a float32 evaluation on the wave-per-row transform uses that path's
-  // workspace only
-  if ((e->dev.flags & GWL_TIME_MARG) && precision == GWL_FP32 && e->dev.approx == GWL_TAYLORF2 &&
-      time_wave_eligible(e))
-    return time_wave_ws_bytes(e, rows);
+  // a float32 evaluation on the block-projected transform uses that path's
+  // workspace only, in as many passes as it takes
+  if (precision == GWL_FP32 && band_eligible(e)) return band_ws_min_bytes(e, rows);
   return workspace_bytes(e, rows);
 }
 
@@ -1136,7 +1134,7 @@ size_t workspace_bytes(const gwl_event* e, int64_t rows) {
         2LL * 8 * wpc * e->ctx->n_cu);
     size_t b = (size_t)bound * (std::min(ev.L, ev.P) * sizeof(double2) + sizeof(double)) +
                time_lse_bytes(rows) + (size_t)rows * 4 * sizeof(double) + 4096;
-    if (ev.approx == GWL_TAYLORF2 && ev.tf2b) b = std::max(b, time_wave_ws_bytes(e, rows));
+    if (ev.band32.uv) b = std::max(b, band_ws_bytes(e, rows));
     return b;
   }
   return reduce_ws_bytes(ev, rows) + 4096;
@@ -1271,15 +1269,17 @@ int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
     const EvDev& ev = m->events[e]->dev;
     const int Q = ev.N / kMultiP;
     const int G = m->groups[e];
-    const int tile = m->wave_path ? 4 : kMultiS;  // rows per item
-    for (long long r0 = 0; r0 < rows[e]; r0 += tile) {
+    static_assert(kBandItemRows == kMultiS, "rows per item");
+    // a row's work is cut by sub-sequences, or by its groups of blocks
+    const int parts = m->wave_path ? kBandGroups : Q, per = m->wave_path ? Q : 1;
+    for (long long r0 = 0; r0 < rows[e]; r0 += kMultiS) {
       for (int g = 0; g < G; ++g) {
         MultiItem it;
         it.e = e;
         it.g = g;
         it.row0 = r0;
         items.push_back(it);
-        cost.push_back(((long long)(g + 1) * Q) / G - ((long long)g * Q) / G);
+        cost.push_back((((long long)(g + 1) * parts) / G - ((long long)g * parts) / G) * per);
       }
     }
     for (long long r0 = 0; r0 < rows[e]; r0 += kEpiRows) {
@@ -1318,8 +1318,8 @@ int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
 // epilogue over every block the work list can hold.
 int multi_launch_raw(gwl_multi* m, hipStream_t st) {
   if (m->wave_path) {
-    if (int rc = multi_launch_wave(m, st)) return rc;
-    return multi_launch_epi(m, st);
+    if (int rc = multi_launch_rowconst(m, st)) return rc;
+    return band_multi_launch(m, st);
   }
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, m->d_counter);
   GWL_HIP_CHECK(hipGetLastError());

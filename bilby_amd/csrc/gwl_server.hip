@@ -531,8 +531,11 @@ int gwl_server_add_group(gwl_server* s, int32_t n, gwl_event* const* events, int
   int64_t b = (int64_t)u->multi->dev_bytes;
   for (int e = 0; e < n; ++e) {
     const int64_t L = events[e]->dev.L;
-    b += s->max_rows * 16 * (L * 16 + 8);
-    if (u->multi->wave_path) b += (int64_t)gwl::roww_bytes(s->max_rows);
+    if (u->multi->wave_path)
+      b += s->max_rows * (int64_t)gwl::band_multi_row_bytes() +
+           (int64_t)gwl::roww_bytes(s->max_rows);
+    else
+      b += s->max_rows * 16 * (L * 16 + 8);
   }
   s->device_bytes += b;
   return add_unit(s, u, n, first_id);
