@@ -11,7 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgwl.so")
 SOURCES = ["gwl_api.hip", "gwl_kernels.hip", "gwl_roq.hip", "gwl_time_wave.hip", "gwl_server.hip",
-           "gwl_band.hip", "gwl_relbin.hip", "gwl_calib.hip",
+           "gwl_band.hip", "gwl_inner.hip", "gwl_relbin.hip", "gwl_calib.hip",
            "gwl_roq_weights.hip", "gwl_window.hip", "gwl_noalloc.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

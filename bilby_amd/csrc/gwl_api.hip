@@ -669,8 +669,10 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
   // TaylorF2 with a 512-point time transform: tables of the wave-per-row
   // kernel, including prefix sums of f^-7/3 sigma^2 / S over bins 0..N
   const bool wave_tables = ev.approx == GWL_TAYLORF2 && (ev.flags & GWL_TIME_MARG) && ev.P == 512;
+  // (and, without time marginalisation, of the inner products)
+  const bool inner = ev.approx == GWL_TAYLORF2 && !(ev.flags & GWL_TIME_MARG);
   std::vector<double> hps;
-  if (wave_tables) {
+  if (wave_tables || inner) {
     hps.assign((size_t)nd * (N + 2), 0.0);
     for (int k = 0; k < nd; ++k) {
       double* ps = hps.data() + (size_t)k * (N + 2);
@@ -698,7 +700,8 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
                                 : 0;
   const bool band = wave_tables && band_tables_wanted(ev);
   const size_t bb = band ? band_table_bytes(ev) + 256 : 0;
-  e->data_bytes = b32 + b64 + bw + bb + 1024;
+  const size_t bi = inner ? inner_table_bytes(ev) + hps.size() * sizeof(double) + 512 : 0;
+  e->data_bytes = b32 + b64 + bw + bb + bi + 1024;
   if (hipMalloc(&e->data, e->data_bytes) != hipSuccess) {
     delete e;
     set_error("hipMalloc failed for event data");
@@ -721,20 +724,31 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
     p += n_el * sizeof(float2);
     ev.hps = reinterpret_cast<double*>(p);
     p += hps.size() * sizeof(double);
+  } else if (inner) {
+    p = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
+    ev.hps = reinterpret_cast<double*>(p);
+    p += hps.size() * sizeof(double);
   }
-  char* const band_mem =
+  char* const band_mem =  // (or the inner products' tables)
       reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
   hipError_t err = hipSuccess;
   if (err == hipSuccess) err = hipMemcpy((void*)ev.dw64, dw64.data(), n_el * sizeof(double2), hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy((void*)ev.w64, w64.data(), n_el * sizeof(double), hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy((void*)ev.dw32, dw32.data(), n_el * sizeof(float2), hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy((void*)ev.w32, w32.data(), n_el * sizeof(float), hipMemcpyHostToDevice);
-  if (err == hipSuccess && wave_tables)
+  if (err == hipSuccess && (wave_tables || inner))
     err = hipMemcpy((void*)ev.hps, hps.data(), hps.size() * sizeof(double), hipMemcpyHostToDevice);
   if (err != hipSuccess) {
     (void)hipFree(e->data);
     delete e;
     return hip_fail(err, "gwl_event_create upload");
+  }
+  if (inner) {
+    if (int rc = inner_table_init(ev, band_mem)) {
+      (void)hipFree(e->data);
+      delete e;
+      return rc;
+    }
   }
   if (wave_tables) {
     int rc = band ? band_table_init(ev, band_mem) : GWL_OK;

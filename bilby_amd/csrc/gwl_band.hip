@@ -35,6 +35,7 @@
 // us; 4096 rows of 16384 bins, three detectors 239 -> 137 us, and 62 us to
 // finish them, where the epilogue was part of the 239.
 #include "gwl_internal.h"
+#include "gwl_tf2_rows.h"
 
 #include <algorithm>
 #include <cmath>
@@ -76,8 +77,6 @@ __host__ __device__ __forceinline__ int band_steps(int N) {
   return s + (s & 1);
 }
 
-__device__ __forceinline__ double fract1(double x) { return __builtin_amdgcn_fract(x); }
-
 // The event fields the integrand reads.
 template <typename T>
 struct BandEv {
@@ -105,57 +104,27 @@ __device__ __forceinline__ BandEv<T> band_ev(const EvDev& ev) {
   return b;
 }
 
-// Row constants in the registers of a wavefront.  The integrand is
-// |C_r| exp(-2 pi i phi(f)) [conj(dw_r) + sum_k rho_k exp(-2 pi i f (dt_k - dt_r)) conj(dw_k)]
-// with r the row's reference detector (its largest amplitude) and phi(f) =
-// Psi(f) / 2pi + f dt_r - arg(C_r) / 2pi in float64, reduced to [0, 1) cycles
-// before the sin / cos; |C_r| scales the row's result.
+// Row constants in the registers of a wavefront, with the rotation of one
+// step and the detectors' tables, the reference detector's first.
 template <typename T, int ND>
-struct BandRow {
+struct BandRow : Tf2Row<T, ND> {
   static constexpr int NO = ND - 1;
-  double c[9];  // c[4] holds c4r
-  double dtr;
-  double dd[NO > 0 ? NO : 1];            // dt_k - dt_r
-  // C_k / C_r, and what rounding it left (a rounding here would shift the
-  // whole row's sum; those of single bins average out)
-  cplx<T> rho[NO > 0 ? NO : 1];
-  cplx<T> rlo[NO > 0 ? NO : 1];
-  cplx<T> w[NO > 0 ? NO : 1];            // exp(-2 pi i 4 df dd): one step
+  cplx<T> w[NO > 0 ? NO : 1];  // exp(-2 pi i 4 df dd): one step
   const cplx<T>* dwr;
   const cplx<T>* dwo[NO > 0 ? NO : 1];
-  int kb, ke;
 };
 
 template <typename T, int ND>
 __device__ __forceinline__ void band_row(const BandEv<T>& ev, const RowW& rw, BandRow<T, ND>& b) {
-  constexpr int NO = ND - 1;
+  tf2_row<T, ND>(rw, b);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) b.c[k] = rw.c[k];
-  b.c[4] = rw.c4r;
-  const int ref = rw.ref;
-  b.dtr = rw.dt[0];
-#pragma unroll
-  for (int d = 1; d < ND; ++d)
-    if (d == ref) b.dtr = rw.dt[d];
-#pragma unroll
-  for (int k = 0; k < NO; ++k) {
-    const int d = k < ref ? k : k + 1;
-    b.dd[k] = (k < ref ? rw.dt[k] : rw.dt[k + 1]) - b.dtr;
-    const double2 w = expm2pi(fract1((4.0 * ev.df) * b.dd[k]));
-    b.w[k] = cmk<cplx<T>>((T)w.x, (T)w.y);
-    // the rounded step w (1 + eps) turns step j of a chunk by (1 + j eps):
-    // taken out on average, 1 - (kChunk - 1) / 2 eps
-    const double hc = 0.5 * (kChunk - 1);
-    const double er = 1.0 - hc * (w.x * (double)b.w[k].x + w.y * (double)b.w[k].y - 1.0);
-    const double ei = -hc * (w.x * (double)b.w[k].y - w.y * (double)b.w[k].x);
-    const double pr = rw.rre[k] * er - rw.rim[k] * ei, pi = rw.rre[k] * ei + rw.rim[k] * er;
-    b.rho[k] = cmk<cplx<T>>((T)pr, (T)pi);
-    b.rlo[k] = cmk<cplx<T>>((T)(pr - (double)b.rho[k].x), (T)(pi - (double)b.rho[k].y));
-    b.dwo[k] = ev.dw + (size_t)d * ev.M;
+  for (int k = 0; k < ND - 1; ++k) {
+    double2 corr = make_double2(1.0, 0.0);
+    b.w[k] = tf2_rotation<T>((4.0 * ev.df) * b.dd[k], 0.5 * (kChunk - 1), corr);
+    tf2_rho<T, ND>(rw, k, corr, b);
+    b.dwo[k] = ev.dw + (size_t)(k < b.ref ? k : k + 1) * ev.M;
   }
-  b.dwr = ev.dw + (size_t)ref * ev.M;
-  b.kb = rw.kb;
-  b.ke = rw.ke;
+  b.dwr = ev.dw + (size_t)b.ref * ev.M;
 }
 
 // What two steps read: the basis, the block function and the data of the
@@ -168,48 +137,30 @@ struct BandIn {
   cplx<T> d[SHARED ? 1 : R][ND][2];
 };
 
-// Uniform base plus a 32-bit byte offset: the load's own addressing does the sum.
-template <typename V>
-__device__ __forceinline__ V band_at(const void* base, unsigned off) {
-  return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + off);
-}
-
-template <typename C>
-__device__ __forceinline__ void band_pair(const C* p, unsigned off, C* to) {
-  if constexpr (sizeof(C) == 8) {
-    const float4 v = band_at<float4>(p, off);
-    to[0] = cmk<C>(v.x, v.y);
-    to[1] = cmk<C>(v.z, v.w);
-  } else {
-    to[0] = band_at<C>(p, off);
-    to[1] = band_at<C>(p, off + sizeof(C));
-  }
-}
-
 // ep: the pair's element (g S + s) / 2 * 64 + lane, sp: s / 2 * 64 + lane.
 template <typename T, int ND, int R, bool SHARED>
 __device__ __forceinline__ void band_load(const BandEv<T>& ev, const BandRow<T, ND>* b,
                                           unsigned ep, unsigned sp, int lane,
                                           BandIn<T, ND, R, SHARED>& in) {
   const unsigned e = 2 * ep - (unsigned)lane;
-  in.uv[0] = band_at<double2>(ev.uv, e * 16u);
-  in.uv[1] = band_at<double2>(ev.uv, e * 16u + 1024u);
-  in.lf = band_at<double2>(ev.lf, ep * 16u);
+  in.uv[0] = load_at<double2>(ev.uv, e * 16u);
+  in.uv[1] = load_at<double2>(ev.uv, e * 16u + 1024u);
+  in.lf = load_at<double2>(ev.lf, ep * 16u);
   if constexpr (sizeof(T) == 4) {
-    const float2 u = band_at<float2>(ev.u, sp * 8u);
+    const float2 u = load_at<float2>(ev.u, sp * 8u);
     in.u[0] = u.x;
     in.u[1] = u.y;
   } else {
-    const double2 u = band_at<double2>(ev.u, sp * 16u);
+    const double2 u = load_at<double2>(ev.u, sp * 16u);
     in.u[0] = u.x;
     in.u[1] = u.y;
   }
 #pragma unroll
   for (int r = 0; r < (SHARED ? 1 : R); ++r) {
-    band_pair(b[r].dwr, ep * (unsigned)(2 * sizeof(cplx<T>)), in.d[r][0]);
+    load_pair(b[r].dwr, ep * (unsigned)(2 * sizeof(cplx<T>)), in.d[r][0]);
 #pragma unroll
     for (int k = 0; k < ND - 1; ++k)
-      band_pair(b[r].dwo[k], ep * (unsigned)(2 * sizeof(cplx<T>)), in.d[r][k + 1]);
+      load_pair(b[r].dwo[k], ep * (unsigned)(2 * sizeof(cplx<T>)), in.d[r][k + 1]);
   }
 }
 
@@ -219,22 +170,9 @@ __device__ __forceinline__ cplx<T> band_value(const BandRow<T, ND>& b, cplx<T>* 
                                               const cplx<T> (*d)[2], int i, int n, double u,
                                               double v, double lf) {
   using C = cplx<T>;
-  // c0 v^5 + c1 v^3 + c2 v^2 + c3 v + c4r + c5 u + c6 u^2 + dt_r u^3 + (c7 + c8 u) ln f
-  double a = fma(b.c[0], v * v, b.c[1]);
-  a = fma(a, v, b.c[2]);
-  a = fma(a, v, b.c[3]);
-  double s = fma(a, v, b.c[4]);
-  s = fma(fma(fma(b.dtr, u, b.c[6]), u, b.c[5]), u, s);
-  s = fma(fma(b.c[8], u, b.c[7]), lf, s);
-  C y = cmk<C>(d[0][i].x, -d[0][i].y);
+  C x = tf2_product<T, ND>(tf2_cycles<T, ND>(b, u, v, lf), rot, d, i);
 #pragma unroll
-  for (int k = 0; k < ND - 1; ++k) {
-    const C dw = d[k + 1][i];
-    y.x = fma(rot[k].x, dw.x, fma(rot[k].y, dw.y, y.x));
-    y.y = fma(rot[k].y, dw.x, fma(-rot[k].x, dw.y, y.y));
-    rot[k] = cmul(rot[k], b.w[k]);
-  }
-  C x = cmul(expm2pi((T)fract1(s)), y);
+  for (int k = 0; k < ND - 1; ++k) rot[k] = cmul_fma(rot[k], b.w[k]);
   if constexpr (MASK) {
     const bool in = n >= b.kb && n <= b.ke;
     x = cmk<C>(in ? x.x : (T)0, in ? x.y : (T)0);
@@ -276,12 +214,7 @@ __device__ __forceinline__ void band_groups(const BandEv<T>& ev, const BandRow<T
         re[r] = (V4){0, 0, 0, 0};
         im[r] = (V4){0, 0, 0, 0};
 #pragma unroll
-        for (int k = 0; k < NO; ++k)
-        {
-          const C e = expm2pi((T)fract1(f0 * b[r].dd[k]));
-          rot[r][k] = cmul(b[r].rho[k], e);
-          if constexpr (sizeof(T) == 4) rot[r][k] = cadd(rot[r][k], cmul(b[r].rlo[k], e));
-        }
+        for (int k = 0; k < NO; ++k) rot[r][k] = tf2_rotated<T, ND>(b[r], k, f0);
       }
       auto pair = [&](int j, const In& v) __attribute__((always_inline)) {
 #pragma unroll
@@ -333,53 +266,12 @@ __device__ __forceinline__ void band_groups(const BandEv<T>& ev, const BandRow<T
   }
 }
 
-// Rows of one workgroup sorted by reference detector (stable), so that the
-// two rows of a wavefront mostly read the detectors' tables in the same
-// order: the index (0 .. count - 1) of the row with rank k.  Lane l < 8 holds
-// row l's key.
-__device__ __forceinline__ int ranked_row(int key, int lane, int k) {
-  const unsigned long long below = (1ull << lane) - 1ull;
-  int rank = 0;
-#pragma unroll
-  for (int d = 0; d <= GWL_MAX_DET; ++d) {
-    const unsigned long long m = __ballot(key == d) & 0xffull;
-    rank += (d < key) ? __popcll(m) : (d == key ? __popcll(m & below) : 0);
-  }
-  const unsigned long long at = __ballot(lane < 8 && rank == k) & 0xffull;
-  return __builtin_ctzll(at | 0x100ull) & 7;
-}
-
-// The wavefront's rows: R consecutive rows of the workgroup's kBandWaves * R
-// in order of their reference detectors; returns how many are live.
-template <int R>
-__device__ __forceinline__ int band_pick_rows(const RowW* rows, long long row0, long long n,
-                                              int lane, int wid, long long* pick) {
-  if constexpr (R == 1) {
-    pick[0] = row0 + wid;
-    return pick[0] < n ? 1 : 0;
-  } else {
-    const long long mine = row0 + lane;
-    const int key = (lane < 8 && mine < n) ? rows[mine].ref : GWL_MAX_DET;
-    int live = 0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int at = __builtin_amdgcn_readfirstlane(ranked_row(key, lane, wid * R + r));
-      pick[r] = row0 + at;
-      if (pick[r] < n) ++live;  // dead rows rank last
-    }
-#pragma unroll
-    for (int r = 1; r < R; ++r)
-      if (r >= live) pick[r] = pick[0];
-    return live;
-  }
-}
-
 template <typename T, int ND, int R>
 __device__ __forceinline__ void band_rows(const EvDev& ev, const RowW* rows, long long row0,
                                           long long n, int g0, int g1, int sb, int se, double* out,
                                           size_t row_stride, int lane, int wid) {
   long long pick[R];
-  const int live = band_pick_rows<R>(rows, row0, n, lane, wid, pick);
+  const int live = pick_rows<R>(rows, row0, n, lane, wid, pick);
   if (live == 0) return;
   const BandEv<T> be = band_ev<T>(ev);
   BandRow<T, ND> b[R];
@@ -390,7 +282,7 @@ __device__ __forceinline__ void band_rows(const EvDev& ev, const RowW* rows, lon
     const RowW& rw = rows[pick[r]];
     band_row<T, ND>(be, rw, b[r]);
     nomask &= rw.nomask;
-    shared &= rw.ref == rows[pick[0]].ref;
+    shared &= b[r].ref == b[0].ref;
     o[r] = out + (size_t)pick[r] * row_stride;
   }
   if (nomask && shared)

@@ -121,6 +121,15 @@ struct BandDev {
   const double2* rot;  // [L] exp(-i pi (B - 1) kappa / N)
 };
 
+// Tables of the inner products without time marginalisation (gwl_inner.hip;
+// uv null: none), bins 0..N in natural order and zeros up to whole units.
+struct InnerDev {
+  const double2* uv;    // (f^1/3, f^-1/3)
+  const double2* lf;    // ln f, two bins each
+  const float2* dw32;   // [nd] d / S f^-7/6
+  const double2* dw64;
+};
+
 struct EvDev {
   int nd, nf, N, P, Q, logP;
   double T, fs, df, start;
@@ -147,6 +156,7 @@ struct EvDev {
   const double* hps;    // [nd][N + 2] prefix sums of f^-7/3 sigma^2 / S over bins
                         //   0..N in natural order, hps[d][n] = sum of bins < n
   BandDev band32;
+  InnerDev inner;
   // Nyquist bin (n = N), kept apart from the power-of-two FFT range
   double dwN[GWL_MAX_DET][2];
   double wN[GWL_MAX_DET];

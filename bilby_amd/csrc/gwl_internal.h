@@ -141,8 +141,9 @@ int launch_epi_time(gwl_event* ev, const double* params, int64_t n, int ld, int 
                     const gwl::EvDev* slice = nullptr, double2* lse = nullptr, int first = 1,
                     int last = 1, const double* rinfo = nullptr);
 // TaylorF2 row constants (gwl_time_wave.hip)
-int launch_rowconst(gwl_event* ev, const double* params, int64_t n, int ld, RowW* rows,
-                    hipStream_t stream);
+// (count: only rows r < *count exist; zero: cleared first)
+int launch_rowconst(const gwl_event* ev, const double* params, int64_t n, int ld, RowW* rows,
+                    hipStream_t stream, const int* count = nullptr, int* zero = nullptr);
 int multi_launch_rowconst(gwl_multi* m, hipStream_t stream);
 int init_time_wave_tables(const EvDev& ev, double* tf2b, float2* dwa32);
 // block-projected window transform (gwl_band.hip)
@@ -154,6 +155,13 @@ size_t band_ws_bytes(const gwl_event* ev, int64_t rows);      // workspace taken
 size_t band_ws_min_bytes(const gwl_event* ev, int64_t rows);  // workspace it can do with
 int launch_band_eval(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
                      hipStream_t stream);
+// TaylorF2 inner products without time marginalisation (gwl_inner.hip):
+// partials [units][n][2] of <d|h> / |C_r|
+int inner_units_of(const EvDev& ev);
+size_t inner_table_bytes(const EvDev& ev);
+int inner_table_init(EvDev& ev, char* p);
+int launch_inner(const gwl_event* ev, bool fp64, const RowW* rows, int64_t n, const int* count,
+                 double* part, hipStream_t stream);
 size_t band_multi_row_bytes();
 size_t band_multi_lds_bytes();
 int band_multi_launch(gwl_multi* m, hipStream_t stream);

@@ -63,13 +63,6 @@ __global__ __launch_bounds__(128) void k_sample_const(EvDev ev, const double* pa
   out[r] = sc;
 }
 
-// A workgroup evaluates S rows over the chunks blockIdx.x, blockIdx.x +
-// gridDim.x, ... of chunk bins each; every chunk's sums go to its own
-// partials, so the values do not depend on the grid.  In natural order
-// (no time marginalisation) a chunk outside the union of the rows' supports
-// [kb, ke] is skipped and its partials are not written: the epilogue sums
-// only the chunks that meet a row's own support, which that row's tile
-// always computes.
 // The sums of one chunk for the S rows of a tile (see k_reduce).
 template <typename R, int WAVE, int ND, int S, int NT>
 __device__ __forceinline__ void reduce_chunk(const RedArgs& a, long long n, int chunk,
@@ -159,14 +152,12 @@ __device__ __forceinline__ void reduce_chunk(const RedArgs& a, long long n, int 
   }
 }
 
-// A workgroup evaluates S rows over one chunk (LOOP false: chunk blockIdx.x)
-// or over the chunks blockIdx.x, blockIdx.x + gridDim.x, ... (LOOP true);
-// every chunk's sums go to its own partials, so the values do not depend
-// on the grid.  In natural order (no time marginalisation) a chunk outside
+// A workgroup evaluates S rows over one chunk; every chunk's sums go to its
+// own partials.  In natural order (no time marginalisation) a chunk outside
 // the union of the rows' supports [kb, ke] is skipped and its partials are
 // not written: the epilogue sums only the chunks that meet a row's own
 // support, which that row's tile always computes.
-template <typename R, int WAVE, int ND, int S, int NT, bool LOOP>
+template <typename R, int WAVE, int ND, int S, int NT>
 __global__ __launch_bounds__(NT) void k_reduce(RedArgs a) {
   __shared__ SampleConst sc[S];
   __shared__ SampleFast<R> sf[S];
@@ -176,14 +167,7 @@ __global__ __launch_bounds__(NT) void k_reduce(RedArgs a) {
   const long long n = live_rows(a.n, a.count);
   if (row0 >= n) return;  // uniform over the workgroup
   tile_prologue_load<R, S>(a.ev, a.rows, n, row0, sc, sf, band);
-  if constexpr (!LOOP) {
-    reduce_chunk<R, WAVE, ND, S, NT>(a, n, blockIdx.x, row0, sc, sf, band, red);
-  } else {
-    for (int chunk = blockIdx.x; chunk < a.nchunk; chunk += gridDim.x) {
-      reduce_chunk<R, WAVE, ND, S, NT>(a, n, chunk, row0, sc, sf, band, red);
-      __syncthreads();  // red is reused by the next chunk
-    }
-  }
+  reduce_chunk<R, WAVE, ND, S, NT>(a, n, blockIdx.x, row0, sc, sf, band, red);
 }
 
 // ------------------------------------------------------------------ k_time
@@ -381,6 +365,9 @@ struct EpiArgs {
   const double* rinfo;      // [n][4] hscale, jitter, valid from the transform (or null)
   int gstride;              // groups per row in part / hhpart (0: G)
   const SampleConst* rows;  // [n] row constants, or null (then computed here)
+  const RowW* roww;         // [n] row constants and k_inner's partials
+  const double2* part2;     // [units][n]
+  int units;
   // live rows and output slots: with count set only rows r < *count exist
   // and row r's results go to out[scatter[r]] (the float64 pass over the
   // escalated rows of a float32 evaluation)
@@ -410,11 +397,44 @@ __device__ inline double escalation_scale(unsigned flags, double dhr, double dhi
   return hypot(dhr, dhi) + hh;
 }
 
-// lnL from the summed inner products (base.py:448-477, 775-792); one thread
-// per row.
+// lnL from a row's <d|h>, <h|h> (base.py:448-477, 775-792) to output slot o,
+// with the row's escalation.
+__device__ __forceinline__ void epi_plain_row(const EpiArgs& a, long long r, long long o,
+                                              double dhr, double dhi, double hh, double hs,
+                                              int valid) {
+  const EvDev& ev = a.ev;
+  if (a.aux) {
+    a.aux[3 * o + 0] = dhr;
+    a.aux[3 * o + 1] = dhi;
+    a.aux[3 * o + 2] = hh;
+  }
+  if (!valid) {
+    a.out[o] = row_valid_sentinel();
+    return;
+  }
+  if (a.esc_count && a.esc_coeff * escalation_scale(ev.flags, dhr, dhi, hh, hs) > a.esc_tol) {
+    const int slot = atomicAdd(a.esc_count, 1);
+    a.esc_idx[slot] = (int)r;
+    const double* src = a.params + r * a.ld;
+    double* dst = a.esc_params + (size_t)slot * GWL_NPARAM;
+    for (int k = 0; k < GWL_NPARAM; ++k) dst[k] = src[k];
+  }
+  double ll;
+  if (ev.flags & GWL_DISTANCE_MARG) {
+    const double d = (ev.flags & GWL_PHASE_MARG) ? cabs2d(dhr, dhi) * hs : dhr * hs;
+    const SplineY yy = spline_y(ev.sp, hh * hs * hs);
+    ll = spline_x(ev.sp, yy, d);
+  } else if (ev.flags & GWL_PHASE_MARG) {
+    ll = ln_i0(hypot(dhr, dhi)) - hh / 2.0;
+  } else {
+    ll = dhr - hh / 2.0;
+  }
+  a.out[o] = ll;
+}
+
+// From k_reduce's chunks, one thread per row.
 __global__ __launch_bounds__(128) void k_epi_plain(EpiArgs a) {
   const EvDev& ev = a.ev;
-  const bool dist = (ev.flags & GWL_DISTANCE_MARG) != 0;
   const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= live_rows(a.n, a.count)) return;
   const long long o = a.scatter ? (long long)a.scatter[r] : r;
@@ -438,36 +458,24 @@ __global__ __launch_bounds__(128) void k_epi_plain(EpiArgs a) {
   }
   const double norm = 4.0 / ev.T;
   // accumulated sum h conj(d)/S; <d|h> = sum conj(h) d / S is its conjugate
-  const double dhr = norm * dr, dhi = -norm * di;
-  hh *= norm;
-  if (a.aux) {
-    a.aux[3 * o + 0] = dhr;
-    a.aux[3 * o + 1] = dhi;
-    a.aux[3 * o + 2] = hh;
+  epi_plain_row(a, r, o, norm * dr, -norm * di, hh * norm, sc.hscale, sc.valid);
+}
+
+// From k_inner's units (rows of one unit are contiguous), one thread per row.
+__global__ __launch_bounds__(64) void k_epi_inner(EpiArgs a) {
+  const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= live_rows(a.n, a.count)) return;
+  const long long o = a.scatter ? (long long)a.scatter[r] : r;
+  const RowW& rw = a.roww[r];
+  double dr = 0.0, di = 0.0;
+#pragma unroll 8
+  for (int u = 0; u < a.units; ++u) {
+    const double2 v = a.part2[(size_t)u * a.n + r];
+    dr += v.x;
+    di += v.y;
   }
-  if (!sc.valid) {
-    a.out[o] = row_valid_sentinel();
-    return;
-  }
-  if (a.esc_count && a.esc_coeff * escalation_scale(ev.flags, dhr, dhi, hh, sc.hscale) > a.esc_tol) {
-    const int slot = atomicAdd(a.esc_count, 1);
-    a.esc_idx[slot] = (int)r;
-    const double* src = a.params + r * a.ld;
-    double* dst = a.esc_params + (size_t)slot * GWL_NPARAM;
-    for (int k = 0; k < GWL_NPARAM; ++k) dst[k] = src[k];
-  }
-  double ll;
-  if (dist) {
-    const double hs = sc.hscale;
-    const double d = (ev.flags & GWL_PHASE_MARG) ? cabs2d(dhr, dhi) * hs : dhr * hs;
-    const SplineY yy = spline_y(ev.sp, hh * hs * hs);
-    ll = spline_x(ev.sp, yy, d);
-  } else if (ev.flags & GWL_PHASE_MARG) {
-    ll = ln_i0(hypot(dhr, dhi)) - hh / 2.0;
-  } else {
-    ll = dhr - hh / 2.0;
-  }
-  a.out[o] = ll;
+  const double norm = 4.0 / a.ev.T, amp = norm * rw.amp;
+  epi_plain_row(a, r, o, amp * dr, -amp * di, norm * rw.hh, rw.hscale, rw.valid);
 }
 
 // Time-marginalised lnL: logsumexp over the prior window (base.py:794-820).
@@ -1002,37 +1010,18 @@ static int launch_reduce(gwl_event* e, const double* params, int64_t n, int ld, 
   ra.rows = ws.rows;
   ra.count = count;
   const long long nblk = (n + S - 1) / S;
-  // chunk groups per tile: every chunk in parallel when the rows' supports
-  // span the band; with the ISCO termination TaylorF2 supports are short,
-  // most chunks lie outside every row's support and fewer, longer
-  // workgroups (one per tile once the tiles alone fill the CUs several
-  // times) avoid launching workgroups that skip them all
-  const long long target = 8LL * e->ctx->n_cu;
-  const int G = (WAVE != GWL_TAYLORF2 || !(ev.flags & GWL_TF2_END_ISCO))
-                    ? ra.nchunk
-                    : (int)std::max<long long>(1, std::min<long long>(
-                                                      ra.nchunk, (target + nblk - 1) / nblk));
   if (!count)
     if (int rc = timing_begin(e, st)) return rc;
   hipLaunchKernelGGL(k_sample_const, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, ev,
                      params, ld, (long long)n, ws.rows, count, esc ? ws.esc_count : nullptr,
                      scatter);
-  const dim3 grid(G, (unsigned)nblk);
-  if (G == ra.nchunk) {
-    if (S == 16)
-      hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 16, NT, false>), grid, dim3(NT), 0, st, ra);
-    else if (S == 4)
-      hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 4, NT, false>), grid, dim3(NT), 0, st, ra);
-    else
-      hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 8, NT, false>), grid, dim3(NT), 0, st, ra);
-  } else {
-    if (S == 16)
-      hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 16, NT, true>), grid, dim3(NT), 0, st, ra);
-    else if (S == 4)
-      hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 4, NT, true>), grid, dim3(NT), 0, st, ra);
-    else
-      hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 8, NT, true>), grid, dim3(NT), 0, st, ra);
-  }
+  const dim3 grid(ra.nchunk, (unsigned)nblk);
+  if (S == 16)
+    hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 16, NT>), grid, dim3(NT), 0, st, ra);
+  else if (S == 4)
+    hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 4, NT>), grid, dim3(NT), 0, st, ra);
+  else
+    hipLaunchKernelGGL((k_reduce<R, WAVE, ND, 8, NT>), grid, dim3(NT), 0, st, ra);
   GWL_HIP_CHECK(hipGetLastError());
   if (!count)
     if (int rc = timing_end(e, st)) return rc;
@@ -1057,6 +1046,66 @@ static int launch_reduce(gwl_event* e, const double* params, int64_t n, int ld, 
     ea.esc_tol = e->esc_tol;
   }
   hipLaunchKernelGGL(k_epi_plain, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, ea);
+  GWL_HIP_CHECK(hipGetLastError());
+  return GWL_OK;
+}
+
+// One pass of the TaylorF2 inner products (arguments as launch_reduce).
+struct InnerWs {
+  double* part;
+  RowW* rows;
+  double* esc_params;
+  int* esc_idx;
+  int* esc_count;
+};
+
+static size_t inner_ws(const EvDev& ev, long long n, char* p, InnerWs* w) {
+  size_t off = 0;
+  auto take = [&](size_t nb) {
+    const size_t at = off;
+    off += (nb + 255) / 256 * 256;
+    return p + at;
+  };
+  w->part = reinterpret_cast<double*>(take((size_t)n * inner_units_of(ev) * sizeof(double2)));
+  w->rows = reinterpret_cast<RowW*>(take((size_t)n * sizeof(RowW)));
+  w->esc_params = reinterpret_cast<double*>(take((size_t)n * GWL_NPARAM * sizeof(double)));
+  w->esc_idx = reinterpret_cast<int*>(take((size_t)n * sizeof(int)));
+  w->esc_count = reinterpret_cast<int*>(take(sizeof(int)));
+  return off;
+}
+
+static int launch_inner_pass(gwl_event* e, bool fp64, const double* params, int64_t n, int ld,
+                             double* out, double* aux, hipStream_t st, const int* count,
+                             const int* scatter, bool esc) {
+  InnerWs ws;
+  inner_ws(e->dev, n, reinterpret_cast<char*>(e->ws), &ws);
+  if (!count)
+    if (int rc = timing_begin(e, st)) return rc;
+  if (int rc = launch_rowconst(e, params, n, ld, ws.rows, st, count, esc ? ws.esc_count : nullptr))
+    return rc;
+  if (int rc = launch_inner(e, fp64, ws.rows, n, count, ws.part, st)) return rc;
+  if (!count)
+    if (int rc = timing_end(e, st)) return rc;
+  EpiArgs ea{};
+  ea.ev = e->dev;
+  ea.params = params;
+  ea.ld = ld;
+  ea.n = n;
+  ea.roww = ws.rows;
+  ea.part2 = reinterpret_cast<const double2*>(ws.part);
+  ea.units = inner_units_of(e->dev);
+  ea.out = out;
+  ea.aux = aux;
+  ea.count = count;
+  ea.scatter = scatter;
+  if (esc) {
+    ea.esc_count = ws.esc_count;
+    ea.esc_idx = ws.esc_idx;
+    ea.esc_params = ws.esc_params;
+    ea.esc_coeff = e->esc_coeff;
+    ea.esc_tol = e->esc_tol;
+  }
+  hipLaunchKernelGGL(k_epi_inner, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, ea);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }
@@ -1091,15 +1140,28 @@ static int eval_typed(gwl_event* e, const double* params, int64_t n, int ld, dou
     return GWL_OK;
   }
   const bool esc = std::is_same<R, float>::value && e->esc_coeff > 0.0;
-  if (int rc = launch_reduce<R, WAVE, ND>(e, params, n, ld, out, aux, st, nullptr, nullptr, esc))
-    return rc;
-  if (!esc) return GWL_OK;
-  // the escalated rows again in float64: same stream, no host round trip;
-  // the grid is sized for n rows and the kernels read the live count
-  const ReduceWs ws = reduce_ws(e, n);
-  e->esc_count_dev = ws.esc_count;
-  return launch_reduce<double, WAVE, ND>(e, ws.esc_params, n, GWL_NPARAM, out, aux, st,
-                                         ws.esc_count, ws.esc_idx, false);
+  if constexpr (WAVE == GWL_TAYLORF2) {
+    if (int rc = launch_inner_pass(e, std::is_same<R, double>::value, params, n, ld, out, aux, st,
+                                   nullptr, nullptr, esc))
+      return rc;
+    if (!esc) return GWL_OK;
+    InnerWs ws;
+    inner_ws(ev, n, reinterpret_cast<char*>(e->ws), &ws);
+    e->esc_count_dev = ws.esc_count;
+    return launch_inner_pass(e, true, ws.esc_params, n, GWL_NPARAM, out, aux, st, ws.esc_count,
+                             ws.esc_idx, false);
+  } else {
+    if (int rc = launch_reduce<R, WAVE, ND>(e, params, n, ld, out, aux, st, nullptr, nullptr,
+                                            esc))
+      return rc;
+    if (!esc) return GWL_OK;
+    // the escalated rows again in float64: same stream, no host round trip;
+    // the grid is sized for n rows and the kernels read the live count
+    const ReduceWs ws = reduce_ws(e, n);
+    e->esc_count_dev = ws.esc_count;
+    return launch_reduce<double, WAVE, ND>(e, ws.esc_params, n, GWL_NPARAM, out, aux, st,
+                                           ws.esc_count, ws.esc_idx, false);
+  }
 }
 
 template <typename R, int WAVE>
@@ -1136,6 +1198,10 @@ size_t workspace_bytes(const gwl_event* e, int64_t rows) {
                time_lse_bytes(rows) + (size_t)rows * 4 * sizeof(double) + 4096;
     if (ev.band32.uv) b = std::max(b, band_ws_bytes(e, rows));
     return b;
+  }
+  if (ev.approx == GWL_TAYLORF2) {
+    InnerWs ws;
+    return inner_ws(ev, rows, nullptr, &ws) + 4096;
   }
   return reduce_ws_bytes(ev, rows) + 4096;
 }

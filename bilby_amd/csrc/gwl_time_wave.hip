@@ -48,6 +48,8 @@ struct RowArgs {
   long long n;
   RowW* rows;
   double2* c64 = nullptr;  // [n][GWL_MAX_DET] float64 detector amplitudes, or null
+  const int* count = nullptr;  // if set: only rows r < *count exist (n bounds it)
+  int* zero = nullptr;         // cleared by the first thread
 };
 
 __device__ inline void rowconst_one(const EvDev& ev, const double* row, RowW* out,
@@ -122,7 +124,8 @@ __global__ __launch_bounds__(256) void k_rowconst(RowArgs a) {
   __shared__ Tf2Part t[kRowconstRows];
   const int k = threadIdx.x >> 1;
   const long long r = (long long)blockIdx.x * kRowconstRows + k;
-  const bool live = r < a.n;
+  const bool live = r < (a.count ? min(a.n, (long long)*a.count) : a.n);
+  if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0;
   if (live && (threadIdx.x & 1)) tf2_part(a.ev, a.params + r * a.ld, t[k]);
   __syncthreads();
   if (live && !(threadIdx.x & 1))
@@ -624,9 +627,9 @@ static size_t cal_time_lds_bytes(const EvDev& ev, bool fp64) {
   return b;
 }
 
-int launch_rowconst(gwl_event* e, const double* params, int64_t n, int ld, RowW* rows,
-                    hipStream_t st) {
-  RowArgs ra{e->dev, params, ld, n, rows};
+int launch_rowconst(const gwl_event* e, const double* params, int64_t n, int ld, RowW* rows,
+                    hipStream_t st, const int* count, int* zero) {
+  RowArgs ra{e->dev, params, ld, n, rows, nullptr, count, zero};
   hipLaunchKernelGGL(k_rowconst, dim3((unsigned)((n + kRowconstRows - 1) / kRowconstRows)),
                      dim3(256), 0, st, ra);
   GWL_HIP_CHECK(hipGetLastError());

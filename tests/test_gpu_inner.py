@@ -1,0 +1,45 @@
+"""GPU check of the tabled TaylorF2 inner products (gwl_inner.hip) against the
+FP64 oracle at the edges of its units of 1024 bins: less than one unit, a unit
+that holds the Nyquist bin alone, bands that start and end inside units, the
+ISCO cut, one to four detectors, one row and rows that do not fill a
+workgroup."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# duration, sampling rate, detectors, rows, ISCO cut
+CASES = [
+    (1.0, 512.0, ("H1",), 1, False),                     # 257 bins
+    (1.0, 2048.0, ("H1", "L1"), 3, False),               # 1025 bins: Nyquist in its own unit
+    (5.0, 2048.0, ("H1", "L1", "V1"), 9, True),          # 5121 bins
+    (8.0, 4096.0, ("H1", "L1", "V1", "K1"), 17, False),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_inner_products_match_oracle(case, precision):
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    from tests.helpers import draws_as_dicts, oracle_from_setup
+    duration, fs, dets, rows, isco = case
+    s = make_taylorf2_marginalised(n_draws=rows, seed=31, duration=duration,
+                                   sampling_frequency=fs, detectors=dets, chi_range=0.5,
+                                   time=False, distance=False, phase=False,
+                                   taylorf2_termination="isco" if isco else None)
+    if len(dets) > 1:  # bins inside one detector's mask only
+        s["interferometers"][1].minimum_frequency = 35.0
+        s["interferometers"][0].maximum_frequency = fs / 2 - 60.0
+    lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                    precision=precision)
+    out = lk.log_likelihood_ratio_batch(s["draws"])
+    olk, _ = oracle_from_setup(s)
+    ref = np.array([olk.log_likelihood_ratio(p) for p in draws_as_dicts(s["draws"], range(rows))])
+    # float64: sums of up to 5e4 terms of size |lnL| and below; float32: rows
+    # past the escalation bound are float64, the others within it
+    tol = 1e-10 * np.maximum(1.0, np.abs(ref)) if precision == "fp64" else 1e-3
+    assert np.all(np.abs(out - ref) < tol), np.abs(out - ref).max()
+    # a row's value does not depend on its slot or its partner
+    again = lk.log_likelihood_ratio_batch({k: v[::-1].copy() for k, v in s["draws"].items()})
+    assert np.array_equal(again[::-1], out)
