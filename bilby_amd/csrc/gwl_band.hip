@@ -33,7 +33,9 @@
 // SIMD).  Against a 512-point FFT of every sub-sequence in registers and LDS
 // (94 instructions a step): 1501 rows of 131072 bins, two detectors 740 -> 315
 // us; 4096 rows of 16384 bins, three detectors 239 -> 137 us, and 62 us to
-// finish them, where the epilogue was part of the 239.
+// finish them, where the epilogue was part of the 239.  float64, 509 rows of
+// 16384 bins, three detectors: 271 us (tiles of 8 rows through LDS
+// transforms, k_time) -> 47, and 17 to finish them.
 #include "gwl_internal.h"
 #include "gwl_tf2_rows.h"
 
@@ -90,8 +92,14 @@ struct BandEv {
 };
 
 template <typename T>
+__host__ __device__ __forceinline__ const BandDev& band_dev(const EvDev& ev) {
+  if constexpr (sizeof(T) == 4) return ev.band32;
+  else return ev.band64;
+}
+
+template <typename T>
 __device__ __forceinline__ BandEv<T> band_ev(const EvDev& ev) {
-  const BandDev& bd = ev.band32;
+  const BandDev& bd = band_dev<T>(ev);
   BandEv<T> b;
   b.uv = bd.uv;
   b.lf = reinterpret_cast<const double2*>(bd.lf);
@@ -476,7 +484,7 @@ __device__ __forceinline__ void band_finish_row(const EvDev& ev, const RowW& rw,
     if (t == 0) *out = row_valid_sentinel();
     return;
   }
-  const BandDev& bd = ev.band32;
+  const BandDev& bd = band_dev<T>(ev);
   double2* tw = x + NB * kPitch + NB / 16;
   const double norm = 4.0 / ev.T;
   const double hh = rw.hh * norm, hs = rw.hscale, jit = rw.jitter, amp = rw.amp * norm;
@@ -740,35 +748,40 @@ __global__ __launch_bounds__(256) void k_band_tables(EvDev ev, int jd, double2* 
   }
 }
 
+// The block functions are set up in extended precision: the float64 transform
+// takes them rounded once.
+using Real = long double;
+using Mat = std::vector<std::vector<Real>>;
+
 // Eigenvectors of a symmetric n x n matrix by cyclic Jacobi rotations, in
 // ascending order of the eigenvalues: vec[k][i].
-void jacobi(std::vector<std::vector<double>> a, std::vector<std::vector<double>>& vec) {
+void jacobi(Mat a, Mat& vec) {
   const int n = (int)a.size();
-  std::vector<std::vector<double>> v(n, std::vector<double>(n, 0.0));
-  for (int i = 0; i < n; ++i) v[i][i] = 1.0;
+  Mat v(n, std::vector<Real>(n, 0.0L));
+  for (int i = 0; i < n; ++i) v[i][i] = 1;
   for (int sweep = 0; sweep < 60; ++sweep) {
-    double off = 0.0, diag = 0.0;
+    Real off = 0, diag = 0;
     for (int i = 0; i < n; ++i)
       for (int j = 0; j < n; ++j) (i == j ? diag : off) += a[i][j] * a[i][j];
-    if (off <= 1e-34 * diag) break;
+    if (off <= 1e-40L * diag) break;
     for (int p = 0; p < n; ++p)
       for (int q = p + 1; q < n; ++q) {
-        if (a[p][q] == 0.0) continue;
-        const double th = (a[q][q] - a[p][p]) / (2.0 * a[p][q]);
-        const double t = (th >= 0 ? 1.0 : -1.0) / (std::fabs(th) + std::sqrt(th * th + 1.0));
-        const double c = 1.0 / std::sqrt(t * t + 1.0), s = t * c;
+        if (a[p][q] == 0) continue;
+        const Real th = (a[q][q] - a[p][p]) / (2 * a[p][q]);
+        const Real t = (th >= 0 ? 1.0L : -1.0L) / (std::fabs(th) + std::sqrt(th * th + 1));
+        const Real c = 1 / std::sqrt(t * t + 1), s = t * c;
         for (int k = 0; k < n; ++k) {
-          const double x = a[k][p], y = a[k][q];
+          const Real x = a[k][p], y = a[k][q];
           a[k][p] = c * x - s * y;
           a[k][q] = s * x + c * y;
         }
         for (int k = 0; k < n; ++k) {
-          const double x = a[p][k], y = a[q][k];
+          const Real x = a[p][k], y = a[q][k];
           a[p][k] = c * x - s * y;
           a[q][k] = s * x + c * y;
         }
         for (int k = 0; k < n; ++k) {
-          const double x = v[k][p], y = v[k][q];
+          const Real x = v[k][p], y = v[k][q];
           v[k][p] = c * x - s * y;
           v[k][q] = s * x + c * y;
         }
@@ -777,7 +790,7 @@ void jacobi(std::vector<std::vector<double>> a, std::vector<std::vector<double>>
   std::vector<int> order(n);
   for (int i = 0; i < n; ++i) order[i] = i;
   std::sort(order.begin(), order.end(), [&](int i, int j) { return a[i][i] < a[j][j]; });
-  vec.assign(n, std::vector<double>(n));
+  vec.assign(n, std::vector<Real>(n));
   for (int k = 0; k < n; ++k)
     for (int i = 0; i < n; ++i) vec[k][i] = v[i][order[k]];
 }
@@ -791,13 +804,13 @@ constexpr int kLeg = 48;  // Legendre terms (c <= 2 pi needs about 30)
 // with psi_p = sum_k beta_pk P_k the transform is
 // V_p(y) = sum_k beta_pk sqrt(2 (2k + 1)) (-i)^k j_k(c y).
 void band_functions(int NB, int B, int L, std::vector<double>& u, std::vector<double>& v) {
-  const double c = kPi * (double)L / (2.0 * (double)NB);
-  std::vector<std::vector<double>> beta(kNP, std::vector<double>(kLeg, 0.0));
+  const Real c = 3.14159265358979323846264338327950288L * L / (2 * NB);
+  Mat beta(kNP, std::vector<Real>(kLeg, 0.0L));
   for (int par = 0; par < 2; ++par) {
     const int n = kLeg / 2;
-    std::vector<std::vector<double>> a(n, std::vector<double>(n, 0.0)), vec;
+    Mat a(n, std::vector<Real>(n, 0.0L)), vec;
     for (int i = 0; i < n; ++i) {
-      const double k = 2 * i + par;
+      const Real k = 2 * i + par;
       a[i][i] = k * (k + 1) + c * c * (2 * k * k + 2 * k - 1) / ((2 * k - 1) * (2 * k + 3));
       if (i + 1 < n)
         a[i][i + 1] = a[i + 1][i] =
@@ -809,46 +822,47 @@ void band_functions(int NB, int B, int L, std::vector<double>& u, std::vector<do
   }
   u.assign((size_t)B * kNP, 0.0);
   for (int t = 0; t < B; ++t) {
-    const double x = (t - 0.5 * (B - 1)) / (0.5 * B);
-    double p0 = 1.0, p1 = x;
+    const Real x = (t - 0.5L * (B - 1)) / (0.5L * B);
+    Real p0 = 1, p1 = x, sum[kNP] = {0};
     for (int k = 0; k < kLeg; ++k) {
-      const double pk = p0 * std::sqrt(k + 0.5);
-      for (int p = k & 1; p < kNP; p += 2) u[(size_t)t * kNP + p] += beta[p][k] * pk;
-      const double p2 = ((2 * k + 3) * x * p1 - (k + 1) * p0) / (k + 2);
+      const Real pk = p0 * std::sqrt(k + 0.5L);
+      for (int p = k & 1; p < kNP; p += 2) sum[p] += beta[p][k] * pk;
+      const Real p2 = ((2 * k + 3) * x * p1 - (k + 1) * p0) / (k + 2);
       p0 = p1;
       p1 = p2;
     }
+    for (int p = 0; p < kNP; ++p) u[(size_t)t * kNP + p] = (double)sum[p];
   }
   v.assign((size_t)kNP * L, 0.0);
   for (int jj = 0; jj < L; ++jj) {
-    const double z = c * (double)(jj - L / 2) / (0.5 * L);
+    const Real z = c * (jj - L / 2) / (0.5L * L);
     // spherical Bessel functions by downward recurrence, sum (2k + 1) j_k^2 = 1
-    double jk[kLeg] = {0.0};
-    if (z == 0.0) {
-      jk[0] = 1.0;
+    Real jk[kLeg] = {0};
+    if (z == 0) {
+      jk[0] = 1;
     } else {
-      const double az = std::fabs(z);
-      long double hi = 0.0L, lo = 1e-300L, norm = 0.0L, val[kLeg] = {0.0L};
+      const Real az = std::fabs(z);
+      Real hi = 0, lo = 1e-300L, norm = 0, val[kLeg] = {0};
       for (int k = kLeg + 40; k >= 0; --k) {  // lo = j_k, hi = j_{k+1} (unnormalised)
         if (k < kLeg) val[k] = lo;
         norm += (2 * k + 1) * lo * lo;
-        const long double down = (2 * k + 1) / (long double)az * lo - hi;
+        const Real down = (2 * k + 1) / az * lo - hi;
         hi = lo;
         lo = down;
       }
-      const long double j0 = std::sin((long double)az) / az;
-      const long double j1 = j0 / az - std::cos((long double)az) / az;
-      long double sc = 1.0L / std::sqrt(norm);
-      const bool by0 = std::fabs((double)j0) > std::fabs((double)j1);
+      const Real j0 = std::sin(az) / az;
+      const Real j1 = j0 / az - std::cos(az) / az;
+      Real sc = 1 / std::sqrt(norm);
+      const bool by0 = std::fabs(j0) > std::fabs(j1);
       if ((by0 ? val[0] * j0 : val[1] * j1) < 0) sc = -sc;
       for (int k = 0; k < kLeg; ++k)
-        jk[k] = (double)(val[k] * sc) * ((z < 0 && (k & 1)) ? -1.0 : 1.0);
+        jk[k] = val[k] * sc * ((z < 0 && (k & 1)) ? -1 : 1);
     }
     for (int p = 0; p < kNP; ++p) {
-      double s = 0.0;
+      Real s = 0;
       for (int k = p & 1; k < kLeg; k += 2)
-        s += beta[p][k] * std::sqrt(2.0 * (2 * k + 1)) * (((k >> 1) & 1) ? -1.0 : 1.0) * jk[k];
-      v[((size_t)(p >> 1) * L + jj) * 2 + (p & 1)] = s;
+        s += beta[p][k] * std::sqrt((Real)(2 * (2 * k + 1))) * (((k >> 1) & 1) ? -1 : 1) * jk[k];
+      v[((size_t)(p >> 1) * L + jj) * 2 + (p & 1)] = (double)s;
     }
   }
 }
@@ -900,13 +914,14 @@ int init_band(EvDev& ev, BandDev& bd, char* p) {
 template <typename T>
 size_t band_bytes(const EvDev& ev) {
   const size_t S = band_steps<T>(ev.N), M = (size_t)BandTypes<T>::NB * 4 * S;
-  return M * 24 + ev.nd * M * sizeof(cplx<T>) + S * 64 * sizeof(T) +
-         (size_t)ev.L * (kNP * 8 + 16) + 8 * 256;
+  const size_t b = M * 24 + ev.nd * M * sizeof(cplx<T>) + S * 64 * sizeof(T) +
+                   (size_t)ev.L * (kNP * 8 + 16) + 8 * 256;
+  return (b + 255) / 256 * 256;
 }
 
-// Rows evaluated per pass: the block sums of a pass (32 KB a row) stay in the
-// 256 MB last-level cache between the two kernels.
-constexpr long long kPassRows = 4096;
+// Block sums of one pass (32 KB a row in float32, 64 in float64): they stay in
+// the 256 MB last-level cache between the two kernels.
+constexpr size_t kPassBytes = (size_t)128 << 20;
 constexpr long long kMinPassRows = 64;
 
 template <typename T> constexpr size_t band_row_bytes() {
@@ -926,7 +941,7 @@ BandSplit band_split(const gwl_event* e, long long n, int& R) {
   const int wpc = e->tile_wg_per_cu;
   const long long target = (long long)e->ctx->n_cu * (wpc > 0 ? wpc : 24);
   const long long least = (long long)e->ctx->n_cu * (wpc > 0 ? wpc : 8);
-  R = n * NG >= 2 * least ? 2 : 1;
+  R = sizeof(T) == 4 && n * NG >= 2 * least ? 2 : 1;
   const long long items = (n + R - 1) / R;
   BandSplit sp{1, 1};
   while (sp.gg < NG && items * sp.gg < target) sp.gg *= 2;
@@ -939,67 +954,65 @@ void launch_band(const BandArgs& a, int R, hipStream_t st) {
   const unsigned nsplit = (unsigned)(a.split.gg * a.split.gs);
   const long long per = kBandWaves * R;
   const dim3 grid((unsigned)((a.n + per - 1) / per), nsplit);
-  if (R == 2)
-    hipLaunchKernelGGL((k_band<T, ND, 2>), grid, dim3(64 * kBandWaves), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_band<T, ND, 1>), grid, dim3(64 * kBandWaves), 0, st, a);
+  if constexpr (sizeof(T) == 4) {
+    if (R == 2) {
+      hipLaunchKernelGGL((k_band<T, ND, 2>), grid, dim3(64 * kBandWaves), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_band<T, ND, 1>), grid, dim3(64 * kBandWaves), 0, st, a);
 }
 
 }  // namespace
 
-bool band_tables_wanted(const EvDev& ev) {
-  return ev.approx == GWL_TAYLORF2 && (ev.flags & GWL_TIME_MARG) && ev.P == 512 && ev.L <= 512;
-}
+namespace {
 
-size_t band_table_bytes(const EvDev& ev) { return band_bytes<float>(ev); }
-
-int band_table_init(EvDev& ev, char* p) { return init_band<float>(ev, ev.band32, p); }
-
-bool band_eligible(const gwl_event* e) {
-  if (!e->dev.band32.uv) return false;
-  if (e->transform == GWL_TRANSFORM_WAVE) return true;
-  return e->transform == GWL_TRANSFORM_AUTO && e->tile_rows == 0;
+// Whole steps of four bins in every block.
+template <typename T>
+bool band_fits(const EvDev& ev) {
+  return ev.approx == GWL_TAYLORF2 && (ev.flags & GWL_TIME_MARG) && ev.P == 512 && ev.L <= 512 &&
+         ev.N % (4 * BandTypes<T>::NB) == 0;
 }
 
 // Row constants of every row, then the block sums of a pass: at least
-// kMinPassRows rows (times the largest number of step parts few rows take),
-// kPassRows where the workspace allows.
-static size_t band_ws(long long rows, long long pass) {
-  return ((size_t)rows * sizeof(RowW) + 255) / 256 * 256 + (size_t)pass * band_row_bytes<float>();
+// kMinPassRows rows, kPassBytes where the workspace allows.
+template <typename T>
+size_t band_ws(long long rows, long long pass) {
+  return ((size_t)rows * sizeof(RowW) + 255) / 256 * 256 + (size_t)pass * band_row_bytes<T>();
 }
 
-size_t band_ws_min_bytes(const gwl_event*, int64_t rows) {
-  return band_ws(rows, std::min<long long>(std::max<long long>(rows, 8), kMinPassRows));
-}
-
-size_t band_ws_bytes(const gwl_event* e, int64_t rows) {
+template <typename T>
+size_t band_ws_bytes_t(const gwl_event* e, int64_t rows) {
+  if (!band_dev<T>(e->dev).uv) return 0;
   // steps are cut (gs <= 8) only below two rounds of whole groups
   const long long wpc = e->tile_wg_per_cu > 0 ? e->tile_wg_per_cu : 8;
-  const long long few = 2 * wpc * e->ctx->n_cu / (BandTypes<float>::NB / 16) + 1;
+  const long long few = 2 * wpc * e->ctx->n_cu / (BandTypes<T>::NB / 16) + 1;
   const long long most = std::max<long long>(rows, 8 * std::min<long long>(rows, few));
-  return band_ws(rows, std::min<long long>(most, kPassRows));
+  return band_ws<T>(rows, std::min<long long>(most, kPassBytes / band_row_bytes<T>()));
 }
 
-int launch_band_eval(gwl_event* e, const double* params, int64_t n, int ld, double* out,
-                     hipStream_t st) {
+template <typename T>
+int launch_band_eval_t(gwl_event* e, const double* params, int64_t n, int ld, double* out,
+                       hipStream_t st) {
   const EvDev& ev = e->dev;
   char* ws = reinterpret_cast<char*>(e->ws);
   RowW* rows = reinterpret_cast<RowW*>(ws);
   const size_t head = ((size_t)n * sizeof(RowW) + 255) / 256 * 256;
   double* c = reinterpret_cast<double*>(ws + head);
   const long long room =
-      e->ws_bytes > head ? (long long)((e->ws_bytes - head) / band_row_bytes<float>()) : 0;
+      e->ws_bytes > head ? (long long)((e->ws_bytes - head) / band_row_bytes<T>()) : 0;
   if (room < 1) {
     set_error("workspace too small for the time transform");
     return GWL_E_INVALID;
   }
-  const size_t lds = finish_lds<float>();
+  const size_t lds = finish_lds<T>();
   if (lds > e->ctx->lds_per_block) {
     set_error("time transform exceeds the LDS of a workgroup");
     return GWL_E_UNSUPPORTED;
   }
   if (int rc = launch_rowconst(e, params, n, ld, rows, st)) return rc;
-  const long long tile = std::min<long long>(std::min<long long>(room, kPassRows), n);
+  const long long tile = std::min<long long>(
+      std::min<long long>(room, kPassBytes / band_row_bytes<T>()), n);
   for (long long r0 = 0; r0 < n; r0 += tile) {
     const long long m = std::min<long long>(tile, n - r0);
     BandArgs a{};
@@ -1007,23 +1020,58 @@ int launch_band_eval(gwl_event* e, const double* params, int64_t n, int ld, doub
     a.ev = ev;
     a.rows = rows + r0;
     a.n = m;
-    a.split = band_split<float>(e, m, R);
+    a.split = band_split<T>(e, m, R);
     while (a.split.gs > 1 && m * a.split.gs > room) a.split.gs /= 2;
     a.out = c;
     if (int rc = timing_begin(e, st)) return rc;
     switch (ev.nd) {
-      case 1: launch_band<float, 1>(a, R, st); break;
-      case 2: launch_band<float, 2>(a, R, st); break;
-      case 3: launch_band<float, 3>(a, R, st); break;
-      default: launch_band<float, 4>(a, R, st); break;
+      case 1: launch_band<T, 1>(a, R, st); break;
+      case 2: launch_band<T, 2>(a, R, st); break;
+      case 3: launch_band<T, 3>(a, R, st); break;
+      default: launch_band<T, 4>(a, R, st); break;
     }
     GWL_HIP_CHECK(hipGetLastError());
     if (int rc = timing_end(e, st)) return rc;
     FinishArgs f{ev, rows + r0, c, a.split.gs, out + r0};
-    hipLaunchKernelGGL(k_band_finish<float>, dim3((unsigned)m), dim3(kFinThreads), lds, st, f);
+    hipLaunchKernelGGL(k_band_finish<T>, dim3((unsigned)m), dim3(kFinThreads), lds, st, f);
     GWL_HIP_CHECK(hipGetLastError());
   }
   return GWL_OK;
+}
+
+}  // namespace
+
+bool band_tables_wanted(const EvDev& ev) { return band_fits<float>(ev); }
+
+size_t band_table_bytes(const EvDev& ev) {
+  return band_bytes<float>(ev) + (band_fits<double>(ev) ? band_bytes<double>(ev) : 0);
+}
+
+int band_table_init(EvDev& ev, char* p) {
+  if (int rc = init_band<float>(ev, ev.band32, p)) return rc;
+  return band_fits<double>(ev) ? init_band<double>(ev, ev.band64, p + band_bytes<float>(ev))
+                               : GWL_OK;
+}
+
+bool band_eligible(const gwl_event* e, bool fp64) {
+  if (!(fp64 ? e->dev.band64.uv : e->dev.band32.uv)) return false;
+  if (e->transform == GWL_TRANSFORM_WAVE) return true;
+  return e->transform == GWL_TRANSFORM_AUTO && e->tile_rows == 0;
+}
+
+size_t band_ws_min_bytes(const gwl_event*, int64_t rows, bool fp64) {
+  const long long pass = std::min<long long>(std::max<long long>(rows, 8), kMinPassRows);
+  return fp64 ? band_ws<double>(rows, pass) : band_ws<float>(rows, pass);
+}
+
+size_t band_ws_bytes(const gwl_event* e, int64_t rows) {
+  return std::max(band_ws_bytes_t<float>(e, rows), band_ws_bytes_t<double>(e, rows));
+}
+
+int launch_band_eval(gwl_event* e, bool fp64, const double* params, int64_t n, int ld,
+                     double* out, hipStream_t st) {
+  return fp64 ? launch_band_eval_t<double>(e, params, n, ld, out, st)
+              : launch_band_eval_t<float>(e, params, n, ld, out, st);
 }
 
 size_t band_multi_row_bytes() { return band_row_bytes<float>(); }

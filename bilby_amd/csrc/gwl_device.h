@@ -155,7 +155,7 @@ struct EvDev {
   const float2* dwa32;  // [nd][N] dw32 f^-7/6, decimated order
   const double* hps;    // [nd][N + 2] prefix sums of f^-7/3 sigma^2 / S over bins
                         //   0..N in natural order, hps[d][n] = sum of bins < n
-  BandDev band32;
+  BandDev band32, band64;
   InnerDev inner;
   // Nyquist bin (n = N), kept apart from the power-of-two FFT range
   double dwN[GWL_MAX_DET][2];

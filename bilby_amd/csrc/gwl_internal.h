@@ -150,11 +150,11 @@ int init_time_wave_tables(const EvDev& ev, double* tf2b, float2* dwa32);
 bool band_tables_wanted(const EvDev& ev);
 size_t band_table_bytes(const EvDev& ev);
 int band_table_init(EvDev& ev, char* p);  // p: band_table_bytes of device memory
-bool band_eligible(const gwl_event* ev);
-size_t band_ws_bytes(const gwl_event* ev, int64_t rows);      // workspace taken
-size_t band_ws_min_bytes(const gwl_event* ev, int64_t rows);  // workspace it can do with
-int launch_band_eval(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
-                     hipStream_t stream);
+bool band_eligible(const gwl_event* ev, bool fp64);
+size_t band_ws_bytes(const gwl_event* ev, int64_t rows);  // workspace taken (either precision)
+size_t band_ws_min_bytes(const gwl_event* ev, int64_t rows, bool fp64);  // it can do with
+int launch_band_eval(gwl_event* ev, bool fp64, const double* params, int64_t n, int ld,
+                     double* out, hipStream_t stream);
 // TaylorF2 inner products without time marginalisation (gwl_inner.hip):
 // partials [units][n][2] of <d|h> / |C_r|
 int inner_units_of(const EvDev& ev);

@@ -1114,8 +1114,9 @@ template <typename R, int WAVE, int ND>
 static int eval_typed(gwl_event* e, const double* params, int64_t n, int ld, double* out,
                       double* aux, hipStream_t st) {
   const EvDev& ev = e->dev;
-  if constexpr (std::is_same<R, float>::value && WAVE == GWL_TAYLORF2) {
-    if (band_eligible(e)) return launch_band_eval(e, params, n, ld, out, st);
+  if constexpr (WAVE == GWL_TAYLORF2) {
+    constexpr bool fp64 = std::is_same<R, double>::value;
+    if (band_eligible(e, fp64)) return launch_band_eval(e, fp64, params, n, ld, out, st);
   }
   if (ev.flags & GWL_TIME_MARG) {
     // a window longer than one transform: slices of P bins, one pass each,
@@ -1178,9 +1179,10 @@ static int eval_nd(gwl_event* e, const double* params, int64_t n, int ld, double
 }
 
 size_t workspace_bytes_for(const gwl_event* e, int64_t rows, int precision) {
-  // a float32 evaluation on the block-projected transform uses that path's
-  // workspace only, in as many passes as it takes
-  if (precision == GWL_FP32 && band_eligible(e)) return band_ws_min_bytes(e, rows);
+  // the block-projected transform uses its own workspace only, in as many
+  // passes as it takes
+  const bool fp64 = precision == GWL_FP64;
+  if (band_eligible(e, fp64)) return band_ws_min_bytes(e, rows, fp64);
   return workspace_bytes(e, rows);
 }
 

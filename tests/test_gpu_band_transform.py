@@ -16,13 +16,18 @@ CASES = [
     (6.0, 4096.0, ("H1", "L1"), 0.1, 5),             # 12288 bins: three chunks
     (7.0, 1024.0, ("V1",), 0.2, 8),                  # 3584 bins: seven steps, padded to eight
     (8.0, 4096.0, ("H1", "L1", "V1", "K1"), 0.002, 33),  # a window of 14 bins
+    (2.0, 2048.0, ("H1", "L1"), 0.1, 2),               # 2048 bins: two steps
     (8.0, 4096.0, ("H1", "L1", "V1"), 0.1237, 1),    # all 512 bins of the window, one row
 ]
 
 
-@pytest.mark.parametrize("case", CASES)
+# float64 takes whole steps in 256 blocks: multiples of 1024 bins
+RUNS = [(c, "fp32") for c in CASES] + [(c, "fp64") for c in CASES if c[0] * c[1] % 2048 == 0]
+
+
+@pytest.mark.parametrize("case,precision", RUNS)
 @pytest.mark.parametrize("split", [1, 64])
-def test_window_transform_matches_oracle(case, split):
+def test_window_transform_matches_oracle(case, precision, split):
     from bilby_amd.autotune import set_tile, set_transform
     from bilby_amd.configs import make_taylorf2_marginalised
     from bilby_amd.likelihood import GravitationalWaveTransient
@@ -40,7 +45,7 @@ def test_window_transform_matches_oracle(case, split):
     priors = s["priors"].copy()
     lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
                                     time_marginalization=True, phase_marginalization=True,
-                                    priors=priors, precision="fp32")
+                                    priors=priors, precision=precision)
     draws = fixed_marginalised(s["draws"], priors)
     set_transform(lk, 2)
     set_tile(lk, 0, split)   # target wavefronts per CU: unsplit, and cut as far as it goes
@@ -48,5 +53,7 @@ def test_window_transform_matches_oracle(case, split):
     olk, _ = oracle_from_setup(s)
     ref = np.array([olk.log_likelihood_ratio(p) for p in draws_as_dicts(draws, range(rows))])
     # float32 integrand (2^-24 per factor) under a float64 sum: a few 1e-7 of
-    # the inner products, which are of the order of |lnL| + rho^2 / 2 < 2000
-    assert np.max(np.abs(out - ref)) < 1e-3, np.abs(out - ref).max()
+    # the inner products, which are of the order of |lnL| + rho^2 / 2 < 2000;
+    # float64: 1e-14 (block functions at 512 bins) and the sums' rounding
+    tol = 1e-3 if precision == "fp32" else 1e-10
+    assert np.max(np.abs(out - ref)) < tol, np.abs(out - ref).max()
