@@ -35,6 +35,31 @@ static int ilog2(long long x) {
 // thread (one h-axis point) streams them with a running-max logsumexp.
 constexpr int kTabChunk = 2048;
 
+// ln I0 for the distance table, which subtracts h s^2 / 2 from it: where both
+// are 1e6 the difference is of order one and shows each rounding of the
+// larger terms, so from 30 on the value is x - ln(2 pi x) / 2 + ln(sum) in
+// this order (ln_i0, rounded once, is nearer but moves table values by
+// 1e-10).  sum = sum_k a_k y^k, y = 1/(8x), a_k = ((2k-1)!!)^2 / k!
+// (Abramowitz & Stegun 9.7.1): at y <= 1/240 the term a_18 y^18 is below
+// 1e-17 and the terms are still falling, so 19 give float64 round-off.
+struct I0Asymptotic {
+  double a[19];
+  constexpr I0Asymptotic() : a() {
+    a[0] = 1.0;
+    for (int k = 1; k < 19; ++k) a[k] = a[k - 1] * (double)((2 * k - 1) * (2 * k - 1)) / (double)k;
+  }
+};
+constexpr I0Asymptotic kI0Asymptotic{};
+
+__device__ double ln_i0_table(double x) {
+  if (x < 30.0) return ln_i0(x);
+  const double y = 1.0 / (8.0 * x);
+  double s = kI0Asymptotic.a[18];
+#pragma unroll
+  for (int k = 17; k >= 0; --k) s = fma(s, y, kI0Asymptotic.a[k]);
+  return x - 0.5 * log(kTwoPi * x) + log(s);
+}
+
 __global__ __launch_bounds__(256) void k_distance_table(const double* dist, const double* prior,
                                                         int nk, double dref, int phase,
                                                         double delta, const double* daxis, int nd,
@@ -60,7 +85,7 @@ __global__ __launch_bounds__(256) void k_distance_table(const double* dist, cons
     for (int k = threadIdx.x; k < kn; k += 256) {
       const double sc = dref / dist[k0 + k];
       const double dv = x * sc;
-      dterm[k] = phase ? ln_i0(fabs(dv)) : dv;
+      dterm[k] = phase ? ln_i0_table(fabs(dv)) : dv;
       s2[k] = sc * sc;
       const double b = prior[k0 + k] * delta;
       lb[k] = b;

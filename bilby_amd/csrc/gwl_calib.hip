@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_cal_epi(CalArgs a) {
       const SplineY yy = spline_y(ev.sp, hh * hs * hs);
       v = spline_x(ev.sp, yy, dd);
     } else if (ev.flags & GWL_PHASE_MARG) {
-      v = ln_i0(hypot(dr, di)) - hh / 2.0;
+      v = ln_i0_abs(dr, di) - hh / 2.0;
     } else {
       v = dr - hh / 2.0;
     }

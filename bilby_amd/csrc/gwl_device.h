@@ -511,20 +511,24 @@ __device__ inline void compute_sample_const(const EvDev& ev, const double* row, 
 
 // ------------------------------------------------------------ special functions
 // ln I0(x) (bilby/gw/utils.py:1006-1022 computes log(i0e(x)) + |x|).
-// Power series I0(x) = sum_k c_k q^k, q = x^2/4, c_k = 1/(k!)^2, for
-// x < 30, in Horner form over a compile-time table of c_k (all terms
-// positive: no cancellation, relative error ~ K ulp) truncated at K terms
-// chosen per range so that c_K q^K < 1e-17 I0(x): K = 24 for x <= 8,
-// 40 for x <= 16, 60 below 30.  For x >= 30 the large-argument expansion
-// I0(x) = e^x / sqrt(2 pi x) sum_k ((2k-1)!!)^2 / (k! (8x)^k)
-// (Abramowitz & Stegun 9.7.1), summed until float64 round-off (its terms
-// fall below 1e-17 long before they start to grow at k ~ 2x).
+// x <= 8: power series I0(x) = sum_k c_k q^k, q = x^2/4, c_k = 1/(k!)^2, 24
+// terms (c_24 q^24 < 1e-17 I0), all positive: no cancellation.
+// x > 8: g(t) = sqrt(x) e^-x I0(x) is smooth in t = 16/x - 1 on (-1, 1]; its
+// Chebyshev interpolant, computed in 70 digits from the power series and
+// written as a polynomial of 26 terms, is exact to 1.3e-16 (the power
+// coefficients fall from 0.4 to 3e-3 at once, so nothing cancels).
+// Then ln I0 = x + ln(g^2 / x) / 2: one logarithm for both ranges, and two
+// polynomials where the lanes of a wavefront straddle 8.  Series by range
+// (24, 40 and 60 terms, an asymptotic sum from 30 on) before: four
+// polynomials and five logarithms in such a wavefront, and the marginalised
+// epilogue's values do straddle: the 1000 times of a reduced-order row run
+// from the noise to the peak.
 struct I0Series {
-  double c[60];
+  double c[24];
   constexpr I0Series() : c() {
     double f = 1.0;
     c[0] = 1.0;
-    for (int k = 1; k < 60; ++k) {
+    for (int k = 1; k < 24; ++k) {
       f *= (double)k;
       c[k] = 1.0 / (f * f);
     }
@@ -532,45 +536,46 @@ struct I0Series {
 };
 constexpr I0Series kI0Series{};
 
-// The large-argument coefficients a_k = ((2k-1)!!)^2 / k!, k < 19: at
-// x >= 30 (y = 1/(8x) <= 1/240) the term a_18 y^18 is below 1e-17 and the
-// terms are still falling, so 19 terms give float64 round-off.
-struct I0Asymptotic {
-  double a[19];
-  constexpr I0Asymptotic() : a() {
-    a[0] = 1.0;
-    for (int k = 1; k < 19; ++k) a[k] = a[k - 1] * (double)((2 * k - 1) * (2 * k - 1)) / (double)k;
-  }
-};
-constexpr I0Asymptotic kI0Asymptotic{};
-
-// sum_{k < K} c_k q^k in Horner form, unrolled (the coefficients become
-// wave-uniform constants)
-template <int K>
-__host__ __device__ __forceinline__ double i0_series(double q) {
-  double s = kI0Series.c[K - 1];
-#pragma unroll
-  for (int k = K - 2; k >= 0; --k) s = fma(s, q, kI0Series.c[k]);
-  return s;
-}
+constexpr double kI0Large[26] = {
+    0x1.9bd428ad249a5p-2, 0x1.b87969bb93bc0p-9, 0x1.1daa72b5e2bd7p-13,
+    0x1.75e5ee702007ep-17, 0x1.8e513a708989ep-20, 0x1.3f49ad6d6f0a1p-22,
+    0x1.7d0f1670e44e2p-24, 0x1.51cbf2b8d32b7p-25, 0x1.7232c4c122295p-26,
+    0x1.03e3a46a554fap-27, -0x1.cfb20ddb53edep-28, -0x1.ce4513f876844p-27,
+    -0x1.7369bf37c026dp-28, 0x1.087d59e67c7aep-27, 0x1.fe9e1dd494c83p-28,
+    -0x1.0693a8366885ap-28, -0x1.99204d1a8bb30p-28, 0x1.10973e09f287bp-29,
+    0x1.f3ff264907758p-29, -0x1.1a39fc6f3bf71p-30, -0x1.bd05a336c6a58p-30,
+    0x1.e28f74bf3432cp-32, 0x1.f741903e631b4p-32, -0x1.1153c28a5c59fp-33,
+    -0x1.0adb754ca8b1dp-34, 0x1.24d48c789b287p-36};
 
 // Not inlined: inlined into a loop, its coefficients would be hoisted into
-// vector registers of the caller.  The series length follows the range (the
-// K of the comment above); lanes of one wavefront hold neighbouring window
-// bins, so they mostly take the same branch.
+// vector registers of the caller.
 __host__ __device__ inline __attribute__((noinline)) double ln_i0(double x) {
   x = fabs(x);
-  if (x < 30.0) {
+  double arg, base = 0.0, scale = 1.0;
+  if (x <= 8.0) {
     const double q = 0.25 * x * x;
-    if (x <= 8.0) return log(i0_series<24>(q));
-    if (x <= 16.0) return log(i0_series<40>(q));
-    return log(i0_series<60>(q));
-  }
-  const double y = 1.0 / (8.0 * x);
-  double s = kI0Asymptotic.a[18];
+    double s = kI0Series.c[23];
 #pragma unroll
-  for (int k = 17; k >= 0; --k) s = fma(s, y, kI0Asymptotic.a[k]);
-  return x - 0.5 * log(kTwoPi * x) + log(s);
+    for (int k = 22; k >= 0; --k) s = fma(s, q, kI0Series.c[k]);
+    arg = s;
+  } else {
+    const double rx = 1.0 / x;
+    const double t = fma(16.0, rx, -1.0);
+    double s = kI0Large[25];
+#pragma unroll
+    for (int k = 24; k >= 0; --k) s = fma(s, t, kI0Large[k]);
+    arg = s * s * rx;
+    base = x;
+    scale = 0.5;
+  }
+  return fma(scale, log(arg), base);
+}
+
+// ln I0(|x + i y|): the plain root where the squares neither overflow nor
+// lose digits (below, ln I0 is zero to rounding), else the scaling hypot.
+__host__ __device__ __forceinline__ double ln_i0_abs(double x, double y) {
+  const double r2 = fma(x, x, y * y);
+  return ln_i0(r2 < 1e300 ? sqrt(r2) : hypot(x, y));
 }
 
 // Largest l in [3, ncoef - 1] with t[l] <= x (FITPACK fpbisp interval rule).
@@ -877,7 +882,7 @@ __device__ inline double epi_value(unsigned flags, const SplineDev& sp, const Sp
     const double d = (flags & GWL_PHASE_MARG) ? cabs2d(xr, xi) * hs : xr * hs;
     return spline_x(sp, yy, d);
   }
-  if (flags & GWL_PHASE_MARG) return ln_i0(hypot(xr, xi)) - hh / 2.0;
+  if (flags & GWL_PHASE_MARG) return ln_i0_abs(xr, xi) - hh / 2.0;
   return xr - hh / 2.0;
 }
 
@@ -916,14 +921,15 @@ __device__ __forceinline__ double time_lse_scale(const EvDev& ev, double delta_t
   return ev.tpd ? delta_tc : delta_tc / (ev.tmax - ev.tmin);
 }
 
-// Running logsumexp state (max m, sum s of exp(v - m)).
+// Running logsumexp state (max m, sum s of exp(v - m)); NaN and -inf add
+// nothing.  One exponential for both outcomes: lanes that meet a new maximum
+// and lanes that do not share a wavefront (m = -inf: exp(-inf) = 0).
 __device__ __forceinline__ void lse_push(double& m, double& s, double v) {
-  if (v > m) {
-    s = (m > -INFINITY ? s * exp(m - v) : 0.0) + 1.0;
-    m = v;
-  } else if (v > -INFINITY) {
-    s += exp(v - m);
-  }
+  if (!(v > -INFINITY)) return;
+  const bool up = v > m;
+  const double e = exp(up ? m - v : v - m);
+  s = fma(up ? s : 1.0, e, up ? 1.0 : s);
+  m = up ? v : m;
 }
 
 // Merge the logsumexp states of the 64 lanes of a wavefront: the maximum

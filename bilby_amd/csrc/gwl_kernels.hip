@@ -425,7 +425,7 @@ __device__ __forceinline__ void epi_plain_row(const EpiArgs& a, long long r, lon
     const SplineY yy = spline_y(ev.sp, hh * hs * hs);
     ll = spline_x(ev.sp, yy, d);
   } else if (ev.flags & GWL_PHASE_MARG) {
-    ll = ln_i0(hypot(dhr, dhi)) - hh / 2.0;
+    ll = ln_i0_abs(dhr, dhi) - hh / 2.0;
   } else {
     ll = dhr - hh / 2.0;
   }
@@ -545,7 +545,7 @@ __device__ __forceinline__ double epi_bin_value(const EvDev& ev, const SplineY& 
     const double d = (ev.flags & GWL_PHASE_MARG) ? cabs2d(xr, xi) * hs : xr * hs;
     v = spline_x(ev.sp, yy, d);
   } else if (ev.flags & GWL_PHASE_MARG) {
-    v = ln_i0(hypot(xr, xi)) - hh / 2.0;
+    v = ln_i0_abs(xr, xi) - hh / 2.0;
   } else {
     v = xr - hh / 2.0;
   }

@@ -810,7 +810,7 @@ __global__ __launch_bounds__(128) void k_relbin_epi(RelbinArgs a) {
     const SplineY yy = spline_y(ev.sp, h2 * hs * hs);
     ll = spline_x(ev.sp, yy, dd);
   } else if (ev.flags & GWL_PHASE_MARG) {
-    ll = ln_i0(hypot(dh_re, dh_im)) - h2 / 2.0;
+    ll = ln_i0_abs(dh_re, dh_im) - h2 / 2.0;
   } else {
     ll = dh_re - h2 / 2.0;
   }

