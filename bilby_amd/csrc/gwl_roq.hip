@@ -628,8 +628,8 @@ __device__ __forceinline__ bool roq_dh_at(const RoqDev& rd, const T* zr, const R
 }
 
 // Bound by the float64 instructions of one (row, time): interpolation of each
-// detector, one ln I0 or table look-up, one exponential.  4096 rows of 1000
-// times on three detectors with phase marginalisation: 700 us (1118 with a
+// detector, one ln I0 or table look-up, one exponential.  65536 rows on two
+// detectors with time and phase marginalisation: 700 us (1118 with a
 // sample-difference form of the interpolation, ln I0 by four ranges and an
 // exponential for each outcome of the running maximum).
 template <typename T>

@@ -5,11 +5,13 @@
 #include "gwl_window.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace gwl {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 size_t al256(size_t x) { return (x + 255) / 256 * 256; }
 long long up(long long x, long long a) { return (x + a - 1) / a * a; }
@@ -127,74 +129,102 @@ __global__ __launch_bounds__(256) void k_win_clear(void* a, int fp64, long long 
 // Split-K partials: C_z[M][N] = A[:, k in chunk z] . Bt[:, k in chunk z]^T
 // (float32), chunk z = blockIdx.z of kWinKc columns; M % 128 == 0,
 // N % 128 == 0, K % 32 == 0, row strides K.  Inside a chunk the MFMA
-// accumulators restart every kFlush k-tiles (32 columns, 16 MFMA steps)
+// accumulators restart every TILES k-tiles (32 columns, 16 MFMA steps each)
 // after adding into a float32 chunk total; the epilogue adds the chunk
 // totals in float64.  The chunks also multiply the workgroups of a short
-// row tile.
+// row tile.  A sum of m totals of n products each rounds like n + m: from
+// chunks of 2048 columns on two tiles round no worse than one (64 + m / 2
+// against 32 + m) and need half the additions.
 // A workgroup of 4 waves computes a 128 x 128 tile, each wave 2 x 2 MFMA
 // 32 x 32 blocks (output layout: lane l, accumulator v -> row
 // 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32).
-constexpr int kBM = 128, kBN = 128, kBK = 32, kFlush = 1;
+//
+// Bound by the float32 MFMA rate, which nothing overlaps on the same SIMD, so
+// everything else is kept off it: the next k-tile is loaded into registers
+// while this one is multiplied and goes to the other half of the LDS buffer
+// (one barrier a tile); lane half h takes columns 8 g + 4 h ... + 3 of each
+// eight, in A and B alike, so that one 16-byte LDS read feeds four MFMAs; the
+// first MFMA of a sum starts from a zero operand instead of cleared
+// registers.  Rows of 36 floats: 16-byte aligned, and 16 rows fall into
+// different 16-byte slots.  999 rows, 1000 response curves, 8 s at 2048 Hz
+// from 20 Hz on two detectors (161 GFLOP, padded 169): 1321 us for both
+// products, of which 1000 are MFMA issue at the 2.1 GHz that the clock holds
+// under them (1522 with one LDS buffer, loads at their use and clears).
+constexpr int kBM = 128, kBN = 128, kBK = 32, kLd = kBK + 4;
 
-__global__ __launch_bounds__(256) void k_win_gemm_f32(const float* __restrict__ A,
-                                                      const float* __restrict__ Bt,
-                                                      float* __restrict__ C, int M, int N, int K,
-                                                      int kc) {
-  __shared__ float As[kBM][kBK + 1];
-  __shared__ float Bs[kBN][kBK + 1];
+template <int TILES>
+__global__ __launch_bounds__(256, 2) void k_win_gemm_f32(const float* __restrict__ A,
+                                                         const float* __restrict__ Bt,
+                                                         float* __restrict__ C, int M, int N,
+                                                         int K, int kc) {
+  __shared__ float As[2][kBM][kLd];
+  __shared__ float Bs[2][kBN][kLd];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
   const int wr = (w >> 1) * 64, wc = (w & 1) * 64;
   const int kb = blockIdx.z * kc, ke = min(K, kb + kc);
-  f32x16 acc[2][2];
-  float tot[2][2][16];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc[i][j][v] = 0.f;
-        tot[i][j][v] = 0.f;
-      }
-  int tiles = 0;
-  for (int k0 = kb; k0 < ke; k0 += kBK) {
+  const int lr = tid >> 3, lc = (tid & 7) * 4;  // this thread's rows lr + 32 q, columns lc ...
+  const unsigned lo = (unsigned)lr * (unsigned)K + (unsigned)lc;
+  f32x4 va[4], vb[4];
+  auto load = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int idx = tid + 256 * q;
-      const int row = idx >> 3, c4 = (idx & 7) * 4;
-      const float4 va = *reinterpret_cast<const float4*>(A + (size_t)(m0 + row) * K + k0 + c4);
-      const float4 vb = *reinterpret_cast<const float4*>(Bt + (size_t)(n0 + row) * K + k0 + c4);
-      As[row][c4 + 0] = va.x; As[row][c4 + 1] = va.y; As[row][c4 + 2] = va.z; As[row][c4 + 3] = va.w;
-      Bs[row][c4 + 0] = vb.x; Bs[row][c4 + 1] = vb.y; Bs[row][c4 + 2] = vb.z; Bs[row][c4 + 3] = vb.w;
+      va[q] = *reinterpret_cast<const f32x4*>(A + (size_t)(m0 + 32 * q) * K + k0 + lo);
+      vb[q] = *reinterpret_cast<const f32x4*>(Bt + (size_t)(n0 + 32 * q) * K + k0 + lo);
     }
+  };
+  auto store = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      *reinterpret_cast<f32x4*>(&As[p][lr + 32 * q][lc]) = va[q];
+      *reinterpret_cast<f32x4*>(&Bs[p][lr + 32 * q][lc]) = vb[q];
+    }
+  };
+  f32x16 tot[2][2] = {};
+  load(kb);
+  store(0);
+  f32x16 acc[2][2];
+  // multiply the tile in half P of the buffer while the one at column kn is
+  // loaded (past the last one: the last one again)
+  auto tile = [&](auto P, int kn) __attribute__((always_inline)) {
+    constexpr int p = decltype(P)::value;
     __syncthreads();
+    load(min(kn, ke - kBK));
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int kk = 0; kk < kBK; kk += 2) {
-      float a[2], b[2];
+    for (int g = 0; g < kBK / 8; ++g) {
+      f32x4 a[2], b[2];
+      const int c = 8 * g + 4 * (lane >> 5);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = As[wr + i * 32 + (lane & 31)][kk + (lane >> 5)];
+      for (int i = 0; i < 2; ++i) {
+        a[i] = *reinterpret_cast<const f32x4*>(&As[p][wr + i * 32 + (lane & 31)][c]);
+        b[i] = *reinterpret_cast<const f32x4*>(&Bs[p][wc + i * 32 + (lane & 31)][c]);
+      }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = Bs[wc + j * 32 + (lane & 31)][kk + (lane >> 5)];
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                a[i][e], b[j][e], (TILES == 1 || p == 0) && g + e == 0 ? f32x16{} : acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
-    if (++tiles == kFlush || k0 + kBK >= ke) {
-      tiles = 0;
+    store(p ^ 1);
+  };
+  auto flush = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            tot[i][j][v] += acc[i][j][v];
-            acc[i][j][v] = 0.f;
-          }
+      for (int j = 0; j < 2; ++j) tot[i][j] += acc[i][j];
+  };
+  for (int k0 = kb; k0 < ke; k0 += 2 * kBK) {
+    tile(std::integral_constant<int, 0>{}, k0 + kBK);
+    if (TILES == 1) flush();
+    if (k0 + kBK < ke) {
+      tile(std::integral_constant<int, 1>{}, k0 + 2 * kBK);
+      if (TILES == 1) flush();
     }
+    if (TILES == 2) flush();
   }
   float* Cz = C + (size_t)blockIdx.z * M * N;
 #pragma unroll
@@ -334,7 +364,8 @@ int win_gemm_f32(const float* A, const float* Bt, float* C, int Mp, int Np, int 
     return GWL_E_INVALID;
   }
   const int nz = (Kp + kc - 1) / kc;
-  hipLaunchKernelGGL(k_win_gemm_f32, dim3((unsigned)(Np / kBN), (unsigned)(Mp / kBM), (unsigned)nz),
+  hipLaunchKernelGGL(kc >= 2048 ? k_win_gemm_f32<2> : k_win_gemm_f32<1>,
+                     dim3((unsigned)(Np / kBN), (unsigned)(Mp / kBM), (unsigned)nz),
                      dim3(256), 0, st, A, Bt, C, Mp, Np, Kp, kc);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
@@ -437,7 +468,7 @@ int win_finish(gwl_event* ev, const WinBasis& wb, const void* a, bool fp64, void
                           wb.Np, wb.Kp, st))
       return rc;
   } else {
-    hipLaunchKernelGGL(k_win_gemm_f32,
+    hipLaunchKernelGGL(k_win_gemm_f32<1>,
                        dim3((unsigned)(wb.Np / kBN), (unsigned)(Mp / kBM), (unsigned)nchunk),
                        dim3(256), 0, st, static_cast<const float*>(a), wb.bt32,
                        static_cast<float*>(c), (int)Mp, wb.Np, wb.Kp, kWinKc);
