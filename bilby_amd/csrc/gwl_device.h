@@ -423,55 +423,72 @@ __device__ inline void tf2_part(const EvDev& ev, const double* row, Tf2Part& t) 
   t.ci = cos(row[GWL_P_THETA_JN]);
 }
 
-// Per-row prologue: everything that depends on the parameter row only.
-// pre: the TaylorF2 part computed elsewhere (another lane), or null.
-__device__ inline void compute_sample_const(const EvDev& ev, const double* row, SampleConst& sc,
-                                            const Tf2Part* pre = nullptr) {
-  double ra = row[GWL_P_RA], dec = row[GWL_P_DEC], psi = row[GWL_P_PSI];
-  double tc = row[GWL_P_GEOCENT_TIME], jit = row[GWL_P_TIME_JITTER];
-  double dl = row[GWL_P_LUMINOSITY_DISTANCE];
-  sc.row = 0;
-  bool timem = (ev.flags & GWL_TIME_MARG) != 0;
-  bool jitter = timem && (ev.flags & GWL_JITTER_TIME);
-  // base.py:427-428: geocent_time += time_jitter before the detector loop
-  double gt = jitter ? (tc + jit) : tc;
-  sc.jitter = jitter ? jit : 0.0;
-  sc.hscale = (ev.flags & GWL_DISTANCE_MARG) ? dl / ev.dref : 1.0;
-  int lo = ev.mlo[0], hi = ev.mhi[0];
+// First and last bin of any detector's mask.
+__device__ inline void mask_range(const EvDev& ev, int& lo, int& hi) {
+  lo = ev.mlo[0];
+  hi = ev.mhi[0];
   for (int d = 1; d < ev.nd; ++d) {
     lo = min(lo, ev.mlo[d]);
     hi = max(hi, ev.mhi[d]);
   }
-  double fp[GWL_MAX_DET], fc[GWL_MAX_DET];
+}
+
+// The sky part of a row: antenna patterns, detector time shifts, and the
+// marginalisation's distance scale and time jitter.
+__device__ inline void sky_part(const EvDev& ev, const double* row, double* fp, double* fc,
+                                double* dt, double& hscale, double& jitter) {
+  double ra = row[GWL_P_RA], dec = row[GWL_P_DEC], psi = row[GWL_P_PSI];
+  double tc = row[GWL_P_GEOCENT_TIME], jit = row[GWL_P_TIME_JITTER];
+  double dl = row[GWL_P_LUMINOSITY_DISTANCE];
+  bool timem = (ev.flags & GWL_TIME_MARG) != 0;
+  bool jittered = timem && (ev.flags & GWL_JITTER_TIME);
+  // base.py:427-428: geocent_time += time_jitter before the detector loop
+  double gt = jittered ? (tc + jit) : tc;
+  jitter = jittered ? jit : 0.0;
+  hscale = (ev.flags & GWL_DISTANCE_MARG) ? dl / ev.dref : 1.0;
   const SkyBasis sky = sky_basis(ra, dec, gt, psi);  // once per row, not per detector
   for (int d = 0; d < ev.nd; ++d) {
     double delay;
     detector_projection(ev.tensor[d], ev.vertex[d], sky, fp[d], fc[d], delay);
     double dtg = gt - ev.start;  // interferometer.py:355-358: subtract GPS times first
-    sc.dt[d] = dtg + delay;
+    dt[d] = dtg + delay;
   }
+}
+
+// The bins of a TaylorF2 row.  lalsimulation ends TaylorF2 at the fEnd bilby
+// passes (maximum_frequency); at the ISCO as well only when the event asks
+// for it.  An invalid row has none.
+__device__ inline void tf2_support(const EvDev& ev, double fisco, int valid, int lo, int hi,
+                                   int& kb, int& ke) {
+  const double fmax = (ev.flags & GWL_TF2_END_ISCO) ? fmin(fisco, ev.wf_fmax) : ev.wf_fmax;
+  kb = ev.wf_fmin > 0.0 ? first_bin_ge(ev.wf_fmin, ev.df, lo, hi) : lo;
+  ke = last_bin_le(fmax, ev.df, lo, hi);
+  kb = valid ? max(kb, lo) : 1;
+  ke = valid ? min(ke, hi) : 0;
+}
+
+// Per-row prologue: everything that depends on the parameter row only.
+__device__ inline void compute_sample_const(const EvDev& ev, const double* row, SampleConst& sc) {
+  sc.row = 0;
+  int lo, hi;
+  mask_range(ev, lo, hi);
+  double fp[GWL_MAX_DET], fc[GWL_MAX_DET];
+  sky_part(ev, row, fp, fc, sc.dt, sc.hscale, sc.jitter);
   sc.valid = 1;
   if (ev.approx == GWL_TAYLORF2) {
-    Tf2Part own;
-    if (!pre) tf2_part(ev, row, own);
-    const Tf2Part& t = pre ? *pre : own;
+    Tf2Part t;
+    tf2_part(ev, row, t);
 #pragma unroll
     for (int k = 0; k < 10; ++k) sc.c[k] = t.c[k];
     sc.valid = t.valid;
-    const double amp0 = t.amp0, fisco = t.fisco, ci = t.ci;
+    const double amp0 = t.amp0, ci = t.ci;
     double ap = amp0 * (1.0 + ci * ci) / 2.0, ax = amp0 * ci;
     for (int d = 0; d < ev.nd; ++d) {
       sc.cre[d] = fp[d] * ap;
       sc.cim[d] = -fc[d] * ax;
       sc.cabs2[d] = sc.cre[d] * sc.cre[d] + sc.cim[d] * sc.cim[d];
     }
-    // lalsimulation ends TaylorF2 at the fEnd bilby passes (maximum_frequency);
-    // at the ISCO as well only when the event asks for it
-    const double fmax = (ev.flags & GWL_TF2_END_ISCO) ? fmin(fisco, ev.wf_fmax) : ev.wf_fmax;
-    int kb = ev.wf_fmin > 0.0 ? first_bin_ge(ev.wf_fmin, ev.df, lo, hi) : lo;
-    int ke = last_bin_le(fmax, ev.df, lo, hi);
-    sc.kb = max(kb, lo);
-    sc.ke = min(ke, hi);
+    tf2_support(ev, t.fisco, t.valid, lo, hi, sc.kb, sc.ke);
   } else if (ev.approx == GWL_HOST_POLARIZATIONS) {
     // the caller's polarizations: F+ and Fx (over sigma) per detector
     for (int k = 0; k < 10; ++k) sc.c[k] = 0.0;

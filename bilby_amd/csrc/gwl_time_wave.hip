@@ -52,85 +52,124 @@ struct RowArgs {
   int* zero = nullptr;         // cleared by the first thread
 };
 
-__device__ inline void rowconst_one(const EvDev& ev, const double* row, RowW* out,
-                                    const Tf2Part* pre = nullptr, double2* c64 = nullptr) {
-  SampleConst sc;
-  compute_sample_const(ev, row, sc, pre);
-  if (c64)
+// Row constants of 64 rows by two wavefronts: the first takes the TaylorF2
+// part (phase coefficients, amplitude), then the support and <h|h>; the
+// second the sky part (GMST, antenna patterns, delays), then the reference
+// detector and the relative amplitudes.  Bound by the latency of these
+// float64 chains, a few wavefronts a CU at any batch: the two halves run on
+// two SIMDs at the same time and meet once, in LDS.  As odd and even lanes
+// of one wavefront, which runs them one after the other, with the rest after
+// both: 11.0 us for 33 rows on two detectors and 20 for 1000 on three; now 6.8
+// and 14.
+constexpr int kRowconstRows = 64;
+
+struct RowShare {
+  double fp[GWL_MAX_DET][kRowconstRows], fc[GWL_MAX_DET][kRowconstRows];
+  double amp0[kRowconstRows], ci[kRowconstRows], c4[kRowconstRows];
+};
+
+__device__ inline void rowconst_pair(const EvDev& ev, const double* row, bool live, RowW* w,
+                                     double2* c64, RowShare& sh) {
+  const int l = threadIdx.x & 63;
+  const bool first = threadIdx.x < 64;
+  double fisco = 0.0;
+  int valid = 0;
+  if (live && first) {
+    Tf2Part t;
+    tf2_part(ev, row, t);
 #pragma unroll
-    for (int d = 0; d < GWL_MAX_DET; ++d)
-      c64[d] = d < ev.nd ? make_double2(sc.cre[d], sc.cim[d]) : make_double2(0.0, 0.0);
-  RowW w;
+    for (int k = 0; k < 9; ++k) w->c[k] = t.c[k];
+    sh.amp0[l] = t.amp0;
+    sh.ci[l] = t.ci;
+    sh.c4[l] = t.c[4];
+    fisco = t.fisco;
+    valid = t.valid;
+  } else if (live) {
+    double fp[GWL_MAX_DET], fc[GWL_MAX_DET], dt[GWL_MAX_DET], hscale, jitter;
+    sky_part(ev, row, fp, fc, dt, hscale, jitter);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) w.c[k] = sc.c[k];
-  double hh = 0.0;
+    for (int d = 0; d < GWL_MAX_DET; ++d) {
+      const bool on = d < ev.nd;
+      sh.fp[d][l] = on ? fp[d] : 0.0;
+      sh.fc[d][l] = on ? fc[d] : 0.0;
+      w->dt[d] = on ? dt[d] : 0.0;
+    }
+    w->hscale = hscale;
+    w->jitter = jitter;
+  }
+  __syncthreads();
+  if (!live) return;
+  const double amp0 = sh.amp0[l], ci = sh.ci[l];
+  const double ap = amp0 * (1.0 + ci * ci) / 2.0, ax = amp0 * ci;
+  double cre[GWL_MAX_DET], cim[GWL_MAX_DET], cabs2[GWL_MAX_DET];
 #pragma unroll
   for (int d = 0; d < GWL_MAX_DET; ++d) {
     const bool on = d < ev.nd;
-    w.dt[d] = on ? sc.dt[d] : 0.0;
-    w.cre[d] = on ? (float)sc.cre[d] : 0.f;
-    w.cim[d] = on ? (float)sc.cim[d] : 0.f;
-    w.cabs2[d] = on ? sc.cabs2[d] : 0.0;
-    if (on && sc.kb <= sc.ke) {
-      const double* ps = ev.hps + (size_t)d * (ev.N + 2);
-      hh += sc.cabs2[d] * (ps[sc.ke + 1] - ps[sc.kb]);
-    }
+    cre[d] = on ? sh.fp[d][l] * ap : 0.0;
+    cim[d] = on ? -sh.fc[d][l] * ax : 0.0;
+    cabs2[d] = on ? cre[d] * cre[d] + cim[d] * cim[d] : 0.0;
   }
-  w.hh = hh;
-  w.hscale = sc.hscale;
-  w.jitter = sc.jitter;
-  w.kb = sc.kb;
-  w.ke = sc.ke;
-  w.valid = sc.valid;
-  {
-    int lo = ev.mlo[0], hi = ev.mhi[0];
-    for (int d = 1; d < ev.nd; ++d) {
-      lo = min(lo, ev.mlo[d]);
-      hi = max(hi, ev.mhi[d]);
+  if (first) {
+    int lo, hi, kb, ke;
+    mask_range(ev, lo, hi);
+    tf2_support(ev, fisco, valid, lo, hi, kb, ke);
+    double hh = 0.0;
+#pragma unroll
+    for (int d = 0; d < GWL_MAX_DET; ++d) {
+      w->cabs2[d] = cabs2[d];
+      if (d < ev.nd && kb <= ke) {
+        const double* ps = ev.hps + (size_t)d * (ev.N + 2);
+        hh += cabs2[d] * (ps[ke + 1] - ps[kb]);
+      }
     }
-    w.nomask = (sc.kb <= lo && sc.ke >= hi) ? 1 : 0;
-    w.pad = 0;
+    w->hh = hh;
+    w->kb = kb;
+    w->ke = ke;
+    w->valid = valid;
+    w->nomask = (kb <= lo && ke >= hi) ? 1 : 0;
+    w->pad = 0;
+    return;
   }
   // reference detector: the largest |C_d|, so that |rho_k| <= 1
   int ref = 0;
-  for (int d = 1; d < ev.nd && d < GWL_MAX_DET; ++d)
-    if (sc.cabs2[d] > sc.cabs2[ref]) ref = d;
-  const double cr = sc.cre[ref], ci = sc.cim[ref];
-  const double a2 = cr * cr + ci * ci;
-  w.ref = ref;
-  w.amp = sqrt(a2);
-  w.c4r = sc.c[4] - (a2 > 0.0 ? atan2(ci, cr) / kTwoPi : 0.0);
+  double cr = cre[0], ci_ = cim[0], best = cabs2[0];
+#pragma unroll
+  for (int d = 0; d < GWL_MAX_DET; ++d) {
+    w->cre[d] = (float)cre[d];
+    w->cim[d] = (float)cim[d];
+    if (c64) c64[d] = make_double2(cre[d], cim[d]);
+    if (d > 0 && d < ev.nd && cabs2[d] > best) {
+      ref = d;
+      cr = cre[d];
+      ci_ = cim[d];
+      best = cabs2[d];
+    }
+  }
+  const double a2 = cr * cr + ci_ * ci_;
+  w->ref = ref;
+  w->amp = sqrt(a2);
+  w->c4r = sh.c4[l] - (a2 > 0.0 ? atan2(ci_, cr) / kTwoPi : 0.0);
 #pragma unroll
   for (int k = 0; k < GWL_MAX_DET - 1; ++k) {
     const int d = k < ref ? k : k + 1;
+    const double xr = k < ref ? cre[k] : cre[k + 1], xi = k < ref ? cim[k] : cim[k + 1];
     double re = 0.0, im = 0.0;
     if (d < ev.nd && a2 > 0.0) {  // C_d conj(C_ref) / |C_ref|^2
-      re = (sc.cre[d] * cr + sc.cim[d] * ci) / a2;
-      im = (sc.cim[d] * cr - sc.cre[d] * ci) / a2;
+      re = (xr * cr + xi * ci_) / a2;
+      im = (xi * cr - xr * ci_) / a2;
     }
-    w.rre[k] = re;
-    w.rim[k] = im;
+    w->rre[k] = re;
+    w->rim[k] = im;
   }
-  *out = w;
 }
 
-// Two lanes per row: the odd lane computes the TaylorF2 part of the row's
-// constants while the even lane computes the sky part (GMST, antenna
-// patterns, delays), then the even lane assembles them; the two float64
-// chains run side by side instead of one after the other.
-constexpr int kRowconstRows = 128;  // rows per 256-thread block
-
-__global__ __launch_bounds__(256) void k_rowconst(RowArgs a) {
-  __shared__ Tf2Part t[kRowconstRows];
-  const int k = threadIdx.x >> 1;
-  const long long r = (long long)blockIdx.x * kRowconstRows + k;
+__global__ __launch_bounds__(2 * kRowconstRows) void k_rowconst(RowArgs a) {
+  __shared__ RowShare sh;
+  const long long r = (long long)blockIdx.x * kRowconstRows + (threadIdx.x & 63);
   const bool live = r < (a.count ? min(a.n, (long long)*a.count) : a.n);
   if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0;
-  if (live && (threadIdx.x & 1)) tf2_part(a.ev, a.params + r * a.ld, t[k]);
-  __syncthreads();
-  if (live && !(threadIdx.x & 1))
-    rowconst_one(a.ev, a.params + r * a.ld, a.rows + r, a.ev.approx == GWL_TAYLORF2 ? &t[k] : nullptr,
-                 a.c64 ? a.c64 + r * GWL_MAX_DET : nullptr);
+  rowconst_pair(a.ev, a.params + r * a.ld, live, a.rows + r,
+                a.c64 ? a.c64 + r * GWL_MAX_DET : nullptr, sh);
 }
 
 // The event fields the row loop reads.
@@ -583,11 +622,11 @@ struct RowMultiArgs {
   int ld;
 };
 
-__global__ __launch_bounds__(256) void k_rowconst_multi(RowMultiArgs a) {
+__global__ __launch_bounds__(2 * kRowconstRows) void k_rowconst_multi(RowMultiArgs a) {
+  __shared__ RowShare sh;
   const int e = blockIdx.y;
-  const long long r = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (r >= a.rows[e]) return;
-  rowconst_one(a.evs[e], a.params[e] + r * a.ld, a.roww[e] + r);
+  const long long r = (long long)blockIdx.x * kRowconstRows + (threadIdx.x & 63);
+  rowconst_pair(a.evs[e], a.params[e] + r * a.ld, r < a.rows[e], a.roww[e] + r, nullptr, sh);
 }
 
 // f^1/3, f^-1/3, ln f and dw32 f^-7/6 at every decimated element.
@@ -631,7 +670,7 @@ int launch_rowconst(const gwl_event* e, const double* params, int64_t n, int ld,
                     hipStream_t st, const int* count, int* zero) {
   RowArgs ra{e->dev, params, ld, n, rows, nullptr, count, zero};
   hipLaunchKernelGGL(k_rowconst, dim3((unsigned)((n + kRowconstRows - 1) / kRowconstRows)),
-                     dim3(256), 0, st, ra);
+                     dim3(2 * kRowconstRows), 0, st, ra);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }
@@ -671,7 +710,7 @@ int launch_cal_time(gwl_event* e, const double* params, int64_t n, int ld, int n
   double* lnl = per_curve ? per_curve : reinterpret_cast<double*>(w + cal_time_lnl_offset(n));
   RowArgs ra{ev, params, ld, n, rows, fp64 ? c64 : nullptr};
   hipLaunchKernelGGL(k_rowconst, dim3((unsigned)((n + kRowconstRows - 1) / kRowconstRows)),
-                     dim3(256), 0, st, ra);
+                     dim3(2 * kRowconstRows), 0, st, ra);
   GWL_HIP_CHECK(hipGetLastError());
   CalTimeArgs ca{};
   ca.ev = ev;
@@ -728,8 +767,9 @@ int multi_launch_rowconst(gwl_multi* m, hipStream_t st) {
   a.ld = GWL_NPARAM;
   long long maxr = 1;
   for (int64_t r : m->max_rows) maxr = std::max<long long>(maxr, r);
-  hipLaunchKernelGGL(k_rowconst_multi, dim3((unsigned)((maxr + 255) / 256), (unsigned)m->n_events),
-                     dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_rowconst_multi, dim3((unsigned)((maxr + kRowconstRows - 1) / kRowconstRows),
+                                              (unsigned)m->n_events),
+                     dim3(2 * kRowconstRows), 0, st, a);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }
