@@ -104,8 +104,8 @@ def roofline_block(kname, wave, k_ms, achieved_gbps, bpe, traffic, key):
     wave-instructions per launch (rocprofv3 SQ_INSTS_VALU, a property of the
     kernel and the batch, in profiles/) over its launch time measured here
     with HIP events; the HBM figures are kept under "hbm"."""
-    desc = (" (wave per row: waveform + projection + register radix-8 transform + window + "
-            "fused epilogue)" if wave else " (tiled: waveform + projection + LDS FFT)")
+    desc = (" (waveform + projection + block projections on MFMA; k_band_finish follows)"
+            if wave else " (tiled: waveform + projection + LDS FFT)")
     hbm = {"achieved": achieved_gbps, "peak": 8000.0, "unit": "GB/s",
            "frac": achieved_gbps / 8000.0, "bytes_per_eval": bpe,
            "note": "algorithmic bytes / kernel time; L2/MALL-resident data re-read per row"}
@@ -274,8 +274,8 @@ def bench_uneven(steps):
     abytes = sum(ev["n_rows"] * (sum(int(np.sum(np.asarray(i.frequency_mask)))
                                      for i in lk.interferometers) * 12 + 72)
                  for ev, lk in zip(events, lks))
-    valu = profile_figure("bench-valu-insts", "k_time_w_multi_uneven_64_events")
-    roof = {"kernel": "k_time_w_multi (persistent, all 64 events in one launch)",
+    valu = profile_figure("bench-valu-insts", "k_band_multi_uneven_64_events")
+    roof = {"kernel": "k_band_multi + k_band_finish_multi (all 64 events in one launch each)",
             "algorithmic_bytes_per_launch": abytes,
             "hbm": {"achieved": abytes / dt / 1e9, "peak": 8000.0, "unit": "GB/s",
                     "frac": abytes / dt / 1e9 / 8000.0,
@@ -285,7 +285,7 @@ def bench_uneven(steps):
                     achieved=valu / dt / 1e9, peak=VALU_PEAK_GIPS,
                     unit="G VALU wave-instructions/s", frac=valu / dt / 1e9 / VALU_PEAK_GIPS,
                     valu_source="rocprofv3 SQ_INSTS_VALU per dispatch, profiles/ "
-                                "(bench-valu-insts k_time_w_multi_uneven_64_events); "
+                                "(bench-valu-insts k_band_multi_uneven_64_events); "
                                 "launch time of the graph replay in this run")
     return dict(events=len(events), rows=int(total_rows), ms_per_launch=dt * 1e3,
                 evals_per_s=total_rows / dt, bins_min=int(min(n_bins)), bins_max=int(max(n_bins)),
@@ -971,7 +971,7 @@ def main():
                          "0,0 = the default kernel choice")
     ap.add_argument("--transform", type=int, default=0,
                     help="time transform of the headline event (include/gwl.h gwl_transform): "
-                         "0 automatic, 1 tiled, 2 wave per row")
+                         "0 automatic, 1 tiled, 2 block-projected")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py measures one GPU only; --gpus %d is not supported (parameter rows "
@@ -1055,8 +1055,8 @@ def main():
     achieved = args.batch * bpe / (k_ms * 1e-3) / 1e9
     # the transform that ran: the tile choice (include/gwl.h)
     wave = args.transform == 2 or (args.transform == 0 and tile[0] == 0)
-    kname = "k_time_w" if wave else "k_time"
-    traffic_key = ("k_time_w" if wave else "k_time_tiled") + "_taylorf2_tdp_batch%d" % args.batch
+    kname = "k_band" if wave else "k_time"
+    traffic_key = ("k_band" if wave else "k_time_tiled") + "_taylorf2_tdp_batch%d" % args.batch
     traffic = measured_traffic(traffic_key)
     log("%s: %.3f ms/launch, %.1f GB/s algorithmic, measured traffic %s B/launch"
         % (kname, k_ms, achieved, traffic))

@@ -691,8 +691,8 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
       ev.wN[k] = sg2 / s;
     }
   }
-  // TaylorF2 with a 512-point time transform: tables of the wave-per-row
-  // kernel, including prefix sums of f^-7/3 sigma^2 / S over bins 0..N
+  // TaylorF2 with a 512-point time transform: tables of the per-curve
+  // transforms and of the row constants, including prefix sums of f^-7/3 sigma^2 / S over bins 0..N
   const bool wave_tables = ev.approx == GWL_TAYLORF2 && (ev.flags & GWL_TIME_MARG) && ev.P == 512;
   // (and, without time marginalisation, of the inner products)
   const bool inner = ev.approx == GWL_TAYLORF2 && !(ev.flags & GWL_TIME_MARG);

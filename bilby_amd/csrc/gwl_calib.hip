@@ -303,7 +303,7 @@ int calib_create_time(gwl_event* ev, int nc, const double* curves, int K, gwl_ca
   const EvDev& d = ev->dev;
   if (!cal_time_eligible(ev)) {
     set_error("gwl_calib_create: calibration with time marginalisation needs a TaylorF2 event on "
-              "the wave-per-row transform with a time window of at most 512 bins");
+              "512-point transforms with a time window of at most 512 bins");
     return GWL_E_UNSUPPORTED;
   }
   const int nd = d.nd, N = d.N;

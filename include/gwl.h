@@ -214,7 +214,7 @@ int gwl_event_set_tile(gwl_event* ev, int32_t rows_per_workgroup, int32_t workgr
 int gwl_event_set_multi_steps(gwl_event* ev, int32_t steps);
 
 /* Transform of the time-marginalised TaylorF2 path: automatic (the
- * wave-per-row or tiled kernel as gwl_event_set_tile selects) or one of
+ * block-projected or tiled kernel as gwl_event_set_tile selects) or one of
  * them forced.  No counterpart in the reference (kernel choice). */
 enum gwl_transform {
   GWL_TRANSFORM_AUTO = 0, GWL_TRANSFORM_TILED = 1, GWL_TRANSFORM_WAVE = 2
@@ -593,7 +593,7 @@ int gwl_mb_time_series(gwl_mb* mb, const double* params, int64_t n_rows, int32_t
  * Device memory without time marginalisation: the curves in three
  * precisions, (2 n_curves x 2K + n_curves x K) x 16 bytes; the workspace per
  * row ~ 36 K bytes.  With time marginalisation (base.py:305-324; a TaylorF2
- * event on the wave-per-row transform, time window <= 512 bins): the curves
+ * event with 512-point transforms, time window <= 512 bins): the curves
  * in the transform's order as float32 pairs hi + lo (the float64 value to
  * 48 bits) and per-curve prefix sums for <h|h>, n_curves x n_det x N x 24
  * bytes, and the N twiddles W_N^m in float64; per row (1 + n_curves) x 8
