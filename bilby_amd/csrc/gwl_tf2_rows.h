@@ -128,7 +128,11 @@ __device__ __forceinline__ cplx<T> tf2_product(double cycles, const cplx<T>* rot
     y.x = fma(rot[k].x, dw.x, fma(rot[k].y, dw.y, y.x));
     y.y = fma(rot[k].y, dw.x, fma(-rot[k].x, dw.y, y.y));
   }
-  return cmul_fma(expm2pi((T)fract1(cycles)), y);
+  // float32: the nearest whole number is taken off, not the one below, which
+  // halves the rounding of the fraction: every detector of an element shares
+  // it, so its errors add up over them
+  const double x = sizeof(T) == 4 ? cycles - __builtin_rint(cycles) : fract1(cycles);
+  return cmul_fma(expm2pi((T)x), y);
 }
 
 // Rows of one workgroup sorted by reference detector (stable), so that the
