@@ -868,6 +868,30 @@ __device__ inline double spline_x(const SplineDev& sp, const SplineY& yy, double
 // (the library hypot scales first).
 __device__ __forceinline__ double cabs2d(double x, double y) { return sqrt(fma(x, x, y * y)); }
 
+// Twiddle exponents n2 j mod N of the second transform stage, for sub-sequences
+// n2 = first, first + 1, ... (next()) at the bins j of a window of at most P
+// bins from jlo on; N = P Q, P a power of two, any Q.  With j = P a + b it is
+// P (n2 a mod Q) + n2 b, below 2 N, and the window meets two values of a at
+// most: n2 a mod Q is kept for the first and n2 more is the other.
+template <unsigned P>
+struct WindowTwiddle {
+  unsigned a0, Q, n2, c;  // c = n2 a0 mod Q
+  __host__ __device__ WindowTwiddle(int jlo, int q, int first)
+      : a0((unsigned)jlo / P), Q((unsigned)q), n2((unsigned)first),
+        c((unsigned)((unsigned long long)n2 * a0 % Q)) {}
+  __host__ __device__ void next() {
+    ++n2;
+    c += a0;
+    c -= c >= Q ? Q : 0u;
+  }
+  __host__ __device__ unsigned operator()(unsigned j) const {
+    const unsigned d = c + n2;
+    const unsigned m = j / P == a0 ? c : (d >= Q ? d - Q : d);
+    const unsigned i = P * m + n2 * (j % P);
+    return i >= P * Q ? i - P * Q : i;
+  }
+};
+
 // Per-row constants of the TaylorF2 time transforms (k_rowconst).
 struct RowW {
   double c[9];                 // phase coefficients (cycles), tf2_basis order

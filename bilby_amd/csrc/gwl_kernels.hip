@@ -208,10 +208,11 @@ __device__ __forceinline__ void time_tile(const EvDev& ev, int nd, const double*
 #pragma unroll
     for (int jt = 0; jt < JT; ++jt) acc[s][jt][0] = acc[s][jt][1] = 0.0;
   }
-  const unsigned nmask = (unsigned)ev.N - 1u;
-  const R invN = (R)1.0 / (R)ev.N;
+  // (float64, rounded once: 1 / N is no float32 number where N is no power of two)
+  const double invN = 1.0 / (double)ev.N;
+  WindowTwiddle<P> wt(ev.jlo, Q, n2b);
 
-  for (int n2 = n2b; n2 < n2e; ++n2) {
+  for (int n2 = n2b; n2 < n2e; ++n2, wt.next()) {
     // 1) integrand of this decimated sub-sequence, S rows, into LDS
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
@@ -257,8 +258,7 @@ __device__ __forceinline__ void time_tile(const EvDev& ev, int nd, const double*
       const int jj = tid + jt * NT;
       if (jj < ev.L) {
         const unsigned j = (unsigned)(ev.jlo + jj);
-        const unsigned idx = ((unsigned)n2 * j) & nmask;
-        const C t = expm2pi((R)idx * invN);
+        const C t = expm2pi((R)((double)wt(j) * invN));
         const int pj = (int)(j & (unsigned)(P - 1));
 #pragma unroll
         for (int s = 0; s < S; ++s) {

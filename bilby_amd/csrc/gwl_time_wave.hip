@@ -238,10 +238,10 @@ __device__ __forceinline__ void integrand_tf2_det(const WaveEv& ev, const RowW& 
 }
 
 // The three radix-8 passes of one 512-point sub-sequence transform (inputs
-// x[s] = element l + 64 s of lane l) and the window accumulation of
-// sub-sequence n2 into accr / acci (bins j = l + 64 s mod 512), as in
-// wave_row.
-__device__ __forceinline__ void wave_transform_accumulate(const WaveEv& ev, float2* x, int n2,
+// x[s] = element l + 64 s of lane l) and the window accumulation of the
+// sub-sequence of wt into accr / acci (bins j = l + 64 s mod 512).
+__device__ __forceinline__ void wave_transform_accumulate(const WaveEv& ev, float2* x,
+                                                          const WindowTwiddle<kWP>& wt,
                                                           const float2* tw, const float2* tw3,
                                                           float2* xb, int lane, double* accr,
                                                           double* acci) {
@@ -266,15 +266,13 @@ __device__ __forceinline__ void wave_transform_accumulate(const WaveEv& ev, floa
   for (int s = 1; s < 8; ++s) x[s] = cmul(x[s], tw3[(s - 1) * 64 + lane]);
   dft8(x);
   wave_sync();
-  const unsigned nmask = (unsigned)ev.N - 1u;
-  const float invN = 1.0f / (float)ev.N;
+  const double invN = 1.0 / (double)ev.N;
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     const int jj = (lane + 64 * s - ev.jlo) & (kWP - 1);
     if (jj < ev.L) {
       const unsigned j = (unsigned)(ev.jlo + jj);
-      const unsigned idx = ((unsigned)n2 * j) & nmask;
-      const float2 t = expm2pi((float)idx * invN);
+      const float2 t = expm2pi((float)((double)wt(j) * invN));
       const float2 z = cmul(t, x[s]);
       accr[s] += (double)z.x;
       acci[s] += (double)z.y;
@@ -331,7 +329,8 @@ __device__ __forceinline__ void integrand_tf2_det64(const WaveEv& ev, const RowW
 // float64 form of wave_transform_accumulate: the three radix-8 passes in
 // float64 through the wave's exchange buffer, the window accumulation with
 // W_N^(n2 j mod N) from the event's float64 table.
-__device__ __forceinline__ void wave_transform_accumulate64(const WaveEv& ev, double2* x, int n2,
+__device__ __forceinline__ void wave_transform_accumulate64(const WaveEv& ev, double2* x,
+                                                            const WindowTwiddle<kWP>& wt,
                                                             const double2* tw, const double2* tw3,
                                                             double2* xb, int lane,
                                                             const double2* wN, double* accr,
@@ -357,13 +356,12 @@ __device__ __forceinline__ void wave_transform_accumulate64(const WaveEv& ev, do
   for (int s = 1; s < 8; ++s) x[s] = cmul(x[s], tw3[(s - 1) * 64 + lane]);
   dft8(x);
   wave_sync();
-  const unsigned nmask = (unsigned)ev.N - 1u;
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     const int jj = (lane + 64 * s - ev.jlo) & (kWP - 1);
     if (jj < ev.L) {
       const unsigned j = (unsigned)(ev.jlo + jj);
-      const double2 z = cmul(wN[((unsigned)n2 * j) & nmask], x[s]);
+      const double2 z = cmul(wN[wt(j)], x[s]);
       accr[s] += z.x;
       acci[s] += z.y;
     }
@@ -401,7 +399,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
   for (int cc = 0; cc < kCalCurves; ++cc)
 #pragma unroll
     for (int s = 0; s < 8; ++s) accr[cc][s] = acci[cc][s] = 0.0;
-  for (int n2 = 0; n2 < Q; ++n2) {
+  WindowTwiddle<kWP> wt(ev.jlo, Q, 0);
+  for (int n2 = 0; n2 < Q; ++n2, wt.next()) {
     const int ilo = (kb - n2 + Q - 1) / Q;
     const int ihi = ke >= n2 ? (ke - n2) / Q : -1;
     if (ilo > ihi) continue;  // nothing of the support in this sub-sequence
@@ -432,7 +431,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
         }
         x[s] = make_float2(xr, xi);
       }
-      wave_transform_accumulate(wv, x, n2, tw, tw3, xb, lane, accr[cc], acci[cc]);
+      wave_transform_accumulate(wv, x, wt, tw, tw3, xb, lane, accr[cc], acci[cc]);
     }
   }
   // epilogue per curve: time-marginalised lnL (base.py:794-820 per curve)
@@ -522,7 +521,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_cal_time_w64(CalTimeArgs a) 
   for (int cc = 0; cc < kCalCurves; ++cc)
 #pragma unroll
     for (int s = 0; s < 8; ++s) accr[cc][s] = acci[cc][s] = 0.0;
-  for (int n2 = 0; n2 < Q; ++n2) {
+  WindowTwiddle<kWP> wt(ev.jlo, Q, 0);
+  for (int n2 = 0; n2 < Q; ++n2, wt.next()) {
     const int ilo = (kb - n2 + Q - 1) / Q;
     const int ihi = ke >= n2 ? (ke - n2) / Q : -1;
     if (ilo > ihi) continue;
@@ -557,7 +557,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_cal_time_w64(CalTimeArgs a) 
         }
         x[s] = make_double2(xr, xi);
       }
-      wave_transform_accumulate64(wv, x, n2, tw, tw3, xb, lane, a.wN, accr[cc], acci[cc]);
+      wave_transform_accumulate64(wv, x, wt, tw, tw3, xb, lane, a.wN, accr[cc], acci[cc]);
     }
   }
   const double norm = 4.0 / ev.T;
