@@ -274,7 +274,19 @@ __device__ __forceinline__ void band_groups(const BandEv<T>& ev, const BandRow<T
   }
 }
 
-template <typename T, int ND, int R>
+// Groups [ga, gb) that meet bins [kb, ke].  The others' sums are zero, and are
+// neither computed nor written nor read: rows cut at the ISCO use a small part
+// of the band (4096 such rows of 16384 bins, three detectors: 194 us with every
+// group, 95 without; one wavefront per row with the 512-point transform 137).
+// Kernels of events without the cut (CUT false) have none of this, which would
+// take them 1 %.
+template <typename T>
+__device__ __forceinline__ void band_support(int B, int kb, int ke, int& ga, int& gb) {
+  ga = kb / (16 * B);
+  gb = kb <= ke ? min(BandTypes<T>::NB / 16, ke / (16 * B) + 1) : ga;
+}
+
+template <typename T, int ND, int R, bool CUT>
 __device__ __forceinline__ void band_rows(const EvDev& ev, const RowW* rows, long long row0,
                                           long long n, int g0, int g1, int sb, int se, double* out,
                                           size_t row_stride, int lane, int wid) {
@@ -284,7 +296,7 @@ __device__ __forceinline__ void band_rows(const EvDev& ev, const RowW* rows, lon
   const BandEv<T> be = band_ev<T>(ev);
   BandRow<T, ND> b[R];
   double* o[R];
-  int nomask = 1, shared = 1;
+  int nomask = 1, shared = 1, ga = g1, gb = g0;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const RowW& rw = rows[pick[r]];
@@ -292,6 +304,19 @@ __device__ __forceinline__ void band_rows(const EvDev& ev, const RowW* rows, lon
     nomask &= rw.nomask;
     shared &= b[r].ref == b[0].ref;
     o[r] = out + (size_t)pick[r] * row_stride;
+    if constexpr (CUT) {
+      int sa, sz;
+      band_support<T>(be.B, rw.kb, rw.ke, sa, sz);
+      if (sa < sz) {
+        ga = min(ga, sa);
+        gb = max(gb, sz);
+      }
+    }
+  }
+  if constexpr (CUT) {
+    g0 = max(g0, ga);
+    g1 = min(g1, gb);
+    if (g0 >= g1) return;
   }
   if (nomask && shared)
     band_groups<T, ND, R, false, true>(be, b, g0, g1, sb, se, lane, o, live);
@@ -331,7 +356,7 @@ struct BandArgs {
 
 // 2 rows per wavefront share each table load; at 2 wavefronts per SIMD the
 // 256 registers hold both rows' state
-template <typename T, int ND, int R>
+template <typename T, int ND, int R, bool CUT>
 __global__ __launch_bounds__(64 * kBandWaves, 2) void k_band(BandArgs a) {
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -339,7 +364,7 @@ __global__ __launch_bounds__(64 * kBandWaves, 2) void k_band(BandArgs a) {
   int g0, g1, sb, se;
   band_range<T>(band_steps<T>(a.ev.N), a.split, blockIdx.y, g0, g1, sb, se);
   const int ks = blockIdx.y / a.split.gg;
-  band_rows<T, ND, R>(a.ev, a.rows, (long long)blockIdx.x * (kBandWaves * R), a.n, g0, g1, sb, se,
+  band_rows<T, ND, R, CUT>(a.ev, a.rows, (long long)blockIdx.x * (kBandWaves * R), a.n, g0, g1, sb, se,
                       a.out + ks * kRow, kRow * a.split.gs, lane, wid);
 }
 
@@ -475,7 +500,7 @@ __device__ __forceinline__ void fin_distance_values(const SplineDev& sp, const S
 // CU of vector issue, 0.5 of LDS and 0.7 of loads, which overlap only in part
 // at three workgroups per CU (92 us with the distance table gathered from
 // global memory, 68 with the sums staged through LDS first).
-template <typename T>
+template <typename T, bool CUT>
 __device__ __forceinline__ void band_finish_row(const EvDev& ev, const RowW& rw, const double* c,
                                                 int gs, double* out, double2* x, double2* red) {
   constexpr int NB = BandTypes<T>::NB, NG = NB / 16;
@@ -499,12 +524,23 @@ __device__ __forceinline__ void band_finish_row(const EvDev& ev, const RowW& rw,
     const int res = sizeof(T) == 4 ? 4 * h + k : 4 * k + h;
     const double2* src = reinterpret_cast<const double2*>(c) + t;
     double2 y[NG];
+    if constexpr (!CUT) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) y[g] = src[g * 256];
-    for (int i = 1; i < gs; ++i) {
-      src += NB * kNP;
+      for (int g = 0; g < NG; ++g) y[g] = src[g * 256];
+      for (int i = 1; i < gs; ++i) {
+        src += NB * kNP;
 #pragma unroll
-      for (int g = 0; g < NG; ++g) y[g] = cadd(y[g], src[g * 256]);
+        for (int g = 0; g < NG; ++g) y[g] = cadd(y[g], src[g * 256]);
+      }
+    } else {
+      int ga, gb;
+      band_support<T>(ev.N / NB, rw.kb, rw.ke, ga, gb);
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        y[g] = make_double2(0.0, 0.0);
+        if (g >= ga && g < gb)
+          for (int i = 0; i < gs; ++i) y[g] = cadd(y[g], src[g * 256 + i * (NB * kNP)]);
+      }
     }
     if (t < NB) tw[t] = expm2pi((double)t / (double)NB);
     __syncthreads();
@@ -638,13 +674,13 @@ struct FinishArgs {
   double* out;
 };
 
-template <typename T>
+template <typename T, bool CUT>
 __global__ __launch_bounds__(kFinThreads) void k_band_finish(FinishArgs a) {
   extern __shared__ double2 lds[];
   __shared__ double2 red[kFinThreads / 64];
   const long long r = blockIdx.x;
   constexpr size_t kRow = (size_t)BandTypes<T>::NB * kNP * 2;
-  band_finish_row<T>(a.ev, a.rows[r], a.c + (size_t)r * a.gs * kRow, a.gs, a.out + r, lds, red);
+  band_finish_row<T, CUT>(a.ev, a.rows[r], a.c + (size_t)r * a.gs * kRow, a.gs, a.out + r, lds, red);
 }
 
 // ------------------------------------------------------------------ multi-event
@@ -660,6 +696,7 @@ struct BandMultiArgs {
 
 // Workgroup: one item of the longest-first list (8 rows of an event, one of
 // its G parts of the block groups).
+template <bool CUT>
 __global__ __launch_bounds__(64 * kBandWaves, 2) void k_band_multi(BandMultiArgs a) {
   if ((int)blockIdx.x >= *a.n_items) return;
   const MultiItem m = a.items[blockIdx.x];
@@ -672,15 +709,15 @@ __global__ __launch_bounds__(64 * kBandWaves, 2) void k_band_multi(BandMultiArgs
   band_range<float>(band_steps<float>(ev.N), BandSplit{a.groups[m.e], 1}, m.g, g0, g1, sb, se);
   switch (ev.nd) {
     case 1:
-      band_rows<float, 1, 2>(ev, a.roww[m.e], m.row0, a.rows[m.e], g0, g1, sb, se, a.c[m.e], kRow,
+      band_rows<float, 1, 2, CUT>(ev, a.roww[m.e], m.row0, a.rows[m.e], g0, g1, sb, se, a.c[m.e], kRow,
                              lane, wid);
       break;
     case 2:
-      band_rows<float, 2, 2>(ev, a.roww[m.e], m.row0, a.rows[m.e], g0, g1, sb, se, a.c[m.e], kRow,
+      band_rows<float, 2, 2, CUT>(ev, a.roww[m.e], m.row0, a.rows[m.e], g0, g1, sb, se, a.c[m.e], kRow,
                              lane, wid);
       break;
     default:
-      band_rows<float, 3, 2>(ev, a.roww[m.e], m.row0, a.rows[m.e], g0, g1, sb, se, a.c[m.e], kRow,
+      band_rows<float, 3, 2, CUT>(ev, a.roww[m.e], m.row0, a.rows[m.e], g0, g1, sb, se, a.c[m.e], kRow,
                              lane, wid);
   }
 }
@@ -697,6 +734,7 @@ struct FinishMultiArgs {
 };
 
 // One workgroup per row; a block of the list covers kMultiEpiRows rows.
+template <bool CUT>
 __global__ __launch_bounds__(kFinThreads) void k_band_finish_multi(FinishMultiArgs a) {
   extern __shared__ double2 lds[];
   __shared__ double2 red[kFinThreads / 64];
@@ -706,8 +744,8 @@ __global__ __launch_bounds__(kFinThreads) void k_band_finish_multi(FinishMultiAr
   const long long r = a.block_row0[blk] + blockIdx.x % kMultiEpiRows;
   if (r >= a.rows[e]) return;
   constexpr size_t kRow = (size_t)BandTypes<float>::NB * kNP * 2;
-  band_finish_row<float>(a.evs[e], a.roww[e][r], a.c[e] + (size_t)r * kRow, 1, a.out[e] + r, lds,
-                         red);
+  band_finish_row<float, CUT>(a.evs[e], a.roww[e][r], a.c[e] + (size_t)r * kRow, 1, a.out[e] + r,
+                              lds, red);
 }
 
 // ------------------------------------------------------------------ tables
@@ -949,18 +987,26 @@ BandSplit band_split(const gwl_event* e, long long n, int& R) {
   return sp;
 }
 
-template <typename T, int ND>
-void launch_band(const BandArgs& a, int R, hipStream_t st) {
+template <typename T, int ND, bool CUT>
+void launch_band_cut(const BandArgs& a, int R, hipStream_t st) {
   const unsigned nsplit = (unsigned)(a.split.gg * a.split.gs);
   const long long per = kBandWaves * R;
   const dim3 grid((unsigned)((a.n + per - 1) / per), nsplit);
   if constexpr (sizeof(T) == 4) {
     if (R == 2) {
-      hipLaunchKernelGGL((k_band<T, ND, 2>), grid, dim3(64 * kBandWaves), 0, st, a);
+      hipLaunchKernelGGL((k_band<T, ND, 2, CUT>), grid, dim3(64 * kBandWaves), 0, st, a);
       return;
     }
   }
-  hipLaunchKernelGGL((k_band<T, ND, 1>), grid, dim3(64 * kBandWaves), 0, st, a);
+  hipLaunchKernelGGL((k_band<T, ND, 1, CUT>), grid, dim3(64 * kBandWaves), 0, st, a);
+}
+
+bool cut_rows(const EvDev& ev) { return (ev.flags & GWL_TF2_END_ISCO) != 0; }
+
+template <typename T, int ND>
+void launch_band(const BandArgs& a, int R, hipStream_t st) {
+  if (cut_rows(a.ev)) launch_band_cut<T, ND, true>(a, R, st);
+  else launch_band_cut<T, ND, false>(a, R, st);
 }
 
 }  // namespace
@@ -1033,7 +1079,8 @@ int launch_band_eval_t(gwl_event* e, const double* params, int64_t n, int ld, do
     GWL_HIP_CHECK(hipGetLastError());
     if (int rc = timing_end(e, st)) return rc;
     FinishArgs f{ev, rows + r0, c, a.split.gs, out + r0};
-    hipLaunchKernelGGL(k_band_finish<T>, dim3((unsigned)m), dim3(kFinThreads), lds, st, f);
+    hipLaunchKernelGGL((cut_rows(ev) ? k_band_finish<T, true> : k_band_finish<T, false>),
+                       dim3((unsigned)m), dim3(kFinThreads), lds, st, f);
     GWL_HIP_CHECK(hipGetLastError());
   }
   return GWL_OK;
@@ -1090,7 +1137,10 @@ int band_multi_launch(gwl_multi* m, hipStream_t st) {
   // eager launches cover the current lists; a captured graph, the largest ones
   const size_t items = m->capturing ? m->max_items : (size_t)std::max(1, m->n_items);
   const size_t blocks = m->capturing ? m->max_blocks : (size_t)std::max(1, m->n_blocks);
-  hipLaunchKernelGGL(k_band_multi, dim3((unsigned)items), dim3(64 * kBandWaves), 0, st, a);
+  bool cut = false;
+  for (const gwl_event* e : m->events) cut = cut || cut_rows(e->dev);
+  hipLaunchKernelGGL(cut ? k_band_multi<true> : k_band_multi<false>, dim3((unsigned)items),
+                     dim3(64 * kBandWaves), 0, st, a);
   GWL_HIP_CHECK(hipGetLastError());
   FinishMultiArgs f;
   f.evs = m->d_evs;
@@ -1101,8 +1151,9 @@ int band_multi_launch(gwl_multi* m, hipStream_t st) {
   f.block_event = m->d_block_event;
   f.block_row0 = m->d_block_row0;
   f.n_blocks = m->d_n_blocks;
-  hipLaunchKernelGGL(k_band_finish_multi, dim3((unsigned)(blocks * kMultiEpiRows)),
-                     dim3(kFinThreads), band_multi_lds_bytes(), st, f);
+  hipLaunchKernelGGL(cut ? k_band_finish_multi<true> : k_band_finish_multi<false>,
+                     dim3((unsigned)(blocks * kMultiEpiRows)), dim3(kFinThreads),
+                     band_multi_lds_bytes(), st, f);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }

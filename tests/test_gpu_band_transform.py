@@ -57,3 +57,46 @@ def test_window_transform_matches_oracle(case, precision, split):
     # float64: 1e-14 (block functions at 512 bins) and the sums' rounding
     tol = 1e-3 if precision == "fp32" else 1e-10
     assert np.max(np.abs(out - ref)) < tol, np.abs(out - ref).max()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("rows", [6, 300])
+def test_rows_cut_at_the_isco(precision, rows):
+    """Supports that end in the first, a middle and the last group of blocks, past
+    the band and below its start (no bin at all), mixed within workgroups, few
+    rows (the steps are split) and more; alone, and as one of several events of
+    which the other has no cut."""
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    from bilby_amd.multi import MultiEventLikelihood
+    from tests.helpers import draws_as_dicts, fixed_marginalised, oracle_from_setup
+    lks, draws, sets = [], [], []
+    for termination in ("isco", None):
+        s = make_taylorf2_marginalised(n_draws=rows, seed=33, duration=4.0,
+                                       sampling_frequency=2048.0, detectors=("H1", "L1"),
+                                       distance=False, taylorf2_termination=termination)
+        # f_ISCO = 4397 Hz / (total mass): 14.7, 29, 129, 550, 970, 1465 Hz of 1024
+        total = np.resize([300.0, 150.0, 34.0, 8.0, 4.53, 3.0], rows)
+        s["draws"]["mass_1"], s["draws"]["mass_2"] = 0.55 * total, 0.45 * total
+        priors = s["priors"].copy()
+        lks.append(GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                              time_marginalization=True,
+                                              phase_marginalization=True, priors=priors,
+                                              precision=precision))
+        draws.append(fixed_marginalised(s["draws"], priors))
+        sets.append(s)
+    out = lks[0].log_likelihood_ratio_batch(draws[0])
+    olk, _ = oracle_from_setup(sets[0])
+    pick = list(range(6)) + [rows - 1]
+    ref = np.array([olk.log_likelihood_ratio(p) for p in draws_as_dicts(draws[0], pick)])
+    # (tolerances as above)
+    tol = 1e-3 if precision == "fp32" else 1e-10
+    assert np.max(np.abs(out[pick] - ref)) < tol, np.abs(out[pick] - ref).max()
+    if precision == "fp32":
+        multi = MultiEventLikelihood(lks, [rows, rows])
+        for e in range(2):
+            multi.set_parameters(e, draws[e])
+        got = [o.cpu().numpy() for o in multi.run()]
+        for e in range(2):  # the same float32 sums, added in float64 in another order
+            one = lks[e].log_likelihood_ratio_batch(draws[e])
+            assert np.max(np.abs(got[e] - one)) < 1e-8
