@@ -683,6 +683,40 @@ __global__ __launch_bounds__(kFinThreads) void k_band_finish(FinishArgs a) {
   band_finish_row<T, CUT>(a.ev, a.rows[r], a.c + (size_t)r * a.gs * kRow, a.gs, a.out + r, lds, red);
 }
 
+// float64 rows of short segments: both in one workgroup per row.  A row's block
+// sums are 64 KB, more than it reads otherwise; here they stay in the LDS that
+// k_band_finish loads them to (the same values, bit for bit).  1024 bins, two
+// detectors, 4096 rows: 165 us in two kernels, 121 in one (148 with tiles of
+// 512-point transforms, k_time); 16384 rows: 632, 444 (432).
+template <int ND, bool CUT>
+__global__ __launch_bounds__(kFinThreads) void k_band_row(BandArgs a) {
+  using T = double;
+  extern __shared__ double2 lds[];
+  __shared__ double2 red[kFinThreads / 64];
+  const long long r = blockIdx.x;
+  const RowW& rw = a.rows[r];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const BandEv<T> be = band_ev<T>(a.ev);
+  constexpr int per = BandTypes<T>::NB / 16 / (kFinThreads / 64);  // groups a wavefront
+  int g0 = wid * per, g1 = g0 + per;
+  if constexpr (CUT) {
+    int ga, gb;
+    band_support<T>(be.B, rw.kb, rw.ke, ga, gb);
+    g0 = max(g0, ga);
+    g1 = min(g1, gb);
+  }
+  if (rw.valid && g0 < g1) {
+    BandRow<T, ND> b[1];
+    band_row<T, ND>(be, rw, b[0]);
+    double* const o[1] = {reinterpret_cast<double*>(lds)};
+    if (rw.nomask) band_groups<T, ND, 1, false, true>(be, b, g0, g1, 0, be.S, lane, o, 1);
+    else band_groups<T, ND, 1, true, true>(be, b, g0, g1, 0, be.S, lane, o, 1);
+  }
+  __syncthreads();
+  band_finish_row<T, CUT>(a.ev, rw, reinterpret_cast<const double*>(lds), 1, a.out + r, lds, red);
+}
+
 // ------------------------------------------------------------------ multi-event
 struct BandMultiArgs {
   const EvDev* evs;
@@ -1009,6 +1043,18 @@ void launch_band(const BandArgs& a, int R, hipStream_t st) {
   else launch_band_cut<T, ND, false>(a, R, st);
 }
 
+template <int ND>
+void launch_band_row(const BandArgs& a, size_t lds, hipStream_t st) {
+  const dim3 grid((unsigned)a.n), block(kFinThreads);
+  if (cut_rows(a.ev)) hipLaunchKernelGGL((k_band_row<ND, true>), grid, block, lds, st, a);
+  else hipLaunchKernelGGL((k_band_row<ND, false>), grid, block, lds, st, a);
+}
+
+// One kernel from a row per CU on, on segments where it was slower than k_time.
+bool band_row_wins(const gwl_event* e, int64_t n) {
+  return e->dev.N <= 2048 && n >= e->ctx->n_cu;
+}
+
 }  // namespace
 
 namespace {
@@ -1057,6 +1103,22 @@ int launch_band_eval_t(gwl_event* e, const double* params, int64_t n, int ld, do
     return GWL_E_UNSUPPORTED;
   }
   if (int rc = launch_rowconst(e, params, n, ld, rows, st)) return rc;
+  if (sizeof(T) == 8 && band_row_wins(e, n)) {
+    BandArgs a{};
+    a.ev = ev;
+    a.rows = rows;
+    a.n = n;
+    a.out = out;
+    if (int rc = timing_begin(e, st)) return rc;
+    switch (ev.nd) {
+      case 1: launch_band_row<1>(a, lds, st); break;
+      case 2: launch_band_row<2>(a, lds, st); break;
+      case 3: launch_band_row<3>(a, lds, st); break;
+      default: launch_band_row<4>(a, lds, st); break;
+    }
+    GWL_HIP_CHECK(hipGetLastError());
+    return timing_end(e, st);
+  }
   const long long tile = std::min<long long>(
       std::min<long long>(room, kPassBytes / band_row_bytes<T>()), n);
   for (long long r0 = 0; r0 < n; r0 += tile) {

@@ -144,6 +144,12 @@ int launch_epi_time(gwl_event* ev, const double* params, int64_t n, int ld, int 
 // (count: only rows r < *count exist; zero: cleared first)
 int launch_rowconst(const gwl_event* ev, const double* params, int64_t n, int ld, RowW* rows,
                     hipStream_t stream, const int* count = nullptr, int* zero = nullptr);
+// short segments: whole evaluation of a row by one wavefront (float32), where
+// it is faster than block projections
+constexpr int kTimeRowBins = 8192;
+bool time_row_wins(const gwl_event* ev, int64_t rows);
+int launch_time_row(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
+                    hipStream_t stream);
 int multi_launch_rowconst(gwl_multi* m, hipStream_t stream);
 int init_time_wave_tables(const EvDev& ev, double* tf2b, float2* dwa32);
 // block-projected window transform (gwl_band.hip)

@@ -1116,7 +1116,10 @@ static int eval_typed(gwl_event* e, const double* params, int64_t n, int ld, dou
   const EvDev& ev = e->dev;
   if constexpr (WAVE == GWL_TAYLORF2) {
     constexpr bool fp64 = std::is_same<R, double>::value;
-    if (band_eligible(e, fp64)) return launch_band_eval(e, fp64, params, n, ld, out, st);
+    if (band_eligible(e, fp64)) {
+      if (!fp64 && time_row_wins(e, n)) return launch_time_row(e, params, n, ld, out, st);
+      return launch_band_eval(e, fp64, params, n, ld, out, st);
+    }
   }
   if (ev.flags & GWL_TIME_MARG) {
     // a window longer than one transform: slices of P bins, one pass each,

@@ -1,12 +1,14 @@
 // Per-row constants of the TaylorF2 time-marginalised likelihood (k_rowconst:
 // phase coefficients, detector amplitudes and delays, support, and <h|h> from
-// per-event prefix sums of f^-7/3 sigma^2 / S, gw/utils.py:118-138), and the
+// per-event prefix sums of f^-7/3 sigma^2 / S, gw/utils.py:118-138), the
+// evaluation of short segments by one wavefront per row, and the
 // window transform under calibration marginalisation: one wavefront per (row,
 // pair of response curves), 512-point transforms of the decimated
 // sub-sequences as three radix-8 passes on registers (lane l holds elements
 // l + 64 s) with two LDS transposes private to the wavefront, the window bins
 // accumulated in float64.
 #include "gwl_internal.h"
+#include "gwl_tf2_rows.h"
 
 #include <algorithm>
 
@@ -192,6 +194,200 @@ __device__ __forceinline__ WaveEv wave_ev(const EvDev& ev) {
   w.nd = ev.nd;
   w.pad = 0;
   return w;
+}
+
+// ------------------------------------------------------------------ short segments
+// One wavefront evaluates one row from the integrand to the marginalised lnL
+// (float32 integrand, float64 from there on): 512-point transforms of the Q
+// sub-sequences as three radix-8 passes on registers with two exchanges
+// through LDS private to the wavefront, the window sums by Horner's rule over
+// descending sub-sequences (acc <- acc W_N^j + Y_n2[j mod 512]), the
+// marginalisation (base.py:794-820) in the same wavefront.
+//
+// Bound: vector issue.  Block projections (gwl_band.hip) take half of the
+// instructions a bin but finish a row in 15 to 20 ns however short the segment
+// is; here that is 3 to 6.  The transform is float64 because its vector
+// instructions issue at the rate of unpacked float32 ones: float32 passes were
+// 9 % faster (4096 rows of 4096 bins, two detectors) at 1.4 times the error.
+// Exchanges move the real parts, then the imaginary ones, which leaves room for
+// four workgroups a CU (76 us; whole values at three 87); the integrand stays
+// in float32 until all of it is there (68).
+constexpr int kTw2 = 7 * 8;  // pass-2 twiddles W_64^(s k), [s - 1][k]
+
+// tw2[s - 1][k] = W_64^(s k) (lane l uses k = l mod 8), tw3[s - 1][l] =
+// W_512^(s l), and wt[l + 64 s] = W_N^j for the window bin j = l + 64 s (mod 512).
+__device__ inline void init_row_tables(double2* tw2, double2* tw3, double2* wt, int N, int jlo) {
+  double sn, cs;
+  for (int k = threadIdx.x; k < kTw2; k += 64 * kWaves) {
+    sincospi(-2.0 * (double)(((k / 8 + 1) * (k & 7)) & 63) / 64.0, &sn, &cs);
+    tw2[k] = make_double2(cs, sn);
+  }
+  for (int k = threadIdx.x; k < kTw3; k += 64 * kWaves) {
+    sincospi(-2.0 * (double)(((k / 64 + 1) * (k & 63)) & (kWP - 1)) / (double)kWP, &sn, &cs);
+    tw3[k] = make_double2(cs, sn);
+  }
+  for (int k = threadIdx.x; k < kWP; k += 64 * kWaves) {
+    const int j = jlo + ((k - jlo) & (kWP - 1));
+    sincospi(-2.0 * (double)j / (double)N, &sn, &cs);
+    wt[k] = make_double2(cs, sn);
+  }
+}
+
+// x[s] goes to element to + s step, then lane l takes elements l + 64 s: the
+// real parts, then the imaginary ones through the same buffer.
+__device__ __forceinline__ void row_exchange(double2* x, double* xb, int to, int step, int lane) {
+#pragma unroll
+  for (int s = 0; s < 8; ++s) xb[xpad(to + s * step)] = x[s].x;
+  wave_sync();
+#pragma unroll
+  for (int s = 0; s < 8; ++s) x[s].x = xb[xpad(lane + 64 * s)];
+  wave_sync();
+#pragma unroll
+  for (int s = 0; s < 8; ++s) xb[xpad(to + s * step)] = x[s].y;
+  wave_sync();
+#pragma unroll
+  for (int s = 0; s < 8; ++s) x[s].y = xb[xpad(lane + 64 * s)];
+  wave_sync();
+}
+
+// A row's constants, with the detectors' rotations of one step of 64 elements
+// and their tables, the reference detector's first.
+template <int ND>
+struct TimeRow : Tf2Row<float, ND> {
+  static constexpr int NO = ND - 1;
+  float2 w[NO > 0 ? NO : 1];
+  const float2* dwr;
+  const float2* dwo[NO > 0 ? NO : 1];
+};
+
+// Sub-sequence n2 of one row: integrand (with MASK, zero outside [kb, ke], and
+// slots of 64 elements outside it are not evaluated), transform, Horner step.
+template <int ND, bool MASK>
+__device__ __forceinline__ void time_row_step(const WaveEv& ev, const TimeRow<ND>& b, int n2,
+                                              const double2* tw2l, const double2* tw3,
+                                              const double2* wt, double* xb, int lane, int base2,
+                                              double* accr, double* acci) {
+  constexpr int NO = ND - 1;
+  const int Q = ev.Q;
+  // elements of the support: kb <= Q i + n2 <= ke
+  const int ilo = MASK ? (b.kb - n2 + Q - 1) / Q : 0;
+  const int ihi = !MASK ? kWP - 1 : b.ke >= n2 ? (b.ke - n2) / Q : -1;
+  double2 x[8];
+  if (ilo <= ihi) {  // (uniform)
+    const double f0 = (double)(Q * lane + n2) * ev.df;
+    float2 rot[NO > 0 ? NO : 1];
+#pragma unroll
+    for (int k = 0; k < NO; ++k) rot[k] = tf2_rotated<float, ND>(b, k, f0);
+    const size_t e0 = (size_t)n2 * kWP + lane;
+    const double* tb = ev.tf2b + 3 * e0;
+    float2 v[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      v[s] = make_float2(0.f, 0.f);
+      if (!MASK || (64 * s <= ihi && 64 * s + 63 >= ilo)) {  // (uniform)
+        float2 d[ND][2];
+        d[0][0] = b.dwr[e0 + 64 * s];
+#pragma unroll
+        for (int k = 0; k < NO; ++k) d[k + 1][0] = b.dwo[k][e0 + 64 * s];
+        const double* t = tb + 3 * 64 * s;
+        v[s] = tf2_product<float, ND>(tf2_cycles<float, ND>(b, t[0], t[1], t[2]), rot, d, 0);
+        if constexpr (MASK) {
+          const int i = lane + 64 * s;
+          const bool in = i >= ilo && i <= ihi;
+          v[s] = make_float2(in ? v[s].x : 0.f, in ? v[s].y : 0.f);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NO; ++k) rot[k] = cmul_fma(rot[k], b.w[k]);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) x[s] = make_double2(v[s].x, v[s].y);
+    dft8(x);
+    row_exchange(x, xb, 8 * lane, 1, lane);
+#pragma unroll
+    for (int s = 1; s < 8; ++s) x[s] = cmul(x[s], tw2l[(s - 1) * 8]);
+    dft8(x);
+    row_exchange(x, xb, base2, 8, lane);
+#pragma unroll
+    for (int s = 1; s < 8; ++s) x[s] = cmul(x[s], tw3[(s - 1) * 64 + lane]);
+    dft8(x);
+  } else {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) x[s] = make_double2(0.0, 0.0);
+  }
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const double2 w = wt[lane + 64 * s];
+    const double ar = accr[s], ai = acci[s];
+    accr[s] = fma(ar, w.x, fma(-ai, w.y, x[s].x));
+    acci[s] = fma(ar, w.y, fma(ai, w.x, x[s].y));
+  }
+}
+
+struct TimeRowArgs {
+  EvDev ev;
+  const RowW* rows;
+  long long n;
+  double* out;
+};
+
+template <int ND>
+__global__ __launch_bounds__(64 * kWaves, 4) void k_time_row(TimeRowArgs a) {
+  __shared__ double2 wt[kWP], tw2[kTw2], tw3[kTw3];
+  __shared__ double xch[kWaves * kXch];
+  const EvDev& ev = a.ev;
+  init_row_tables(tw2, tw3, wt, ev.N, ev.jlo);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long r = (long long)blockIdx.x * kWaves + wid;
+  if (r >= a.n) return;
+  const RowW& rw = a.rows[r];
+  if (!rw.valid) {
+    if (lane == 0) a.out[r] = row_valid_sentinel();
+    return;
+  }
+  const WaveEv wv = wave_ev(ev);
+  TimeRow<ND> b;
+  tf2_row<float, ND>(rw, b);
+#pragma unroll
+  for (int k = 0; k < ND - 1; ++k) {
+    double2 corr = make_double2(1.0, 0.0);
+    b.w[k] = tf2_rotation<float>((64.0 * (double)ev.Q * ev.df) * b.dd[k], 3.5, corr);
+    tf2_rho<float, ND>(rw, k, corr, b);
+    b.dwo[k] = ev.dwa32 + (size_t)(k < b.ref ? k : k + 1) * ev.N;
+  }
+  b.dwr = ev.dwa32 + (size_t)b.ref * ev.N;
+  double* xb = xch + wid * kXch;
+  const double2* tw2l = tw2 + (lane & 7);
+  const int base2 = 64 * (lane >> 3) + (lane & 7);
+  double accr[8], acci[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) accr[s] = acci[s] = 0.0;
+  if (rw.nomask)
+    for (int n2 = ev.Q - 1; n2 >= 0; --n2)
+      time_row_step<ND, false>(wv, b, n2, tw2l, tw3, wt, xb, lane, base2, accr, acci);
+  else
+    for (int n2 = ev.Q - 1; n2 >= 0; --n2)
+      time_row_step<ND, true>(wv, b, n2, tw2l, tw3, wt, xb, lane, base2, accr, acci);
+  const double norm = 4.0 / ev.T, amp = rw.amp * norm;
+  const double hh = rw.hh * norm, hs = rw.hscale, jit = rw.jitter;
+  SplineY yy;
+  if (ev.flags & GWL_DISTANCE_MARG) yy = spline_y(ev.sp, hh * hs * hs);
+  double m = -INFINITY, sum = 0.0;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int jj = (lane + 64 * s - ev.jlo) & (kWP - 1);
+    if (jj < ev.L) {
+      const double t = (ev.start + (double)(ev.jlo + jj + 1) * ev.tstep) + jit;
+      if (t >= ev.tmin && t <= ev.tmax)
+        lse_push(m, sum, epi_value(ev.flags, ev.sp, yy, hh, hs, amp * accr[s], amp * acci[s]) +
+                             time_log_weight(ev, t));
+    }
+  }
+  lse_wave(m, sum);
+  if (lane == 0)
+    a.out[r] = (m > -INFINITY) ? log(time_lse_scale(ev, ev.tdelta) * sum) + m : -INFINITY;
 }
 
 // ------------------------------------------------------------------ calibration
@@ -673,6 +869,41 @@ int launch_rowconst(const gwl_event* e, const double* params, int64_t n, int ld,
                      dim3(2 * kRowconstRows), 0, st, ra);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
+}
+
+// Short segments and many rows: a wavefront per row fills the chip from about
+// 16 rows per CU on, and its time goes with the bins; block projections keep
+// the chip busy with few rows, and most of their time goes with the rows.
+// Per launch, us, this and block projections, two detectors: 1024 bins 23 and 31
+// (512 rows), 24 and 49 (1024), 36 and 91 (4096), 105 and 339 (16384); 2048 bins
+// 33 and 46 (1024), 53 and 88 (4096); 4096 bins 47 and 68 (2048), 68 and 102
+// (4096), 229 and 384 (16384); 8192 bins 116 and 123 (4096), 406 and 468 (16384);
+// below the line 4096 bins 48 and 51 (1024), 8192 bins 85 and 78 (2048).
+bool time_row_wins(const gwl_event* e, int64_t n) {
+  return e->transform == GWL_TRANSFORM_AUTO && e->dev.tf2b && e->dev.N <= kTimeRowBins &&
+         512 * n >= (int64_t)e->ctx->n_cu * e->dev.N;
+}
+
+int launch_time_row(gwl_event* e, const double* params, int64_t n, int ld, double* out,
+                    hipStream_t st) {
+  const EvDev& ev = e->dev;
+  RowW* rows = reinterpret_cast<RowW*>(e->ws);
+  if (roww_bytes(n) > e->ws_bytes) {
+    set_error("workspace too small for the time transform");
+    return GWL_E_INVALID;
+  }
+  if (int rc = launch_rowconst(e, params, n, ld, rows, st)) return rc;
+  const TimeRowArgs a{ev, rows, (long long)n, out};
+  const dim3 grid((unsigned)((n + kWaves - 1) / kWaves)), block(64 * kWaves);
+  if (int rc = timing_begin(e, st)) return rc;
+  switch (ev.nd) {
+    case 1: hipLaunchKernelGGL(k_time_row<1>, grid, block, 0, st, a); break;
+    case 2: hipLaunchKernelGGL(k_time_row<2>, grid, block, 0, st, a); break;
+    case 3: hipLaunchKernelGGL(k_time_row<3>, grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL(k_time_row<4>, grid, block, 0, st, a); break;
+  }
+  GWL_HIP_CHECK(hipGetLastError());
+  return timing_end(e, st);
 }
 
 size_t roww_bytes(int64_t rows) { return (size_t)rows * sizeof(RowW); }
