@@ -1181,28 +1181,35 @@ static int eval_nd(gwl_event* e, const double* params, int64_t n, int ld, double
   return GWL_E_INVALID;
 }
 
+// The tiled transform's workspace: partials [n][G][L] double2 + [n][G] double;
+// n G <= max(n, 2 S 8 n_cu) for every n <= rows (G halves as the row blocks
+// double).
+static size_t tiled_ws_bytes(const gwl_event* e, int64_t rows) {
+  const EvDev& ev = e->dev;
+  const int S = time_tile_rows(ev.P, rows, e->tile_rows);
+  const int wpc = e->tile_wg_per_cu > 0 ? e->tile_wg_per_cu : 8;
+  const long long bound = std::max<long long>(
+      (long long)rows * time_tile_groups(ev, rows, S, e->ctx->n_cu, e->tile_wg_per_cu),
+      2LL * 8 * wpc * e->ctx->n_cu);
+  return (size_t)bound * (std::min(ev.L, ev.P) * sizeof(double2) + sizeof(double)) +
+         time_lse_bytes(rows) + (size_t)rows * 4 * sizeof(double) + 4096;
+}
+
+// What one evaluation needs on the path it will take.
 size_t workspace_bytes_for(const gwl_event* e, int64_t rows, int precision) {
   // the block-projected transform uses its own workspace only, in as many
   // passes as it takes
   const bool fp64 = precision == GWL_FP64;
   if (band_eligible(e, fp64)) return band_ws_min_bytes(e, rows, fp64);
-  return workspace_bytes(e, rows);
+  return e->dev.flags & GWL_TIME_MARG ? tiled_ws_bytes(e, rows) : workspace_bytes(e, rows);
 }
 
+// Room for any path and precision.
 size_t workspace_bytes(const gwl_event* e, int64_t rows) {
   const EvDev& ev = e->dev;
   if (ev.flags & GWL_TIME_MARG) {
-    // partials [n][G][L] double2 + [n][G] double; n G <= max(n, 2 S 8 n_cu)
-    // for every n <= rows (G halves as the row blocks double)
-    const int S = time_tile_rows(ev.P, rows, e->tile_rows);
-    const int wpc = e->tile_wg_per_cu > 0 ? e->tile_wg_per_cu : 8;
-    const long long bound = std::max<long long>(
-        (long long)rows * time_tile_groups(ev, rows, S, e->ctx->n_cu, e->tile_wg_per_cu),
-        2LL * 8 * wpc * e->ctx->n_cu);
-    size_t b = (size_t)bound * (std::min(ev.L, ev.P) * sizeof(double2) + sizeof(double)) +
-               time_lse_bytes(rows) + (size_t)rows * 4 * sizeof(double) + 4096;
-    if (ev.band32.uv) b = std::max(b, band_ws_bytes(e, rows));
-    return b;
+    const size_t b = tiled_ws_bytes(e, rows);
+    return ev.band32.uv ? std::max(b, band_ws_bytes(e, rows)) : b;
   }
   if (ev.approx == GWL_TAYLORF2) {
     InnerWs ws;

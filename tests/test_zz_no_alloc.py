@@ -100,3 +100,34 @@ def test_noalloc_rejects_a_batch_beyond_the_scratch():
     assert rc != 0
     assert b"scratch" in LIB.gwl_last_error()
     assert float(out.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("duration, precision, transform", [
+    (4.0, "fp32", 1),     # the tiled transform, forced
+    (1.5, "fp64", 0),     # 1536 bins: float64 has no block projections
+])
+def test_noalloc_takes_the_tiled_transform_of_a_short_window(duration, precision, transform):
+    """A window of 14 bins needs 232 bytes a row and group: 2000 rows fit the
+    scratch, whatever other transforms of the event would need."""
+    from bilby_amd._lib import LIB, FP32, FP64
+    from bilby_amd.autotune import set_transform
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    from bilby_amd.prior import Uniform
+    from tests.helpers import fixed_marginalised
+    s = make_taylorf2_marginalised(n_draws=2000, seed=8, duration=duration,
+                                   sampling_frequency=2048.0, detectors=("H1", "L1"),
+                                   distance=False)
+    centre = s["priors"]["geocent_time"].minimum + 0.1
+    s["priors"]["geocent_time"] = Uniform(centre - 0.002, centre + 0.002, name="geocent_time")
+    priors = s["priors"].copy()
+    lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                    time_marginalization=True, phase_marginalization=True,
+                                    priors=priors, precision=precision)
+    set_transform(lk, transform)
+    rows = _rows(lk, fixed_marginalised(s["draws"], priors))
+    prec = FP64 if precision == "fp64" else FP32
+    rc0, ref, _ = _eval(LIB.gwl_eval, lk, rows, prec)
+    rc1, got, _ = _eval(LIB.gwl_eval_noalloc, lk, rows, prec)
+    assert rc0 == 0 and rc1 == 0, LIB.gwl_last_error()
+    assert np.array_equal(got, ref)
