@@ -43,3 +43,26 @@ def test_inner_products_match_oracle(case, precision):
     # a row's value does not depend on its slot or its partner
     again = lk.log_likelihood_ratio_batch({k: v[::-1].copy() for k, v in s["draws"].items()})
     assert np.array_equal(again[::-1], out)
+
+
+@pytest.mark.parametrize("duration", [8.0, 32.0])
+def test_prefix_sums_of_hh_are_rounded_once(duration):
+    """<h|h> comes from per-event prefix sums, so their error would be that of
+    every row.  Bound: the row's amplitude and the oracle's take about ten
+    roundings each (1e-15, random over rows: the median of 40 is a few times
+    below), the sums themselves one; rounded at each of 16384 steps and more they
+    are 5e-15 and more off."""
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    from tests.helpers import draws_as_dicts, oracle_from_setup
+    s = make_taylorf2_marginalised(n_draws=40, seed=6, duration=duration,
+                                   sampling_frequency=4096.0, detectors=("H1",), time=False,
+                                   distance=False, phase=False)
+    lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                    precision="fp64")
+    _, aux = lk.log_likelihood_ratio_batch(s["draws"], return_inner_products=True)
+    olk, _ = oracle_from_setup(s)
+    hh = np.array([olk.plain_inner_products(p)[1]
+                   for p in draws_as_dicts(s["draws"], range(40))])
+    rel = aux[:, 2] / hh - 1.0
+    assert np.abs(np.median(rel)) < 1e-15, (np.median(rel), np.abs(rel).max())
