@@ -804,7 +804,7 @@ __global__ __launch_bounds__(256) void k_band_tables(EvDev ev, int jd, double2* 
     tf2_basis((double)n * ev.df, b);
     b2 = make_double2(b[5], b[3]);
     ln = b[7];
-    amp = b[1] * sqrt(b[3]);
+    amp = b[1] * sqrt(b[3]) * (sizeof(T) == 4 ? kExpm2piGain : 1.0);
   }
   const long long e2 = (((long long)g * (S / 2) + (s >> 1)) * 64 + l) * 2 + (s & 1);
   uv[e] = b2;

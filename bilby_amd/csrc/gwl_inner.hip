@@ -215,7 +215,8 @@ __global__ __launch_bounds__(256) void k_inner_tables(EvDev ev, double2* uv, dou
     else if (n == ev.N) w = make_double2(ev.dwN[d][0], ev.dwN[d][1]);
     w = make_double2(w.x * amp, w.y * amp);
     dw64[(size_t)d * M + n] = w;
-    dw32[(size_t)d * M + n] = make_float2((float)w.x, (float)w.y);
+    dw32[(size_t)d * M + n] =
+        make_float2((float)(w.x * kExpm2piGain), (float)(w.y * kExpm2piGain));
   }
 }
 

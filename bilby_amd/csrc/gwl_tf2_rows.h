@@ -38,7 +38,7 @@ __device__ __forceinline__ void load_pair(const C* p, unsigned off, C* to) {
 // The integrand is |C_r| exp(-2 pi i phi(f)) [conj(dw_r) + sum_k rho_k
 // exp(-2 pi i f (dt_k - dt_r)) conj(dw_k)] with r the row's reference detector
 // (its largest amplitude) and phi(f) = Psi(f) / 2pi + f dt_r - arg(C_r) / 2pi
-// in float64, reduced to [0, 1) cycles before the sin / cos; |C_r| scales the
+// in float64, without whole cycles before the sin / cos; |C_r| scales the
 // row's result.
 template <typename T, int ND>
 struct Tf2Row {
@@ -82,19 +82,30 @@ __device__ __forceinline__ cplx<T> tf2_rotation(double cycles, double mean, doub
   return r;
 }
 
-// rho_k times the rotations' correction, as a sum of two numbers.
+// rho_k times the rotations' correction and, in float32, the gain of
+// tf2_rotated's exponential (the shared one's is in the tables), as a sum of
+// two numbers.
 template <typename T, int ND>
 __device__ __forceinline__ void tf2_rho(const RowW& rw, int k, double2 corr, Tf2Row<T, ND>& b) {
-  const double pr = rw.rre[k] * corr.x - rw.rim[k] * corr.y;
-  const double pi = rw.rre[k] * corr.y + rw.rim[k] * corr.x;
+  constexpr double gain = sizeof(T) == 4 ? kExpm2piGain : 1.0;
+  const double pr = gain * (rw.rre[k] * corr.x - rw.rim[k] * corr.y);
+  const double pi = gain * (rw.rre[k] * corr.y + rw.rim[k] * corr.x);
   b.rho[k] = cmk<cplx<T>>((T)pr, (T)pi);
   b.rlo[k] = cmk<cplx<T>>((T)(pr - (double)b.rho[k].x), (T)(pi - (double)b.rho[k].y));
+}
+
+// Cycles without their whole number.  float32: the nearest one is taken off,
+// not the one below, which halves the rounding of the fraction: every detector
+// of an element shares it, so its errors add up over them.
+template <typename T>
+__device__ __forceinline__ double tf2_fraction(double x) {
+  return sizeof(T) == 4 ? x - __builtin_rint(x) : fract1(x);
 }
 
 // rho_k exp(-2 pi i f dd_k)
 template <typename T, int ND>
 __device__ __forceinline__ cplx<T> tf2_rotated(const Tf2Row<T, ND>& b, int k, double f) {
-  const cplx<T> e = expm2pi((T)fract1(f * b.dd[k]));
+  const cplx<T> e = expm2pi((T)tf2_fraction<T>(f * b.dd[k]));
   cplx<T> r = cmul_fma(b.rho[k], e);
   if constexpr (sizeof(T) == 4) {
     r.x = fma(b.rlo[k].x, e.x, fma(-b.rlo[k].y, e.y, r.x));
@@ -128,11 +139,7 @@ __device__ __forceinline__ cplx<T> tf2_product(double cycles, const cplx<T>* rot
     y.x = fma(rot[k].x, dw.x, fma(rot[k].y, dw.y, y.x));
     y.y = fma(rot[k].y, dw.x, fma(-rot[k].x, dw.y, y.y));
   }
-  // float32: the nearest whole number is taken off, not the one below, which
-  // halves the rounding of the fraction: every detector of an element shares
-  // it, so its errors add up over them
-  const double x = sizeof(T) == 4 ? cycles - __builtin_rint(cycles) : fract1(cycles);
-  return cmul_fma(expm2pi((T)x), y);
+  return cmul_fma(expm2pi((T)tf2_fraction<T>(cycles)), y);
 }
 
 // Rows of one workgroup sorted by reference detector (stable), so that the

@@ -208,7 +208,7 @@ __device__ __forceinline__ WaveEv wave_ev(const EvDev& ev) {
 // instructions a bin but finish a row in 15 to 20 ns however short the segment
 // is; here that is 3 to 6.  The transform is float64 because its vector
 // instructions issue at the rate of unpacked float32 ones: float32 passes were
-// 9 % faster (4096 rows of 4096 bins, two detectors) at 1.4 times the error.
+// 9 % faster (4096 rows of 4096 bins, two detectors) and added 1e-7 to the error.
 // Exchanges move the real parts, then the imaginary ones, which leaves room for
 // four workgroups a CU (76 us; whole values at three 87); the integrand stays
 // in float32 until all of it is there (68).
@@ -352,8 +352,10 @@ __global__ __launch_bounds__(64 * kWaves, 4) void k_time_row(TimeRowArgs a) {
   tf2_row<float, ND>(rw, b);
 #pragma unroll
   for (int k = 0; k < ND - 1; ++k) {
+    // (most of a signal's weight lies in the first slots: element i is the
+    // frequency i / 1024 of the sampling rate)
     double2 corr = make_double2(1.0, 0.0);
-    b.w[k] = tf2_rotation<float>((64.0 * (double)ev.Q * ev.df) * b.dd[k], 3.5, corr);
+    b.w[k] = tf2_rotation<float>((64.0 * (double)ev.Q * ev.df) * b.dd[k], 1.0, corr);
     tf2_rho<float, ND>(rw, k, corr, b);
     b.dwo[k] = ev.dwa32 + (size_t)(k < b.ref ? k : k + 1) * ev.N;
   }
@@ -844,7 +846,8 @@ __global__ __launch_bounds__(256) void k_tf2_tables(EvDev ev, double* tb, float2
   tb[3 * (size_t)i + 2] = lf;
   for (int d = 0; d < ev.nd; ++d) {
     const double2 w = ev.dw64[(size_t)d * ev.N + i];
-    dwa[(size_t)d * ev.N + i] = make_float2((float)(w.x * amp), (float)(w.y * amp));
+    dwa[(size_t)d * ev.N + i] =
+        make_float2((float)(w.x * amp * kExpm2piGain), (float)(w.y * amp * kExpm2piGain));
   }
 }
 
