@@ -1139,7 +1139,7 @@ int launch_band_eval_t(gwl_event* e, const double* params, int64_t n, int ld, do
       default: launch_band<T, 4>(a, R, st); break;
     }
     GWL_HIP_CHECK(hipGetLastError());
-    if (int rc = timing_end(e, st)) return rc;
+    if (int rc = timing_end(e, st, r0 + m == n)) return rc;
     FinishArgs f{ev, rows + r0, c, a.split.gs, out + r0};
     hipLaunchKernelGGL((cut_rows(ev) ? k_band_finish<T, true> : k_band_finish<T, false>),
                        dim3((unsigned)m), dim3(kFinThreads), lds, st, f);

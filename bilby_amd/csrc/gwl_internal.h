@@ -126,7 +126,8 @@ int noalloc_scratch_init(int device, void** ptr);
 int launch_eval(gwl_event* ev, const double* params, int64_t n, int ld, int precision, double* out,
                 double* aux, hipStream_t stream);
 int timing_begin(gwl_event* ev, hipStream_t stream);
-int timing_end(gwl_event* ev, hipStream_t stream);
+// (last: an evaluation in several passes counts once)
+int timing_end(gwl_event* ev, hipStream_t stream, bool last = true);
 // Split-bfloat16 x3 GEMM over K chunks into float32 partials C[z][M][N]
 // (z < ceil(K / kcol)); M, N multiples of 128, K and kcol multiples of 32.
 int gemm_bf16x3_split(const __bf16* Ah, const __bf16* Al, const __bf16* Bh, const __bf16* Bl,

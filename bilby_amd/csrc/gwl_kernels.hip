@@ -1447,14 +1447,14 @@ int timing_begin(gwl_event* e, hipStream_t st) {
   return GWL_OK;
 }
 
-int timing_end(gwl_event* e, hipStream_t st) {
+int timing_end(gwl_event* e, hipStream_t st, bool last) {
   if (!e->timing) return GWL_OK;
   GWL_HIP_CHECK(hipEventRecord(e->t1, st));
   GWL_HIP_CHECK(hipEventSynchronize(e->t1));
   float ms = 0.f;
   GWL_HIP_CHECK(hipEventElapsedTime(&ms, e->t0, e->t1));
   e->timed_ms += ms;
-  e->timed_launches += 1;
+  if (last) e->timed_launches += 1;
   return GWL_OK;
 }
 

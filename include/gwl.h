@@ -240,10 +240,13 @@ int gwl_event_set_escalation(gwl_event* ev, double coeff, double tol);
 int gwl_event_escalated_rows(gwl_event* ev, int64_t* rows);
 
 /* Kernel timing for measurement: while enabled, every gwl_eval on this event
- * brackets its dominant kernel (the fused inner-product or time-marginalised
- * kernel) with HIP events on the launch stream and waits for them; the
- * accumulated milliseconds and launch count are read (and reset) with
- * gwl_event_timing_read.  No counterpart in the reference (measurement). */
+ * brackets its dominant kernel with HIP events on the launch stream and waits
+ * for them: the time transform (of block projections the projections, without
+ * row constants and k_band_finish), or the float32 or float64 inner products
+ * with their row constants.  An evaluation in several passes adds them up and
+ * counts once (a window in slices counts each).  The accumulated milliseconds
+ * and the count are read (and reset) with gwl_event_timing_read.  No
+ * counterpart in the reference (measurement). */
 int gwl_event_timing(gwl_event* ev, int32_t enable);
 int gwl_event_timing_read(gwl_event* ev, double* total_ms, int64_t* launches);
 
