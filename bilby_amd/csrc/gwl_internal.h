@@ -142,9 +142,10 @@ int launch_epi_time(gwl_event* ev, const double* params, int64_t n, int ld, int 
                     const gwl::EvDev* slice = nullptr, double2* lse = nullptr, int first = 1,
                     int last = 1, const double* rinfo = nullptr);
 // TaylorF2 row constants (gwl_time_wave.hip)
-// (count: only rows r < *count exist; zero: cleared first)
+// (count: only rows r < *count exist; zero: cleared first; index: parameter rows)
 int launch_rowconst(const gwl_event* ev, const double* params, int64_t n, int ld, RowW* rows,
-                    hipStream_t stream, const int* count = nullptr, int* zero = nullptr);
+                    hipStream_t stream, const int* count = nullptr, int* zero = nullptr,
+                    const int* index = nullptr);
 // short segments: whole evaluation of a row by one wavefront (float32), where
 // it is faster than block projections
 constexpr int kTimeRowBins = 8192;

@@ -374,7 +374,7 @@ struct EpiArgs {
   const int* count;
   const int* scatter;
   // escalation (float32 pass): rows with esc_coeff * Q > esc_tol append
-  // their index to esc_idx and their parameter row to esc_params
+  // their index to esc_idx and (where set) their parameter row to esc_params
   // ([n][GWL_NPARAM]) through the counter esc_count
   int* esc_count;
   int* esc_idx;
@@ -415,9 +415,11 @@ __device__ __forceinline__ void epi_plain_row(const EpiArgs& a, long long r, lon
   if (a.esc_count && a.esc_coeff * escalation_scale(ev.flags, dhr, dhi, hh, hs) > a.esc_tol) {
     const int slot = atomicAdd(a.esc_count, 1);
     a.esc_idx[slot] = (int)r;
-    const double* src = a.params + r * a.ld;
-    double* dst = a.esc_params + (size_t)slot * GWL_NPARAM;
-    for (int k = 0; k < GWL_NPARAM; ++k) dst[k] = src[k];
+    if (a.esc_params) {
+      const double* src = a.params + r * a.ld;
+      double* dst = a.esc_params + (size_t)slot * GWL_NPARAM;
+      for (int k = 0; k < GWL_NPARAM; ++k) dst[k] = src[k];
+    }
   }
   double ll;
   if (ev.flags & GWL_DISTANCE_MARG) {
@@ -1050,11 +1052,11 @@ static int launch_reduce(gwl_event* e, const double* params, int64_t n, int ld, 
   return GWL_OK;
 }
 
-// One pass of the TaylorF2 inner products (arguments as launch_reduce).
+// One pass of the TaylorF2 inner products (arguments as launch_reduce; the
+// float64 pass reads the escalated rows through their indices, scatter).
 struct InnerWs {
   double* part;
   RowW* rows;
-  double* esc_params;
   int* esc_idx;
   int* esc_count;
 };
@@ -1068,7 +1070,6 @@ static size_t inner_ws(const EvDev& ev, long long n, char* p, InnerWs* w) {
   };
   w->part = reinterpret_cast<double*>(take((size_t)n * inner_units_of(ev) * sizeof(double2)));
   w->rows = reinterpret_cast<RowW*>(take((size_t)n * sizeof(RowW)));
-  w->esc_params = reinterpret_cast<double*>(take((size_t)n * GWL_NPARAM * sizeof(double)));
   w->esc_idx = reinterpret_cast<int*>(take((size_t)n * sizeof(int)));
   w->esc_count = reinterpret_cast<int*>(take(sizeof(int)));
   return off;
@@ -1081,7 +1082,8 @@ static int launch_inner_pass(gwl_event* e, bool fp64, const double* params, int6
   inner_ws(e->dev, n, reinterpret_cast<char*>(e->ws), &ws);
   if (!count)
     if (int rc = timing_begin(e, st)) return rc;
-  if (int rc = launch_rowconst(e, params, n, ld, ws.rows, st, count, esc ? ws.esc_count : nullptr))
+  if (int rc = launch_rowconst(e, params, n, ld, ws.rows, st, count, esc ? ws.esc_count : nullptr,
+                               scatter))
     return rc;
   if (int rc = launch_inner(e, fp64, ws.rows, n, count, ws.part, st)) return rc;
   if (!count)
@@ -1101,7 +1103,6 @@ static int launch_inner_pass(gwl_event* e, bool fp64, const double* params, int6
   if (esc) {
     ea.esc_count = ws.esc_count;
     ea.esc_idx = ws.esc_idx;
-    ea.esc_params = ws.esc_params;
     ea.esc_coeff = e->esc_coeff;
     ea.esc_tol = e->esc_tol;
   }
@@ -1152,8 +1153,8 @@ static int eval_typed(gwl_event* e, const double* params, int64_t n, int ld, dou
     InnerWs ws;
     inner_ws(ev, n, reinterpret_cast<char*>(e->ws), &ws);
     e->esc_count_dev = ws.esc_count;
-    return launch_inner_pass(e, true, ws.esc_params, n, GWL_NPARAM, out, aux, st, ws.esc_count,
-                             ws.esc_idx, false);
+    return launch_inner_pass(e, true, params, n, ld, out, aux, st, ws.esc_count, ws.esc_idx,
+                             false);
   } else {
     if (int rc = launch_reduce<R, WAVE, ND>(e, params, n, ld, out, aux, st, nullptr, nullptr,
                                             esc))

@@ -52,6 +52,7 @@ struct RowArgs {
   double2* c64 = nullptr;  // [n][GWL_MAX_DET] float64 detector amplitudes, or null
   const int* count = nullptr;  // if set: only rows r < *count exist (n bounds it)
   int* zero = nullptr;         // cleared by the first thread
+  const int* index = nullptr;  // if set: row r's parameters are row index[r]
 };
 
 // Row constants of 64 rows by two wavefronts: the first takes the TaylorF2
@@ -170,7 +171,8 @@ __global__ __launch_bounds__(2 * kRowconstRows) void k_rowconst(RowArgs a) {
   const long long r = (long long)blockIdx.x * kRowconstRows + (threadIdx.x & 63);
   const bool live = r < (a.count ? min(a.n, (long long)*a.count) : a.n);
   if (a.zero && blockIdx.x == 0 && threadIdx.x == 0) *a.zero = 0;
-  rowconst_pair(a.ev, a.params + r * a.ld, live, a.rows + r,
+  const long long at = a.index && live ? (long long)a.index[r] : r;
+  rowconst_pair(a.ev, a.params + at * a.ld, live, a.rows + r,
                 a.c64 ? a.c64 + r * GWL_MAX_DET : nullptr, sh);
 }
 
@@ -866,8 +868,8 @@ static size_t cal_time_lds_bytes(const EvDev& ev, bool fp64) {
 }
 
 int launch_rowconst(const gwl_event* e, const double* params, int64_t n, int ld, RowW* rows,
-                    hipStream_t st, const int* count, int* zero) {
-  RowArgs ra{e->dev, params, ld, n, rows, nullptr, count, zero};
+                    hipStream_t st, const int* count, int* zero, const int* index) {
+  RowArgs ra{e->dev, params, ld, n, rows, nullptr, count, zero, index};
   hipLaunchKernelGGL(k_rowconst, dim3((unsigned)((n + kRowconstRows - 1) / kRowconstRows)),
                      dim3(2 * kRowconstRows), 0, st, ra);
   GWL_HIP_CHECK(hipGetLastError());

@@ -131,3 +131,26 @@ def test_noalloc_takes_the_tiled_transform_of_a_short_window(duration, precision
     rc1, got, _ = _eval(LIB.gwl_eval_noalloc, lk, rows, prec)
     assert rc0 == 0 and rc1 == 0, LIB.gwl_last_error()
     assert np.array_equal(got, ref)
+
+
+def test_noalloc_takes_large_batches_of_short_plain_segments():
+    """1024 bins without time marginalisation: a row needs 320 bytes of sums and
+    constants and its place in the escalation list, so 160000 rows fit."""
+    from bilby_amd._lib import LIB, FP32, FP64
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    s = make_taylorf2_marginalised(n_draws=160000, seed=8, duration=1.0,
+                                   sampling_frequency=2048.0, detectors=("H1", "L1"),
+                                   time=False, distance=False, phase=False)
+    lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                    precision="fp32")
+    lk.set_precision_escalation(2e-7, 1e-5)   # escalates a good part of the rows
+    rows = _rows(lk, s["draws"])
+    for prec in (FP32, FP64):
+        rc0, ref, aux0 = _eval(LIB.gwl_eval, lk, rows, prec, aux=True)
+        if prec == FP32:
+            n = lk.escalated_rows()
+            assert 1000 < n < 159000, n
+        rc1, got, aux1 = _eval(LIB.gwl_eval_noalloc, lk, rows, prec, aux=True)
+        assert rc0 == 0 and rc1 == 0, LIB.gwl_last_error()
+        assert np.array_equal(got, ref) and np.array_equal(aux1, aux0)
