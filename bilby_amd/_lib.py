@@ -102,6 +102,8 @@ def _load():
                                 _dp, ctypes.c_int32, _dp, ctypes.c_int32, _dp], ctypes.c_int),
         "gwl_spline2d_coefficients": ([ctypes.c_int32, ctypes.c_int32, _dp, _dp, _dp, _dp, _dp, _dp],
                                       ctypes.c_int),
+        "gwl_band_functions_host": ([ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _dp, _dp],
+                                    ctypes.c_int),
         "gwl_spline2d_eval_host": ([ctypes.c_int32, ctypes.c_int32, _dp, _dp, _dp, ctypes.c_int64,
                                     _dp, _dp, _dp], ctypes.c_int),
         "gwl_fft_batch": ([vp, vp, vp, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, vp],
@@ -232,7 +234,7 @@ EXPORTED_SYMBOLS = [
     "gwl_ctx_create", "gwl_ctx_destroy", "gwl_last_error", "gwl_event_create",
     "gwl_event_destroy", "gwl_event_set_distance_spline", "gwl_event_reserve", "gwl_eval",
     "gwl_detector_response", "gwl_distance_table", "gwl_spline2d_coefficients",
-    "gwl_spline2d_eval_host", "gwl_fft_batch", "gwl_ln_i0", "gwl_noise_log_likelihood",
+    "gwl_spline2d_eval_host", "gwl_band_functions_host", "gwl_fft_batch", "gwl_ln_i0", "gwl_noise_log_likelihood",
     "gwl_event_timing", "gwl_event_timing_read", "gwl_event_set_tile",
     "gwl_roq_create", "gwl_roq_destroy", "gwl_roq_set_distance_spline", "gwl_roq_eval",
     "gwl_gemm", "gwl_multi_create", "gwl_multi_set_rows", "gwl_multi_set_tile",

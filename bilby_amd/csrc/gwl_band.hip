@@ -13,9 +13,10 @@
 //   exp(-i c x y) = sum_{p < 16} U_p(x) V_p(y),   x = t / (B/2), y = kappa / (L/2)
 // with U_p the prolate spheroidal functions of bandwidth c = pi B L / (2 N)
 // (D. Slepian, H. O. Pollak, Bell Syst. Tech. J. 40, 1961) and V_p their
-// transforms; the largest error over t and kappa is 4e-11 at L = 420 and
-// 9e-10 at L = 512 for NB = 128 (float32 arithmetic), below 1e-14 for
-// NB = 256 (float64).  Then
+// transforms.  The largest error over t and kappa grows with the window and a
+// little with B: for NB = 128 (float32 arithmetic) 5e-11 at L = 420, 1.2e-9 at
+// L = 512 (B = 128), 1.2e-10 and 2.9e-9 at B = 1024; for NB = 256 (float64) below
+// 2e-15 at L = 420, 1.4e-14 at L = 512 (B = 64), 3.8e-14 at B = 512.  Then
 //   C[b][p] = sum_t x[b B + t] U_p(t)              k_band: MFMA, M = 16 blocks, N = 16 p, K = bins
 //   D_p[q] = sum_b C[b][p] W_NB^(b q)              k_band_finish: 16 DFTs of NB points
 //   X[j] = exp(-i pi (B - 1) kappa / N) sum_p V_p(kappa) D_p[kappa mod NB]
@@ -892,12 +893,18 @@ void band_functions(int NB, int B, int L, std::vector<double>& u, std::vector<do
     for (int p = 0; p < kNP / 2; ++p)
       for (int i = 0; i < n; ++i) beta[2 * p + par][2 * i + par] = vec[p][i];
   }
+  // (the square roots once: in the loops they were most of an event's set-up)
+  Real up[kLeg], vp[kLeg];
+  for (int k = 0; k < kLeg; ++k) {
+    up[k] = std::sqrt(k + 0.5L);
+    vp[k] = std::sqrt((Real)(2 * (2 * k + 1))) * (((k >> 1) & 1) ? -1 : 1);
+  }
   u.assign((size_t)B * kNP, 0.0);
   for (int t = 0; t < B; ++t) {
     const Real x = (t - 0.5L * (B - 1)) / (0.5L * B);
     Real p0 = 1, p1 = x, sum[kNP] = {0};
     for (int k = 0; k < kLeg; ++k) {
-      const Real pk = p0 * std::sqrt(k + 0.5L);
+      const Real pk = p0 * up[k];
       for (int p = k & 1; p < kNP; p += 2) sum[p] += beta[p][k] * pk;
       const Real p2 = ((2 * k + 3) * x * p1 - (k + 1) * p0) / (k + 2);
       p0 = p1;
@@ -906,35 +913,35 @@ void band_functions(int NB, int B, int L, std::vector<double>& u, std::vector<do
     for (int p = 0; p < kNP; ++p) u[(size_t)t * kNP + p] = (double)sum[p];
   }
   v.assign((size_t)kNP * L, 0.0);
-  for (int jj = 0; jj < L; ++jj) {
-    const Real z = c * (jj - L / 2) / (0.5L * L);
+  for (int m = 0; m <= L / 2; ++m) {  // kappa = m and -m: V_p(-y) = (-1)^p V_p(y)
+    const Real z = c * m / (0.5L * L);
     // spherical Bessel functions by downward recurrence, sum (2k + 1) j_k^2 = 1
     Real jk[kLeg] = {0};
-    if (z == 0) {
+    if (m == 0) {
       jk[0] = 1;
     } else {
-      const Real az = std::fabs(z);
       Real hi = 0, lo = 1e-300L, norm = 0, val[kLeg] = {0};
       for (int k = kLeg + 40; k >= 0; --k) {  // lo = j_k, hi = j_{k+1} (unnormalised)
         if (k < kLeg) val[k] = lo;
         norm += (2 * k + 1) * lo * lo;
-        const Real down = (2 * k + 1) / az * lo - hi;
+        const Real down = (2 * k + 1) / z * lo - hi;
         hi = lo;
         lo = down;
       }
-      const Real j0 = std::sin(az) / az;
-      const Real j1 = j0 / az - std::cos(az) / az;
+      const Real j0 = std::sin(z) / z;
+      const Real j1 = j0 / z - std::cos(z) / z;
       Real sc = 1 / std::sqrt(norm);
       const bool by0 = std::fabs(j0) > std::fabs(j1);
       if ((by0 ? val[0] * j0 : val[1] * j1) < 0) sc = -sc;
-      for (int k = 0; k < kLeg; ++k)
-        jk[k] = val[k] * sc * ((z < 0 && (k & 1)) ? -1 : 1);
+      for (int k = 0; k < kLeg; ++k) jk[k] = val[k] * sc;
     }
     for (int p = 0; p < kNP; ++p) {
       Real s = 0;
       for (int k = p & 1; k < kLeg; k += 2)
-        s += beta[p][k] * std::sqrt((Real)(2 * (2 * k + 1))) * (((k >> 1) & 1) ? -1 : 1) * jk[k];
-      v[((size_t)(p >> 1) * L + jj) * 2 + (p & 1)] = (double)s;
+        s += beta[p][k] * vp[k] * jk[k];
+      double* vp2 = v.data() + ((size_t)(p >> 1) * L + L / 2) * 2 + (p & 1);
+      if (L / 2 + m < L) vp2[2 * m] = (double)s;
+      vp2[-2 * m] = (p & 1) ? -(double)s : (double)s;
     }
   }
 }
@@ -1005,8 +1012,9 @@ template <typename T> constexpr size_t band_row_bytes() {
 // How a batch is cut: R rows per wavefront, then the groups, so that 24 to 48
 // wavefronts per CU are queued (8 run at once, and three rounds or more even out
 // the ends: 4096 rows of 16384 bins take 208, 199, 194 and 194 us with 8, 16, 32
-// and 64, parts of 8, 4, 2 and one group; 24 asks for the third of these), then, where all groups leave the chip short of 8, the steps (each part adds
-// a row of sums to read back).  A caller's tile sets both targets.
+// and 64, parts of 8, 4, 2 and one group; 24 asks for the third of these), then,
+// where all groups leave the chip short of 8, the steps (each part adds a row
+// of sums to read back).  A caller's tile sets both targets.
 template <typename T>
 BandSplit band_split(const gwl_event* e, long long n, int& R) {
   const EvDev& ev = e->dev;
@@ -1223,3 +1231,17 @@ int band_multi_launch(gwl_multi* m, hipStream_t st) {
 }
 
 }  // namespace gwl
+
+extern "C" int gwl_band_functions_host(int32_t n_blocks, int32_t n_bins, int32_t n_window,
+                                       double* u, double* v) {
+  if ((n_blocks != 128 && n_blocks != 256) || n_bins < 1 || n_window < 1 || n_window > 512 || !u ||
+      !v) {
+    gwl::set_error("gwl_band_functions_host: invalid argument");
+    return GWL_E_INVALID;
+  }
+  std::vector<double> hu, hv;
+  gwl::band_functions(n_blocks, n_bins, n_window, hu, hv);
+  std::copy(hu.begin(), hu.end(), u);
+  std::copy(hv.begin(), hv.end(), v);
+  return GWL_OK;
+}

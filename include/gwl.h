@@ -303,6 +303,15 @@ int gwl_spline2d_eval_host(int32_t nx, int32_t ny, const double* tx, const doubl
                            const double* c, int64_t m, const double* x, const double* y,
                            double* out);
 
+/* Functions of the block-projected window transform (host only; for checking
+ * them): with x = (t - (n_bins - 1) / 2) / (n_bins / 2), y = kappa /
+ * (n_window / 2), kappa = j - n_window / 2 and c = pi n_window / (2 n_blocks),
+ * exp(-i c x y) = sum over 16 p of u[t][p] v_p(j), v_p(j) = v[p / 2][j][0] for
+ * even p, -i v[p / 2][j][1] for odd p.  n_blocks 128 or 256, n_window <= 512;
+ * u: [n_bins][16], v: [8][n_window][2].  No counterpart in the reference. */
+int gwl_band_functions_host(int32_t n_blocks, int32_t n_bins, int32_t n_window, double* u,
+                            double* v);
+
 /* Batched complex FFT of length P (power of two, 2..16 x the longest LDS
  * transform: 131072 in float64, 262144 in float32 on gfx950) with the LDS
  * radix kernel used by time marginalisation (numpy.fft.fft as called at
