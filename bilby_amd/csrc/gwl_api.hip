@@ -677,7 +677,7 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
         }
       }
       const size_t o = (size_t)k * N + i;
-      dw32[o] = make_float2((float)re, (float)im);
+      dw32[o] = make_float2((float)(re * kExpm2piGain), (float)(im * kExpm2piGain));
       w32[o] = (float)w;
       dw64[o] = make_double2(re, im);
       w64[o] = w;

@@ -185,7 +185,7 @@ __device__ __forceinline__ void bin_rows(int n, double f, const cplx<R>* dw, con
         const R hr = p.x * e.x - p.y * e.y, hi = p.x * e.y + p.y * e.x;
         ar += hr * dw[d].x + hi * dw[d].y;
         ai += hi * dw[d].x - hr * dw[d].y;
-        hw += (hr * hr + hi * hi) * w[d];
+        hw += (p.x * p.x + p.y * p.y) * w[d];
       }
       I[s] = cmk<C>(ar, ai);
       hh[s] += hw;

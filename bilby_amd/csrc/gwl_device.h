@@ -131,7 +131,7 @@ struct BandDev {
 struct InnerDev {
   const double2* uv;    // (f^1/3, f^-1/3)
   const double2* lf;    // ln f, two bins each
-  const float2* dw32;   // [nd] d / S f^-7/6
+  const float2* dw32;   // [nd] d / S f^-7/6 (times kExpm2piGain)
   const double2* dw64;
 };
 
@@ -151,13 +151,13 @@ struct EvDev {
   double tp_t0, tp_ih;
   int tp_n;
   // data in decimated order: element i <-> bin n = Q*(i % P) + i / P, i < N.
-  const float2* dw32;  // [nd][N]  (d/S) * sigma
+  const float2* dw32;  // [nd][N]  (d/S) * sigma, times kExpm2piGain
   const float* w32;    // [nd][N]  sigma^2 / S
   const double2* dw64;
   const double* w64;
   // TaylorF2 tables of the time transforms (null otherwise):
   const double* tf2b;   // [N][3] (f^1/3, f^-1/3, ln f), decimated order
-  const float2* dwa32;  // [nd][N] dw32 f^-7/6, decimated order
+  const float2* dwa32;  // [nd][N] the same times f^-7/6, decimated order
   const double* hps;    // [nd][N + 2] prefix sums of f^-7/3 sigma^2 / S over bins
                         //   0..N in natural order, hps[d][n] = sum of bins < n
   BandDev band32, band64;

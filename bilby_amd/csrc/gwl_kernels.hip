@@ -288,7 +288,8 @@ __device__ __forceinline__ void time_tile(const EvDev& ev, int nd, const double*
 #pragma unroll
     for (int s = 0; s < S; ++s) hacc[s] += (double)h[s];
   }
-  // write window partials
+  // write window partials (with what the float32 twiddles lose)
+  constexpr double gain = sizeof(R) == 4 ? kExpm2piGain : 1.0;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const long long r = row0 + s;
@@ -297,7 +298,7 @@ __device__ __forceinline__ void time_tile(const EvDev& ev, int nd, const double*
 #pragma unroll
       for (int jt = 0; jt < JT; ++jt) {
         const int jj = tid + jt * NT;
-        if (jj < ev.L) dst[jj] = make_double2(acc[s][jt][0], acc[s][jt][1]);
+        if (jj < ev.L) dst[jj] = make_double2(gain * acc[s][jt][0], gain * acc[s][jt][1]);
       }
     }
   }

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
     }
   }
   // epilogue per curve: time-marginalised lnL (base.py:794-820 per curve)
-  const double norm = 4.0 / ev.T;
+  const double norm = 4.0 / ev.T, xnorm = norm * kExpm2piGain;  // (the window's twiddles)
   const double hs = rw.hscale, jit = rw.jitter;
   const double b = time_lse_scale(ev, ev.tdelta);
 #pragma unroll
@@ -661,8 +661,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_cal_time_w(CalTimeArgs a) {
         const int j = ev.jlo + jj;
         const double t = (ev.start + (double)(j + 1) * ev.tstep) + jit;
         if (t >= ev.tmin && t <= ev.tmax)
-          lse_push(m, sum, epi_value(ev.flags, ev.sp, yy, hh, hs, norm * accr[cc][s],
-                                     norm * acci[cc][s]) +
+          lse_push(m, sum, epi_value(ev.flags, ev.sp, yy, hh, hs, xnorm * accr[cc][s],
+                                     xnorm * acci[cc][s]) +
                                time_log_weight(ev, t));
       }
     }
@@ -829,7 +829,7 @@ __global__ __launch_bounds__(2 * kRowconstRows) void k_rowconst_multi(RowMultiAr
   rowconst_pair(a.evs[e], a.params[e] + r * a.ld, r < a.rows[e], a.roww[e] + r, nullptr, sh);
 }
 
-// f^1/3, f^-1/3, ln f and dw32 f^-7/6 at every decimated element.
+// f^1/3, f^-1/3, ln f and d / S f^-7/6 at every decimated element.
 __global__ __launch_bounds__(256) void k_tf2_tables(EvDev ev, double* tb, float2* dwa) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= ev.N) return;

@@ -57,3 +57,22 @@ def test_time_marginalised(duration, fs, rows):
     out = [lk.log_likelihood_ratio_batch(draws, precision=p) for p in ("fp32", "fp64")]
     rel = out[0] / out[1] - 1.0
     assert np.abs(np.median(rel)) < 6e-8, np.median(rel)
+
+
+def test_sine_gaussian_inner_products():
+    """(limits as for TaylorF2; a burst's sum counts some 100 bins)"""
+    from bilby_amd.configs import make_sine_gaussian_plain
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    s = make_sine_gaussian_plain(n_draws=500, seed=3)
+    rng = np.random.default_rng(3)
+    for k, w in dict(frequency=3.0, Q=0.5, hrss=1e-23, ra=0.05, dec=0.03, psi=0.1,
+                     geocent_time=1e-3).items():
+        s["draws"][k] = s["injection"][k] + w * rng.normal(size=500)
+    lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                    precision="fp32")
+    lk.set_precision_escalation(0.0)
+    aux = [lk.log_likelihood_ratio_batch(s["draws"], precision=p,
+                                         return_inner_products=True)[1] for p in ("fp32", "fp64")]
+    z = [a[:, 0] + 1j * a[:, 1] for a in aux]
+    rel = (z[0] * z[1].conj()).real / np.abs(z[1]) ** 2 - 1.0
+    assert np.abs(np.median(rel)) < 2e-8, np.median(rel)
