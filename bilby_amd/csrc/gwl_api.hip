@@ -691,8 +691,9 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
       ev.wN[k] = sg2 / s;
     }
   }
-  // TaylorF2 with a 512-point time transform: tables of the per-curve
-  // transforms and of the row constants, including prefix sums of f^-7/3 sigma^2 / S over bins 0..N
+  // TaylorF2 with a 512-point time transform: tables of the block projections
+  // and of the row constants (prefix sums of f^-7/3 sigma^2 / S over bins 0..N);
+  // short segments, those of the wavefront-per-row evaluation
   const bool wave_tables = ev.approx == GWL_TAYLORF2 && (ev.flags & GWL_TIME_MARG) && ev.P == 512;
   // (and, without time marginalisation, of the inner products)
   const bool inner = ev.approx == GWL_TAYLORF2 && !(ev.flags & GWL_TIME_MARG);
@@ -724,9 +725,9 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
   e->ctx = ctx;
   const size_t b32 = n_el * (sizeof(float2) + sizeof(float));
   const size_t b64 = n_el * (sizeof(double2) + sizeof(double));
-  const size_t bw = wave_tables ? ((size_t)N * 3 * sizeof(double) + n_el * sizeof(float2)) +
-                                      hps.size() * sizeof(double) + 4096
-                                : 0;
+  const bool row_tables = wave_tables && N <= kTimeRowBins;
+  const size_t bw = (row_tables ? time_wave_table_bytes(ev) : 0) +
+                    (wave_tables ? hps.size() * sizeof(double) + 4096 : 0);
   const bool band = wave_tables && band_tables_wanted(ev);
   const size_t bb = band ? band_table_bytes(ev) + 256 : 0;
   const size_t bi = inner ? inner_table_bytes(ev) + hps.size() * sizeof(double) + 512 : 0;
@@ -737,6 +738,7 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
     return GWL_E_NOMEM;
   }
   char* p = reinterpret_cast<char*>(e->data);
+  char* wave_mem = nullptr;
   ev.dw64 = reinterpret_cast<double2*>(p);
   p += n_el * sizeof(double2);
   ev.w64 = reinterpret_cast<double*>(p);
@@ -747,10 +749,8 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
   p += n_el * sizeof(float);
   if (wave_tables) {
     p = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
-    ev.tf2b = reinterpret_cast<double*>(p);
-    p += (size_t)N * 3 * sizeof(double);
-    ev.dwa32 = reinterpret_cast<float2*>(p);
-    p += n_el * sizeof(float2);
+    wave_mem = p;
+    if (row_tables) p += time_wave_table_bytes(ev);
     ev.hps = reinterpret_cast<double*>(p);
     p += hps.size() * sizeof(double);
   } else if (inner) {
@@ -781,8 +781,7 @@ int gwl_event_create(gwl_ctx* ctx, const gwl_event_desc* d, gwl_event** out, int
   }
   if (wave_tables) {
     int rc = band ? band_table_init(ev, band_mem) : GWL_OK;
-    if (rc == GWL_OK)
-      rc = init_time_wave_tables(ev, const_cast<double*>(ev.tf2b), const_cast<float2*>(ev.dwa32));
+    if (rc == GWL_OK && row_tables) rc = init_time_wave_tables(ev, wave_mem);
     if (rc != GWL_OK) {
       (void)hipFree(e->data);
       delete e;
@@ -894,6 +893,7 @@ int gwl_event_destroy(gwl_event* e) {
   if (e->t1) (void)hipEventDestroy(e->t1);
   if (e->data) (void)hipFree(e->data);
   if (e->spline) (void)hipFree(e->spline);
+  if (e->wave_mem) (void)hipFree(e->wave_mem);
   if (e->tprior) (void)hipFree(e->tprior);
   if (e->ws) (void)hipFree(e->ws);
   delete e;
@@ -952,7 +952,7 @@ int gwl_event_reserve(gwl_event* e, int64_t rows) {
 
 int gwl_event_device_bytes(gwl_event* e, int64_t* bytes) {
   if (!e || !bytes) { set_error("gwl_event_device_bytes: invalid argument"); return GWL_E_INVALID; }
-  *bytes = (int64_t)(e->data_bytes + e->spline_bytes + e->ws_bytes);
+  *bytes = (int64_t)(e->data_bytes + e->wave_bytes + e->spline_bytes + e->ws_bytes);
   return GWL_OK;
 }
 

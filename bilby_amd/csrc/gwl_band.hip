@@ -1168,8 +1168,10 @@ size_t band_table_bytes(const EvDev& ev) {
 
 int band_table_init(EvDev& ev, char* p) {
   if (int rc = init_band<float>(ev, ev.band32, p)) return rc;
-  return band_fits<double>(ev) ? init_band<double>(ev, ev.band64, p + band_bytes<float>(ev))
-                               : GWL_OK;
+  if (band_fits<double>(ev))
+    if (int rc = init_band<double>(ev, ev.band64, p + band_bytes<float>(ev))) return rc;
+  GWL_HIP_CHECK(hipDeviceSynchronize());
+  return GWL_OK;
 }
 
 bool band_eligible(const gwl_event* e, bool fp64) {

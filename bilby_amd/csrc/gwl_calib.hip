@@ -308,6 +308,7 @@ int calib_create_time(gwl_event* ev, int nc, const double* curves, int K, gwl_ca
   }
   const int nd = d.nd, N = d.N;
   GWL_HIP_CHECK(hipSetDevice(ev->ctx->device));
+  if (int rc = time_wave_tables(ev)) return rc;
   std::vector<double> hps((size_t)nd * (N + 2));
   GWL_HIP_CHECK(hipMemcpy(hps.data(), d.hps, hps.size() * 8, hipMemcpyDeviceToHost));
   std::vector<float2> tab, tab_lo;

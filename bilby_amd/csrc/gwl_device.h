@@ -155,7 +155,7 @@ struct EvDev {
   const float* w32;    // [nd][N]  sigma^2 / S
   const double2* dw64;
   const double* w64;
-  // TaylorF2 tables of the time transforms (null otherwise):
+  // TaylorF2 tables of the 512-point transforms in registers (null: none yet):
   const double* tf2b;   // [N][3] (f^1/3, f^-1/3, ln f), decimated order
   const float2* dwa32;  // [nd][N] the same times f^-7/6, decimated order
   const double* hps;    // [nd][N + 2] prefix sums of f^-7/3 sigma^2 / S over bins

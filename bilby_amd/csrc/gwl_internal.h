@@ -26,6 +26,8 @@ struct gwl_event {
   size_t data_bytes = 0;
   double* spline = nullptr;      // device: tx, ty, coefficients
   size_t spline_bytes = 0;
+  void* wave_mem = nullptr;      // tables of the 512-point transforms made later (time_wave_tables)
+  size_t wave_bytes = 0;
   double* tprior = nullptr;      // device: time-prior density table
   void* ws = nullptr;            // device workspace (partials)
   size_t ws_bytes = 0;
@@ -153,7 +155,12 @@ bool time_row_wins(const gwl_event* ev, int64_t rows);
 int launch_time_row(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
                     hipStream_t stream);
 int multi_launch_rowconst(gwl_multi* m, hipStream_t stream);
-int init_time_wave_tables(const EvDev& ev, double* tf2b, float2* dwa32);
+// tables of the 512-point transforms in registers (short segments, and
+// calibration with time marginalisation): into device memory p, or, where the
+// event has none yet, into memory of its own
+size_t time_wave_table_bytes(const EvDev& ev);
+int init_time_wave_tables(EvDev& ev, char* p);
+int time_wave_tables(gwl_event* ev);
 // block-projected window transform (gwl_band.hip)
 bool band_tables_wanted(const EvDev& ev);
 size_t band_table_bytes(const EvDev& ev);

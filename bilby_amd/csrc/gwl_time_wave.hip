@@ -11,6 +11,7 @@
 #include "gwl_tf2_rows.h"
 
 #include <algorithm>
+#include <mutex>
 
 namespace gwl {
 
@@ -853,11 +854,33 @@ __global__ __launch_bounds__(256) void k_tf2_tables(EvDev ev, double* tb, float2
   }
 }
 
-int init_time_wave_tables(const EvDev& ev, double* tb, float2* dwa) {
+size_t time_wave_table_bytes(const EvDev& ev) {
+  return (size_t)ev.N * (3 * sizeof(double) + ev.nd * sizeof(float2));
+}
+
+int init_time_wave_tables(EvDev& ev, char* p) {
+  double* tb = reinterpret_cast<double*>(p);
+  float2* dwa = reinterpret_cast<float2*>(tb + 3 * (size_t)ev.N);
   hipLaunchKernelGGL(k_tf2_tables, dim3((unsigned)((ev.N + 255) / 256)), dim3(256), 0, 0, ev, tb, dwa);
   GWL_HIP_CHECK(hipGetLastError());
   GWL_HIP_CHECK(hipDeviceSynchronize());
+  ev.tf2b = tb;
+  ev.dwa32 = dwa;
   return GWL_OK;
+}
+
+int time_wave_tables(gwl_event* e) {
+  static std::mutex mu;  // (several calibrations of one event made at once)
+  std::lock_guard<std::mutex> lock(mu);
+  if (e->dev.tf2b) return GWL_OK;
+  const size_t bytes = time_wave_table_bytes(e->dev);
+  if (!e->wave_mem && hipMalloc(&e->wave_mem, bytes) != hipSuccess) {
+    e->wave_mem = nullptr;
+    set_error("hipMalloc failed for the transform tables");
+    return GWL_E_NOMEM;
+  }
+  e->wave_bytes = bytes;
+  return init_time_wave_tables(e->dev, static_cast<char*>(e->wave_mem));
 }
 
 // k_cal_time_w: the 512-entry pass-2 table, tw3, the exchange buffers
@@ -915,7 +938,7 @@ size_t roww_bytes(int64_t rows) { return (size_t)rows * sizeof(RowW); }
 
 bool cal_time_eligible(const gwl_event* e) {
   const EvDev& ev = e->dev;
-  return (ev.flags & GWL_TIME_MARG) && ev.approx == GWL_TAYLORF2 && ev.P == kWP && ev.tf2b &&
+  return (ev.flags & GWL_TIME_MARG) && ev.approx == GWL_TAYLORF2 && ev.P == kWP && ev.hps &&
          ev.L <= kWP;
 }
 

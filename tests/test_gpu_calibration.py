@@ -272,3 +272,38 @@ def test_per_detector_log_likelihoods_with_calibration(time, tmp_path):
             got = out["%s_log_likelihood" % ifo.name]
             say(ifo.name, got, ref)
             assert abs(got - ref) < tol
+
+
+def test_tables_of_the_per_curve_transforms_are_made_with_the_curves(tmp_path):
+    """An event of a long segment holds the transforms' tables (24 bytes a bin
+    and 8 more a detector) only where calibration with time needs them; a short
+    one's batches use them as well."""
+    import ctypes
+    from bilby_amd import calibration as cal
+    from bilby_amd._lib import LIB, check
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+
+    def device_bytes(duration, curves):
+        s = make_taylorf2_marginalised(n_draws=2, seed=9, duration=duration,
+                                       sampling_frequency=2048.0, detectors=("H1", "L1"),
+                                       distance=False)
+        kw = {}
+        if curves:
+            for ifo in s["interferometers"]:
+                ifo.calibration_model = cal.CubicSpline("recalib_%s_" % ifo.name, 20.0, 512.0, 5)
+                s["priors"].update(cal.constant_uncertainty_spline_priors(0.1, 0.1, 20.0, 512.0, 5,
+                                                                          ifo.name))
+            kw = dict(calibration_marginalization=True, number_of_response_curves=2,
+                      calibration_lookup_table={
+                          ifo.name: str(tmp_path / ("%s_%g.npz" % (ifo.name, duration)))
+                          for ifo in s["interferometers"]})
+        lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                        time_marginalization=True, phase_marginalization=True,
+                                        priors=s["priors"].copy(), **kw)
+        b = ctypes.c_int64()
+        check(LIB.gwl_event_device_bytes(lk._event, ctypes.byref(b)))
+        return b.value
+
+    for duration, more in ((16.0, 16384 * (24 + 16)), (8.0, 0)):
+        assert device_bytes(duration, True) - device_bytes(duration, False) == more
