@@ -5,8 +5,9 @@ parameter batch per workgroup, target resident workgroups per CU; rows 0
 selects the block-projected TaylorF2 time transform where the event allows it,
 and the second number is then the target wavefronts per CU) on the
 device with HIP events, keeps the fastest, and caches the choice per
-(device, source model, marginalisation flags, detectors, bin-count bucket,
-batch bucket) in a JSON file so later processes reuse it.
+(kernel generation, device, source model, marginalisation flags, detectors,
+bin-count bucket, batch bucket) in a JSON file so later processes reuse it.
+TaylorF2 without time marginalisation has one form and nothing to tune.
 """
 import ctypes
 import json
@@ -15,10 +16,14 @@ import os
 
 import torch
 
-from ._lib import LIB, check
+from ._lib import LIB, TAYLORF2, check
 
-DEFAULT_CANDIDATES_TIME = [(0, 8), (0, 16), (0, 32), (0, 64), (8, 2), (8, 4), (8, 8), (4, 4),
-                           (4, 8), (2, 8), (1, 8), (8, 16)]
+# Raised when kernels change what a tile means or which are worth trying: a choice
+# made among other kernels would keep an event on the slower of today's.
+KERNEL_GENERATION = 2
+
+DEFAULT_CANDIDATES_TIME = [(0, 8), (0, 16), (0, 24), (0, 32), (0, 64), (8, 2), (8, 4), (8, 8),
+                           (4, 4), (4, 8), (2, 8), (1, 8), (8, 16)]
 DEFAULT_CANDIDATES_PLAIN = [(4, 0), (8, 0), (16, 0)]
 CACHE_PATH = os.environ.get("BILBY_AMD_AUTOTUNE_CACHE",
                             os.path.join(os.path.expanduser("~"), ".cache", "bilby_amd",
@@ -30,7 +35,8 @@ def bucket_key(likelihood, n_rows):
     n_freq = len(ifos.frequency_array)
     dev = torch.cuda.get_device_name(likelihood.device)
     return "|".join(str(x) for x in (
-        dev, likelihood.waveform_generator.approximant, likelihood._flags(), len(ifos),
+        "kernels %d" % KERNEL_GENERATION, dev, likelihood.waveform_generator.approximant,
+        likelihood._flags(), len(ifos),
         int(math.log2(max(2, n_freq - 1))), int(math.log2(max(1, n_rows))), likelihood.precision))
 
 
@@ -67,7 +73,7 @@ MULTI_CANDIDATES = (8, 16, 32, 64)
 
 
 def multi_bucket_key(likelihoods, rows):
-    """Cache key of a multi-event set: the device and every event's
+    """Cache key of a multi-event set: the kernels, the device and every event's
     (source, flags, detectors, log2 bins, log2 rows), sorted."""
     dev = torch.cuda.get_device_name(likelihoods[0].device)
     shapes = sorted("%d:%d:%d:%d:%d" % (lk.waveform_generator.approximant, lk._flags(),
@@ -75,7 +81,7 @@ def multi_bucket_key(likelihoods, rows):
                                           int(math.log2(max(2, len(lk.interferometers.frequency_array) - 1))),
                                           int(math.log2(max(1, n))))
                     for lk, n in zip(likelihoods, rows))
-    return dev + "|multi|" + ",".join(shapes)
+    return "kernels %d|%s|multi|%s" % (KERNEL_GENERATION, dev, ",".join(shapes))
 
 
 def set_multi_steps(likelihood, steps):
@@ -147,6 +153,10 @@ def time_tile(likelihood, rows_t, tile, repeats=5, precision=None):
 def autotune(likelihood, rows_t, candidates=None, repeats=5, use_cache=True, precision=None):
     """Pick and apply the fastest tile for this likelihood and batch shape.
     Returns (tile, {tile: ms})."""
+    plain = not likelihood.time_marginalization
+    if plain and likelihood.waveform_generator.approximant == TAYLORF2:
+        set_tile(likelihood, 0, 0)
+        return (0, 0), {}
     key = bucket_key(likelihood, rows_t.shape[0])
     cache = _load_cache() if use_cache else {}
     if use_cache and key in cache:

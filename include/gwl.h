@@ -204,9 +204,10 @@ int gwl_event_time_window(gwl_event* ev, int64_t* j_first, int32_t* n_window, do
  * transform uses the block-projected transform, and workgroups_per_cu is the
  * target wavefronts per CU (default 24); in float32, batches of at least half
  * as many rows as bins on segments of up to 8192 bins use one wavefront per row
- * instead (their values agree with smaller batches' to float32 rounding).  Float64 evaluations without time
- * marginalisation use 4 rows per workgroup whatever is set here.  Used by the
- * autotuner; no counterpart in the reference. */
+ * instead (their values agree with smaller batches' to float32 rounding).
+ * Without time marginalisation TaylorF2 takes no tile, and other sources use 4
+ * rows per workgroup in float64, whatever is set here.  Used by the autotuner;
+ * no counterpart in the reference. */
 int gwl_event_set_tile(gwl_event* ev, int32_t rows_per_workgroup, int32_t workgroups_per_cu);
 
 /* This event's tile inside multi-event launches: decimated sub-sequence
