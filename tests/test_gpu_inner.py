@@ -66,3 +66,33 @@ def test_prefix_sums_of_hh_are_rounded_once(duration):
                    for p in draws_as_dicts(s["draws"], range(40))])
     rel = aux[:, 2] / hh - 1.0
     assert np.abs(np.median(rel)) < 1e-15, (np.median(rel), np.abs(rel).max())
+
+
+def test_escalated_rows_carry_the_float64_bits():
+    """Without escalation the float32 error stays below the coefficient that
+    selects rows, times Q = |<d|h>| + <h|h>, where that matters (Q above 1000: the
+    selection starts at 4000); with it the selected rows are those past the
+    tolerance, with float64's values, and every row is within 1e-3."""
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    s = make_taylorf2_marginalised(n_draws=4095, seed=5, duration=4.0, sampling_frequency=2048.0,
+                                   detectors=("H1", "L1", "V1"), time=False, distance=False,
+                                   phase=False)
+    rng = np.random.default_rng(5)
+    s["draws"]["luminosity_distance"] = np.exp(rng.uniform(np.log(30.0), np.log(2000.0), 4095))
+    lk = GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                    precision="fp32")
+    d = s["draws"]
+    out64, aux64 = lk.log_likelihood_ratio_batch(d, precision="fp64", return_inner_products=True)
+    lk.set_precision_escalation(0.0)
+    raw32 = lk.log_likelihood_ratio_batch(d)
+    q = np.hypot(aux64[:, 0], aux64[:, 1]) + aux64[:, 2]
+    loud = q > 1000.0
+    assert np.max((np.abs(raw32 - out64) / q)[loud]) < 2e-7
+    lk.set_precision_escalation()
+    out32, aux32 = lk.log_likelihood_ratio_batch(d, return_inner_products=True)
+    sure, maybe = 2e-7 * q > 8e-4 * 1.01, 2e-7 * q > 8e-4 * 0.99
+    assert 100 < np.sum(sure) <= lk.escalated_rows() <= np.sum(maybe) < 4000
+    assert np.array_equal(out32[sure], out64[sure]) and np.array_equal(aux32[sure], aux64[sure])
+    assert np.array_equal(out32[~maybe], raw32[~maybe])
+    assert np.max(np.abs(out32 - out64)) < 1e-3
