@@ -1229,6 +1229,8 @@ int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
     m->groups.push_back(multi_groups(m, Q, st));
     items += (size_t)((max_rows[e] + 7) / 8) * (m->wave_path ? kBandGroups : std::min(Q, 16));
     blocks += (size_t)((max_rows[e] + 3) / 4);
+    m->row_form.push_back(m->wave_path && time_row_wins(ev, max_rows[e]));
+    if (m->row_form.back()) m->max_rblocks += (size_t)((max_rows[e] + 3) / 4);
   }
   m->max_items = std::max<size_t>(items, 1);
   m->max_blocks = std::max<size_t>(blocks, 1);
@@ -1264,7 +1266,8 @@ int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
   const size_t ne = (size_t)n_events;
   const size_t bytes = ne * sizeof(EvDev) + 6 * ne * sizeof(void*) + ne * sizeof(long long) +
                        ne * sizeof(int) + m->max_items * sizeof(MultiItem) +
-                       m->max_blocks * (sizeof(int) + sizeof(long long)) + 64 * 8 + 16 * 256;
+                       (m->max_blocks + m->max_rblocks) * (sizeof(int) + sizeof(long long)) +
+                       64 * 8 + 16 * 256;
   if (hipMalloc(&m->dev, bytes) != hipSuccess) {
     gwl_multi_destroy(m);
     set_error("hipMalloc failed for multi-event tables");
@@ -1288,9 +1291,12 @@ int gwl_multi_create(gwl_ctx* ctx, int32_t n_events, gwl_event* const* events,
   m->d_items = reinterpret_cast<MultiItem*>(take(m->max_items * sizeof(MultiItem)));
   m->d_block_event = reinterpret_cast<int*>(take(m->max_blocks * sizeof(int)));
   m->d_block_row0 = reinterpret_cast<long long*>(take(m->max_blocks * sizeof(long long)));
-  m->d_n_items = reinterpret_cast<int*>(take(sizeof(int)));
-  m->d_counter = reinterpret_cast<int*>(take(sizeof(int)));
-  m->d_n_blocks = reinterpret_cast<int*>(take(sizeof(int)));
+  m->d_n_items = reinterpret_cast<int*>(take(4 * sizeof(int)));  // (multi_set_rows writes the four)
+  m->d_n_blocks = m->d_n_items + 1;
+  m->d_n_rblocks = m->d_n_items + 2;
+  m->d_counter = m->d_n_items + 3;
+  m->d_rblock_event = reinterpret_cast<int*>(take(m->max_rblocks * sizeof(int)));
+  m->d_rblock_row0 = reinterpret_cast<long long*>(take(m->max_rblocks * sizeof(long long)));
   std::vector<EvDev> evs;
   for (auto* ev : m->events) evs.push_back(ev->dev);
   hipError_t err = hipMemcpy(m->d_evs, evs.data(), ne * sizeof(EvDev), hipMemcpyHostToDevice);

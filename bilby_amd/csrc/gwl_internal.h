@@ -92,7 +92,14 @@ struct gwl_multi {
   int* d_block_event = nullptr;
   long long* d_block_row0 = nullptr;
   int* d_n_blocks = nullptr;
-  size_t max_items = 0, max_blocks = 0;
+  // rows that take one wavefront each (time_row_wins), out of the lists above;
+  // row_form: the events that have room for it
+  std::vector<char> row_form;
+  int* d_rblock_event = nullptr;
+  long long* d_rblock_row0 = nullptr;
+  int* d_n_rblocks = nullptr;
+  size_t max_items = 0, max_blocks = 0, max_rblocks = 0;
+  int n_rblocks = 0;
   int n_items = 0;
   bool captured = false;
   hipGraph_t graph = nullptr;
@@ -154,6 +161,7 @@ constexpr int kTimeRowBins = 8192;
 bool time_row_wins(const gwl_event* ev, int64_t rows);
 int launch_time_row(gwl_event* ev, const double* params, int64_t n, int ld, double* out,
                     hipStream_t stream);
+int multi_launch_time_row(gwl_multi* m, hipStream_t stream);
 int multi_launch_rowconst(gwl_multi* m, hipStream_t stream);
 // tables of the 512-point transforms in registers (short segments, and
 // calibration with time marginalisation): into device memory p, or, where the

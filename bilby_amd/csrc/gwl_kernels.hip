@@ -1337,8 +1337,8 @@ size_t multi_lds_bytes() {
 // decreasing cost (sub-sequence steps) order, and the epilogue blocks.
 int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
   std::vector<MultiItem> items;
-  std::vector<int> bev;
-  std::vector<long long> brow;
+  std::vector<int> bev, rbev;
+  std::vector<long long> brow, rbrow;
   std::vector<long long> cost;
   for (int e = 0; e < m->n_events; ++e) {
     if (rows[e] < 0 || rows[e] > m->max_rows[e]) {
@@ -1346,6 +1346,14 @@ int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
       return GWL_E_INVALID;
     }
     m->rows[e] = rows[e];
+    // whole batches of short segments as the event's own evaluation takes them
+    if (m->row_form[e] && time_row_wins(m->events[e], rows[e])) {
+      for (long long r0 = 0; r0 < rows[e]; r0 += kEpiRows) {
+        rbev.push_back(e);
+        rbrow.push_back(r0);
+      }
+      continue;
+    }
     const EvDev& ev = m->events[e]->dev;
     const int Q = ev.N / kMultiP;
     const int G = m->groups[e];
@@ -1367,7 +1375,8 @@ int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
       brow.push_back(r0);
     }
   }
-  if (items.size() > m->max_items || bev.size() > m->max_blocks) {
+  if (items.size() > m->max_items || bev.size() > m->max_blocks ||
+      rbev.size() > m->max_rblocks) {
     set_error("gwl_multi_set_rows: work list larger than allocated");
     return GWL_E_INVALID;
   }
@@ -1382,14 +1391,20 @@ int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
   GWL_HIP_CHECK(hipMemcpy(m->d_rows, rr.data(), rr.size() * sizeof(long long), hipMemcpyHostToDevice));
   if (n_items)
     GWL_HIP_CHECK(hipMemcpy(m->d_items, sorted.data(), n_items * sizeof(MultiItem), hipMemcpyHostToDevice));
-  GWL_HIP_CHECK(hipMemcpy(m->d_n_items, &n_items, sizeof(int), hipMemcpyHostToDevice));
   if (n_blocks) {
     GWL_HIP_CHECK(hipMemcpy(m->d_block_event, bev.data(), n_blocks * sizeof(int), hipMemcpyHostToDevice));
     GWL_HIP_CHECK(hipMemcpy(m->d_block_row0, brow.data(), n_blocks * sizeof(long long), hipMemcpyHostToDevice));
   }
-  GWL_HIP_CHECK(hipMemcpy(m->d_n_blocks, &n_blocks, sizeof(int), hipMemcpyHostToDevice));
+  const int n_rblocks = (int)rbev.size();
+  if (n_rblocks) {
+    GWL_HIP_CHECK(hipMemcpy(m->d_rblock_event, rbev.data(), n_rblocks * sizeof(int), hipMemcpyHostToDevice));
+    GWL_HIP_CHECK(hipMemcpy(m->d_rblock_row0, rbrow.data(), n_rblocks * sizeof(long long), hipMemcpyHostToDevice));
+  }
+  const int counts[4] = {n_items, n_blocks, n_rblocks, 0};  // (the counter)
+  GWL_HIP_CHECK(hipMemcpy(m->d_n_items, counts, sizeof counts, hipMemcpyHostToDevice));
   m->n_items = n_items;
   m->n_blocks = n_blocks;
+  m->n_rblocks = n_rblocks;
   (void)st;
   return GWL_OK;
 }
@@ -1399,7 +1414,8 @@ int multi_set_rows(gwl_multi* m, const int64_t* rows, hipStream_t st) {
 int multi_launch_raw(gwl_multi* m, hipStream_t st) {
   if (m->wave_path) {
     if (int rc = multi_launch_rowconst(m, st)) return rc;
-    return band_multi_launch(m, st);
+    if (int rc = band_multi_launch(m, st)) return rc;
+    return multi_launch_time_row(m, st);
   }
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, m->d_counter);
   GWL_HIP_CHECK(hipGetLastError());

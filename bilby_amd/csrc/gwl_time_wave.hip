@@ -327,27 +327,13 @@ __device__ __forceinline__ void time_row_step(const WaveEv& ev, const TimeRow<ND
   }
 }
 
-struct TimeRowArgs {
-  EvDev ev;
-  const RowW* rows;
-  long long n;
-  double* out;
-};
-
+// One row, after init_row_tables.
 template <int ND>
-__global__ __launch_bounds__(64 * kWaves, 4) void k_time_row(TimeRowArgs a) {
-  __shared__ double2 wt[kWP], tw2[kTw2], tw3[kTw3];
-  __shared__ double xch[kWaves * kXch];
-  const EvDev& ev = a.ev;
-  init_row_tables(tw2, tw3, wt, ev.N, ev.jlo);
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long long r = (long long)blockIdx.x * kWaves + wid;
-  if (r >= a.n) return;
-  const RowW& rw = a.rows[r];
+__device__ __forceinline__ void time_row_eval(const EvDev& ev, const RowW& rw, double* out,
+                                              const double2* tw2, const double2* tw3,
+                                              const double2* wt, double* xb, int lane) {
   if (!rw.valid) {
-    if (lane == 0) a.out[r] = row_valid_sentinel();
+    if (lane == 0) *out = row_valid_sentinel();
     return;
   }
   const WaveEv wv = wave_ev(ev);
@@ -363,7 +349,6 @@ __global__ __launch_bounds__(64 * kWaves, 4) void k_time_row(TimeRowArgs a) {
     b.dwo[k] = ev.dwa32 + (size_t)(k < b.ref ? k : k + 1) * ev.N;
   }
   b.dwr = ev.dwa32 + (size_t)b.ref * ev.N;
-  double* xb = xch + wid * kXch;
   const double2* tw2l = tw2 + (lane & 7);
   const int base2 = 64 * (lane >> 3) + (lane & 7);
   double accr[8], acci[8];
@@ -391,8 +376,59 @@ __global__ __launch_bounds__(64 * kWaves, 4) void k_time_row(TimeRowArgs a) {
     }
   }
   lse_wave(m, sum);
-  if (lane == 0)
-    a.out[r] = (m > -INFINITY) ? log(time_lse_scale(ev, ev.tdelta) * sum) + m : -INFINITY;
+  if (lane == 0) *out = (m > -INFINITY) ? log(time_lse_scale(ev, ev.tdelta) * sum) + m : -INFINITY;
+}
+
+struct TimeRowArgs {
+  EvDev ev;
+  const RowW* rows;
+  long long n;
+  double* out;
+};
+
+template <int ND>
+__global__ __launch_bounds__(64 * kWaves, 4) void k_time_row(TimeRowArgs a) {
+  __shared__ double2 wt[kWP], tw2[kTw2], tw3[kTw3];
+  __shared__ double xch[kWaves * kXch];
+  init_row_tables(tw2, tw3, wt, a.ev.N, a.ev.jlo);
+  __syncthreads();
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long r = (long long)blockIdx.x * kWaves + wid;
+  if (r >= a.n) return;
+  time_row_eval<ND>(a.ev, a.rows[r], a.out + r, tw2, tw3, wt, xch + wid * kXch, threadIdx.x & 63);
+}
+
+// The rows of several events that take this form: four to a workgroup of the
+// list.
+struct TimeRowMultiArgs {
+  const EvDev* evs;
+  const long long* rows;
+  const RowW* const* roww;
+  double* const* out;
+  const int* block_event;
+  const long long* block_row0;
+  const int* n_blocks;
+};
+
+__global__ __launch_bounds__(64 * kWaves, 4) void k_time_row_multi(TimeRowMultiArgs a) {
+  static_assert(kWaves == kMultiEpiRows, "rows per block of the list");
+  __shared__ double2 wt[kWP], tw2[kTw2], tw3[kTw3];
+  __shared__ double xch[kWaves * kXch];
+  if ((int)blockIdx.x >= *a.n_blocks) return;
+  const int e = a.block_event[blockIdx.x];
+  const EvDev& ev = a.evs[e];
+  init_row_tables(tw2, tw3, wt, ev.N, ev.jlo);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long r = a.block_row0[blockIdx.x] + wid;
+  if (r >= a.rows[e]) return;
+  double* xb = xch + wid * kXch;
+  switch (ev.nd) {
+    case 1: time_row_eval<1>(ev, a.roww[e][r], a.out[e] + r, tw2, tw3, wt, xb, lane); break;
+    case 2: time_row_eval<2>(ev, a.roww[e][r], a.out[e] + r, tw2, tw3, wt, xb, lane); break;
+    default: time_row_eval<3>(ev, a.roww[e][r], a.out[e] + r, tw2, tw3, wt, xb, lane);
+  }
 }
 
 // ------------------------------------------------------------------ calibration
@@ -1029,6 +1065,23 @@ int multi_launch_rowconst(gwl_multi* m, hipStream_t st) {
   hipLaunchKernelGGL(k_rowconst_multi, dim3((unsigned)((maxr + kRowconstRows - 1) / kRowconstRows),
                                               (unsigned)m->n_events),
                      dim3(2 * kRowconstRows), 0, st, a);
+  GWL_HIP_CHECK(hipGetLastError());
+  return GWL_OK;
+}
+
+int multi_launch_time_row(gwl_multi* m, hipStream_t st) {
+  TimeRowMultiArgs a;
+  a.evs = m->d_evs;
+  a.rows = m->d_rows;
+  a.roww = reinterpret_cast<const RowW* const*>(m->d_roww);
+  a.out = m->d_outs;
+  a.block_event = m->d_rblock_event;
+  a.block_row0 = m->d_rblock_row0;
+  a.n_blocks = m->d_n_rblocks;
+  // an eager launch covers the current list, a captured graph the largest
+  const size_t blocks = m->capturing ? m->max_rblocks : (size_t)m->n_rblocks;
+  if (!blocks) return GWL_OK;
+  hipLaunchKernelGGL(k_time_row_multi, dim3((unsigned)blocks), dim3(64 * kWaves), 0, st, a);
   GWL_HIP_CHECK(hipGetLastError());
   return GWL_OK;
 }

@@ -89,3 +89,49 @@ def test_multi_event_graph_replays():
         torch.cuda.synchronize()
         for e in range(len(events)):
             assert np.max(np.abs(outs[e] - eager[e])) < 1e-8, (rep, e)
+
+
+def test_short_events_cross_between_forms():
+    """Events of short segments take one wavefront a row from half as many rows as
+    bins on, as in their own evaluation, and block projections below; the row
+    counts of a captured graph cross that line between replays, next to an
+    event that never does and one cut at the ISCO."""
+    import torch
+    from bilby_amd.configs import make_taylorf2_marginalised
+    from bilby_amd.likelihood import GravitationalWaveTransient
+    from bilby_amd.multi import MultiEventLikelihood
+    from tests.helpers import fixed_marginalised
+    say("multi-event: short segments")
+    lks, draws = [], []
+    for k, (duration, dets, rows, isco) in enumerate([
+            (1.0, ("H1",), 601, None), (4.0, ("H1", "L1"), 33, None),
+            (1.5, ("H1", "L1", "V1"), 770, "isco"), (1.0, ("H1", "L1"), 512, None)]):
+        s = make_taylorf2_marginalised(n_draws=rows, seed=50 + k, duration=duration,
+                                       sampling_frequency=2048.0, detectors=dets, distance=k == 3,
+                                       taylorf2_termination=isco)
+        priors = s["priors"].copy()
+        lks.append(GravitationalWaveTransient(s["interferometers"], s["waveform_generator"],
+                                              time_marginalization=True,
+                                              distance_marginalization=k == 3,
+                                              phase_marginalization=True, priors=priors))
+        draws.append({key: np.array(v) for key, v in fixed_marginalised(s["draws"], priors).items()})
+        draws[-1]["mass_1"][rows // 2] = -1.0
+    full = [len(d["mass_1"]) for d in draws]
+    multi = MultiEventLikelihood(lks, full)
+    for captured in (False, True):
+        if captured:
+            multi.capture()
+        for counts in (full, [511, 33, 767, 512], [601, 1, 768, 511], [3, 33, 770, 0], full):
+            sub = [{key: v[len(v) - n:] for key, v in d.items()} for d, n in zip(draws, counts)]
+            for e, n in enumerate(counts):
+                if n:
+                    multi.set_parameters(e, sub[e])
+                else:
+                    multi.rows[e] = 0
+            outs = [o.cpu().numpy().copy() for o in multi.run()]
+            torch.cuda.synchronize()
+            for e, n in enumerate(counts):
+                if n:
+                    one = lks[e].log_likelihood_ratio_batch(sub[e])
+                    # the same kernels' values, sums of blocks in another order
+                    assert np.max(np.abs(outs[e][:n] - one)) < 1e-8, (captured, counts, e)
