@@ -275,7 +275,7 @@ def bench_uneven(steps):
                                      for i in lk.interferometers) * 12 + 72)
                  for ev, lk in zip(events, lks))
     valu = profile_figure("bench-valu-insts", "k_band_multi_uneven_64_events")
-    roof = {"kernel": "k_band_multi + k_band_finish_multi (all 64 events in one launch each)",
+    roof = {"kernel": "k_band_multi + k_band_finish_multi + k_time_row_multi (64 events, one launch each)",
             "algorithmic_bytes_per_launch": abytes,
             "hbm": {"achieved": abytes / dt / 1e9, "peak": 8000.0, "unit": "GB/s",
                     "frac": abytes / dt / 1e9 / 8000.0,
