@@ -233,8 +233,10 @@ int gwl_event_set_transform(gwl_event* ev, int32_t transform);
  * distance marginalisation 2 dt^2 / ht + dt + ht of the table arguments
  * dt = <d|h> d / d_ref, ht = <h|h> (d / d_ref)^2).  coeff = 0 turns it off;
  * defaults coeff = 2e-7 (the largest float32 |dlnL| / Q measured over 10^4
- * sine-Gaussian rows with |lnL| up to 5e5 is 1.4e-7), tol = 8e-4.  The workspace holds the selected rows
- * (gwl_event_reserve sizes it), so the call still allocates nothing. */
+ * sine-Gaussian rows with |lnL| up to 5e5 is 1.4e-7, over 10^4 TaylorF2 rows
+ * with |lnL| up to 1e8 9.3e-8, and 1.6e-8 where Q > 1000), tol = 8e-4.  The
+ * workspace holds the selected rows (TaylorF2: their numbers;
+ * gwl_event_reserve sizes it), so the call still allocates nothing. */
 int gwl_event_set_escalation(gwl_event* ev, double coeff, double tol);
 /* Rows escalated by the last escalating gwl_eval on this event (waits for
  * the device; for measurement). */
